@@ -1,6 +1,6 @@
 /*
  * hipdvr_batch.h -- many volumes, each with its own TF and camera, marched in
- * one persistent launch.
+ * one launch.
  *
  * No counterpart in the reference: Voreen renders one volume per raycaster
  * process() call (cpuraycaster.cpp:90-208; a network of N raycasters makes N
@@ -8,10 +8,9 @@
  * (multi-view dashboards, ensembles): every job is the plain DVR march of
  * hipdvr_render_device (linear filter, TF classification, DVR compositing,
  * optional Phong) with the same result bit for bit, but all jobs' image tiles
- * are handed out by one device work queue to a persistent grid of workgroups,
- * largest jobs first.  The launch can be captured into a hipGraph and
- * replayed; an autotuner picks the wave tile shape, the empty-space brick
- * size and the number of samples fetched together per ray.
+ * are one launch's workgroups, largest jobs first.  The launch can be captured
+ * into a hipGraph and replayed; an autotuner picks the tile shape, the
+ * empty-space brick size and the number of lanes that march a ray together.
  */
 #ifndef HIPDVR_BATCH_H
 #define HIPDVR_BATCH_H
@@ -38,16 +37,17 @@ typedef struct hipdvr_batch_job {
                                classification TF, compositing DVR */
 } hipdvr_batch_job;
 
-/* wave tile shapes (pixels per wavefront) */
+/* tile shapes (pixels per 64-pixel region; a tile is 2x2 regions) */
 enum { HIPDVR_TILE_8x8 = 0, HIPDVR_TILE_16x4 = 1, HIPDVR_TILE_32x2 = 2 };
 
 typedef struct hipdvr_batch_config {
     int32_t tile;           /* HIPDVR_TILE_* */
     int32_t brick_log2;     /* empty-space bricks of 8^3, 16^3, 32^3: 3, 4, 5 */
-    int32_t batch;          /* samples fetched together per ray: 2 or 4 */
-    int32_t resident;       /* persistent workgroups per CU, 1..8 (at most what fits); 0: three
-                               when a job's cell records need 64-bit addressing (their caches
-                               thrash sooner), else as many as fit, at most five */
+    int32_t batch;          /* lanes of a wavefront that march a ray together, each one sample
+                               of a pass: 2 or 4 (launches below 1.5 M pixels take at least
+                               four, those above 6 M two) */
+    int32_t resident;       /* workgroups per CU at a time, 1..8 (at most what fits); 0: as many
+                               as fit */
 } hipdvr_batch_config;
 
 /* Jobs are copied; the volumes, TFs and buffers must outlive the batch.
@@ -63,7 +63,7 @@ int hipdvr_batch_get_config(const hipdvr_batch* b, hipdvr_batch_config* cfg);
  * CU with the fastest; keep the fastest; best_ms (may be NULL) receives its
  * mean launch time. */
 int hipdvr_batch_autotune(hipdvr_batch* b, uint32_t reps, hipdvr_batch_config* best, float* best_ms);
-/* Capture one batched launch (queue reset + persistent march) as a hipGraph
+/* Capture one batched launch as a hipGraph
  * on the context stream; hipdvr_batch_launch then replays it. */
 int hipdvr_batch_capture(hipdvr_batch* b);
 /* Asynchronous on the context stream: the graph when captured, else a direct
@@ -82,15 +82,13 @@ int hipdvr_batch_launch(hipdvr_batch* b, hipdvr_stats* stats);
  * must outlive their use by the batch.  Calling again replaces the set. */
 int hipdvr_batch_set_learned(hipdvr_batch* b, hipdvr_learned* const* learned, uint32_t n,
                              const hipdvr_learned_opts* opts);
-/* One batched launch with learned stepping: one persistent launch marches
+/* One batched launch with learned stepping: one launch marches
  * the judges' plain re-march of every learned view's sparse pixels (each ray
  * whole, so the sparse images equal the plain frames at those pixels
  * exactly) and the learned and plain jobs; then the judges of all learned
  * views run in one launch, and per learned view the plain frame, which runs
  * only when its view fell below the PSNR floor (the steps of
- * hipdvr_render_learned_device, for all views of the batch at once; that
- * entry point re-marches one view's judge rays in segments, equal up to
- * float rounding).  Asynchronous unless stats != NULL:
+ * hipdvr_render_learned_device, for all views of the batch at once).  Asynchronous unless stats != NULL:
  * n_jobs entries in the caller's order, sparse_psnr and fell_back per learned
  * job, samples and shaded the totals of the whole launch. */
 int hipdvr_batch_launch_learned(hipdvr_batch* b, hipdvr_learned_stats* stats);

@@ -165,9 +165,8 @@ int hipdvr_render_learned_device(hipdvr_learned* l, const hipdvr_tf* tf, const f
 int hipdvr_learned_sparse_dims(uint32_t w, uint32_t h, const hipdvr_learned_opts* opts, uint32_t* sw,
                                uint32_t* sh);
 /* The judge's plain re-march on its own, on the grid of
- * hipdvr_learned_sparse_dims, marched by the plain path with each ray cut
- * into segments that run in parallel and are joined front to back (equal to
- * the sequential march up to float rounding of the joins).  d_sparse holds
+ * hipdvr_learned_sparse_dims, marched by the plain path (its pixels equal the
+ * plain frame's).  d_sparse holds
  * `capacity` RGBA float pixels and receives *sw x *sh of them (row-major);
  * HIPDVR_ERR_INVALID when capacity is below that.  Synchronous. */
 int hipdvr_learned_sparse_remarch(hipdvr_learned* l, const hipdvr_tf* tf, const float* d_entry,

@@ -89,17 +89,24 @@ void host_copy(void* dst, const void* src, size_t bytes) {
 
 namespace hipdvr {
 
-// Per-brick occupancy of `vol` under the TF mapping of `tf` (and the volume's
-// real-world mapping); recomputed only when the pair changes.
-void ensure_occupancy(hipdvr_ctx* ctx, hipdvr_volume* vol, const hipdvr_tf* tf) {
-    const uint64_t key[4] = {tf->serial, (fbits(tf->domain_lo) << 32) | fbits(tf->domain_hi),
-                             (fbits(vol->desc.rwm_scale) << 32) | fbits(vol->desc.rwm_offset),
-                             tf->width};
-    if (std::memcmp(key, vol->occ_key, sizeof key) == 0) return;
+namespace {
+
+// The TF mapping a volume's occupancy or skip grid belongs to.
+struct MappingKey {
+    uint64_t k[4];
+    MappingKey(const hipdvr_volume* vol, const hipdvr_tf* tf)
+        : k{tf->serial, (fbits(tf->domain_lo) << 32) | fbits(tf->domain_hi),
+            (fbits(vol->desc.rwm_scale) << 32) | fbits(vol->desc.rwm_offset), tf->width} {}
+};
+
+}  // namespace
+
+OccArgs occupancy_args(const hipdvr_volume* vol, const hipdvr_tf* tf, const uint2* minmax, uint64_t count) {
     OccArgs o;
-    o.minmax = vol->d_minmax;
-    o.occ = vol->d_occ;
-    o.count = vol->brick_count;
+    o.minmax = minmax;
+    o.occ = nullptr;
+    o.bits = nullptr;
+    o.count = count;
     o.dtype = vol->desc.dtype;
     o.rwm_scale = vol->desc.rwm_scale;
     o.rwm_offset = vol->desc.rwm_offset;
@@ -107,10 +114,31 @@ void ensure_occupancy(hipdvr_ctx* ctx, hipdvr_volume* vol, const hipdvr_tf* tf) 
     o.dom_hi = tf->domain_hi;
     o.tf_width = (int32_t)tf->width;
     o.alpha_prefix = tf->d_alpha_prefix;
+    return o;
+}
+
+// Per-brick occupancy of `vol` (bricked and slab kernels) under the TF
+// mapping of `tf` and the volume's real-world mapping; recomputed only when
+// the pair changes.
+void ensure_occupancy(hipdvr_ctx* ctx, hipdvr_volume* vol, const hipdvr_tf* tf) {
+    const MappingKey key(vol, tf);
+    if (std::memcmp(key.k, vol->occ_key, sizeof key.k) == 0) return;
+    OccArgs o = occupancy_args(vol, tf, vol->d_minmax, vol->brick_count);
+    o.occ = vol->d_occ;
     o.bits = vol->d_occ_bits;
     launch_occupancy(o, ctx->stream);
     hip_check(hipGetLastError(), "occupancy kernel launch");
-    std::memcpy(vol->occ_key, key, sizeof key);
+    std::memcpy(vol->occ_key, key.k, sizeof key.k);
+}
+
+// The same for the skip grid of the cell kernels.
+void ensure_skip(hipdvr_ctx* ctx, hipdvr_volume* vol, const hipdvr_tf* tf) {
+    const MappingKey key(vol, tf);
+    if (std::memcmp(key.k, vol->skip_key, sizeof key.k) == 0) return;
+    launch_skip_grid(occupancy_args(vol, tf, vol->d_minmax8, vol->skip_count), vol->nskip, vol->d_skip,
+                     vol->d_skip + vol->skip_count, ctx->stream);
+    hip_check(hipGetLastError(), "skip grid kernel launch");
+    std::memcpy(vol->skip_key, key.k, sizeof key.k);
 }
 
 // Opacity correction per alpha byte: cpuraycaster.cpp:291 with the TF colour
@@ -165,9 +193,12 @@ void fill_march_args(MarchArgs& a, const hipdvr_volume* vol, const hipdvr_tf* tf
     a.occ_bits = vol->d_occ_bits;
     a.occ_words = vol->occ_words;
     a.brick_log2 = v.brick_log2;
+    a.skip = vol->d_skip;
+    a.skip_log2 = kSkipLog2;
     for (int i = 0; i < 3; ++i) {
         a.dims[i] = v.dims[i];
         a.nbricks[i] = vol->nbricks[i];
+        a.nskip[i] = vol->nskip[i];
         a.fdims[i] = (float)v.dims[i];
         a.fdm1[i] = (float)v.dims[i] - 1.0f;
         a.spacing[i] = v.spacing[i];
@@ -209,6 +240,7 @@ void fill_march_args(MarchArgs& a, const hipdvr_volume* vol, const hipdvr_tf* tf
     a.grid_h = (int32_t)h;
     a.stride = 1;
     a.pix_offset = 0;
+    a.pix_block = 1;
     a.cond_flag = nullptr;
     a.counters = counters;
     a.compositing = p->compositing;
@@ -297,8 +329,9 @@ void render_device_impl(hipdvr_ctx* ctx, const hipdvr_volume* vol, const hipdvr_
         ensure_tf2d(mtf, p->step, ctx->stream);
         a.tf2d = mtf->d_tf2d;
     }
-    if (kernel == HIPDVR_KERNEL_BRICKED || cell || slab) ensure_occupancy(ctx, mvol, tf);
+    if (kernel == HIPDVR_KERNEL_BRICKED || slab) ensure_occupancy(ctx, mvol, tf);
     if (cell) {
+        ensure_skip(ctx, mvol, tf);
         ensure_cells(mvol, ctx->stream);
         a.cells = mvol->d_cells;
     }
@@ -312,11 +345,8 @@ void render_device_impl(hipdvr_ctx* ctx, const hipdvr_volume* vol, const hipdvr_
         const int shade = phong ? ((p->exact_shading || p->shading != HIPDVR_SHADE_PHONG) ? 2 : 1) : 0;
         launch_march_slab(a, vol->desc.dtype, shade, count, ctx->stream);
     } else if (kernel == HIPDVR_KERNEL_CELL) {
-        // samples in flight per ray: default_batch (kernels.h)
         const int shade = phong ? ((p->exact_shading || p->shading != HIPDVR_SHADE_PHONG) ? 2 : 1) : 0;
-        launch_march_cell(a, vol->desc.dtype, shade, count, mvol->cells_wide,
-                          p->batch ? p->batch : default_batch(shade), ctx->stream);
-
+        launch_march_cell(a, vol->desc.dtype, shade, count, mvol->cells_wide, p->batch, ctx->stream);
     } else {
         // buffer descriptors address at most 2^32 - 1 bytes
         const uint64_t vsz = vol->desc.dtype == HIPDVR_U8 ? 1 : 2;

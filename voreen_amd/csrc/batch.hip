@@ -1,13 +1,15 @@
-// batch.hip -- many volumes in one persistent launch (include/hipdvr_batch.h).
+// batch.hip -- many volumes in one launch (include/hipdvr_batch.h).
 //
 // Every job is the cell-record march of hipdvr_render_device (march_cell.h),
 // so each job's image is bit-identical to its single-frame render.  The image
 // tiles of all jobs form one list, jobs in decreasing order of estimated cost
-// (pixels x longest volume axis: largest first); a persistent grid of
-// workgroups (CUs x resident workgroups per CU, at most five) takes tiles
-// from a device counter until the list is exhausted, reloading the TF and
-// opacity table in LDS when a tile belongs to another job.  Every workgroup leaves when the
-// counter passes the end of the list, so the grid always drains.
+// (pixels x longest volume axis: largest first), one workgroup per part of a
+// tile, which finds its job in the list's prefix sums and loads that job's TF
+// into LDS.  The hardware's dispatcher is the work queue: workgroups start in
+// list order as others end.  (A persistent grid that took tiles from counters
+// kept every job's arguments live across its loop and spilled 120 to 250
+// scalar registers into the march: 12 views of 512^3 with two lanes per ray
+// 7.1 ms against 6.0.)
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -32,39 +34,41 @@ namespace hipdvr {
 namespace {
 
 constexpr int kTileShapes = 3;
-constexpr int kMaxResidentPerCu = 5;
+constexpr size_t kCuLds = 160 * 1024, kWorkgroupLds = 64 * 1024;
+constexpr size_t kMarchStaticLds = sizeof(uint32_t) * kMaxTfWidth + sizeof(float) * 256;
 constexpr int kBrickSizes = 3;   // brick_log2 3, 4, 5
 
-// pixels per wavefront: 8x8, 16x4, 32x2; a workgroup is 2x2 wavefronts
-__host__ __device__ constexpr int wave_w(int tile) { return tile == 0 ? 8 : (tile == 1 ? 16 : 32); }
+// Pixels per wavefront: 8x8, 16x4, 32x2; a workgroup is 2x2 wavefronts.
+__host__ __device__ constexpr int wave_w(int tile) { return 8 << tile; }
 __host__ __device__ constexpr int wave_h(int tile) { return 64 / wave_w(tile); }
 
-// Tile queues.  The hardware hands the persistent grid's workgroups to the
+// The order of the tiles.  The hardware hands consecutive workgroups to the
 // 8 XCDs in turn (workgroup b to XCD b % 8), and each XCD has its own L2.
-// With kXcdQueues the tiles come in blocks of kBlockW x kBlockH tiles of one
-// job (blocks row by row, tiles row by row inside a block; edge blocks
-// smaller); consecutive runs of kChunk tiles of the launch's tile range are
-// dealt to the XCDs in turn, and each XCD takes its runs from a counter of
-// its own, so the tiles an XCD marches at a time form a compact column of
-// blocks whose rays share that XCD's L2.  An XCD whose runs are taken takes
-// from the others' counters.  Without it: one counter, tiles row by row.
-constexpr bool kXcdQueues = true;
-constexpr int kBlockW = 8, kBlockH = 4;
+// Tiles come in blocks of kBlockW x kBlockH tiles of one job (blocks row by
+// row, tiles row by row inside a block; edge blocks smaller); consecutive runs
+// of kChunk tiles of the launch's tile range are dealt to the XCDs in turn, so
+// the tiles an XCD marches at a time are a few compact blocks whose rays share
+// that XCD's L2, and the eight march neighbouring ones.  Blocks of 2x2 tiles:
+// 64 uneven volumes 709 us, 12 views of 512^3 6.43 ms; 4x4 695 us, 6.51 ms;
+// 8x4 824 us, 6.56 ms.
+constexpr int kBlockW = 2, kBlockH = 2;
 constexpr uint32_t kChunk = kBlockW * kBlockH;
-constexpr uint32_t kCounterStride = 32;   // counters 128 bytes apart
+constexpr uint64_t kMaxTiles = 0x3fffff00;   // of a launch: four parts each below 2^32
 
-__global__ void batch_reset_kernel(uint32_t* counter) {
-    if (threadIdx.x < kXcds) counter[threadIdx.x * kCounterStride] = 0;
+// The run that XCD x takes in round m: the round's eight runs in an order that
+// changes from round to round without a pattern, so that no XCD meets the same
+// column of an image whatever its width (dealt in a fixed order, 12 views of
+// 1024^2 took 13.1 ms, the XCDs of the middle columns marching alone for half
+// of it).
+__host__ __device__ inline uint32_t xcd_run(uint32_t x, uint32_t m) {
+    return kXcds * m + (x ^ ((m * 0x9E3779B1u) >> 29));
 }
 
-// Tiles dealt to XCD x out of total.
-__device__ __forceinline__ uint32_t xcd_tiles(uint32_t x, uint32_t total) {
-    const uint32_t chunks = (total + kChunk - 1) / kChunk;
-    if (x >= chunks) return 0;
-    const uint32_t owned = (chunks - 1 - x) / kXcds + 1;
-    uint32_t n = owned * kChunk;
-    if ((chunks - 1) % kXcds == x) n -= chunks * kChunk - total;   // its last run is the short one
-    return n;
+// Workgroups for `total` tiles in P parts each: whole rounds of runs (those
+// past the last tile leave at once).
+inline uint64_t batch_grid(uint32_t total, int parts) {
+    const uint64_t chunks = ((uint64_t)total + kChunk - 1) / kChunk;
+    return (chunks + kXcds - 1) / kXcds * kXcds * kChunk * (uint64_t)parts;
 }
 
 // Tile (tx, ty) at position lt of a job of tiles_x x tiles_y tiles in block
@@ -84,139 +88,124 @@ __device__ __forceinline__ void block_tile(uint32_t lt, uint32_t tiles_x, uint32
     tx = bx * kBlockW + r2 % bw;
 }
 
-template <bool WIDE, int SHADE, bool COUNT, int K, int TILE>
-__global__ __launch_bounds__(256) void batch_kernel(const LearnedArgs* __restrict__ jobs,
-                                                    const uint32_t* __restrict__ tile_start, uint32_t njobs,
-                                                    uint32_t total_tiles, uint32_t* __restrict__ counter,
-                                                    unsigned long long* __restrict__ counters) {
+// One workgroup per P-th of a tile, P lanes per ray (march_cell.h).  The
+// tile's 2x2 regions of 64 pixels fall into parts of 64 / P rays; wavefront w
+// marches part `part` of region w, or, where the parts of a region are
+// narrower than it, its neighbours in the same part of the tile.
+template <bool WIDE, int SHADE, bool COUNT, int P, bool LEARNED>
+__global__ __launch_bounds__(256, SHADE == 2 ? 4 : (SHADE == 1 ? (LEARNED || COUNT ? 5 : 6) : (COUNT ? 6 : 7))) void batch_kernel(
+    const LearnedArgs* __restrict__ jobs, const uint32_t* __restrict__ tile_start, uint32_t njobs,
+    uint32_t total_tiles, unsigned long long* __restrict__ counters, uint32_t tile_shape) {
+    const uint32_t block = linear_block(), slot = block / kXcds, part = slot % P, i = slot / P;
+    const uint32_t tile = xcd_run(block % kXcds, i / kChunk) * kChunk + i % kChunk;
+    if (tile >= total_tiles) return;
     __shared__ uint32_t s_tf[kMaxTfWidth];
     __shared__ float s_alpha[256];
-    __shared__ uint32_t s_tile;
-    constexpr int WW = wave_w(TILE), WH = wave_h(TILE);
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    int cur_job = -1;
+    // job of this tile: last j with tile_start[j] <= tile
+    uint32_t lo = 0, hi = njobs;
+    while (hi - lo > 1) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (tile_start[mid] <= tile) lo = mid;
+        else hi = mid;
+    }
+    const uint32_t job = __builtin_amdgcn_readfirstlane(lo);
+    const LearnedArgs& la = jobs[job];
+    const MarchArgs& a = la.m;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, ray = lane / P, sub = lane % P;
+    // a region and its parts, all powers of two
+    const int WW = 8 << tile_shape, WH = 8 >> tile_shape;
+    const int RH = ray_h<P>() < WH ? ray_h<P>() : WH, RW = 64 / P / RH, cols = WW / RW;
+    uint32_t tx, ty;
+    block_tile(tile - tile_start[job], (uint32_t)(a.grid_w + 2 * WW - 1) / (2 * WW),
+               (uint32_t)(a.grid_h + 2 * WH - 1) / (2 * WH), tx, ty);
+    // a job marches the pixels of its grid: the whole image, or (a judge's
+    // re-march: pix_block > 1) the sparse pixels judge_pixel places, written
+    // to out[gy * grid_w + gx]; their samples are not counted (the learned
+    // frame's statistics leave the judge out)
+    const bool sparse = a.pix_block > 1;
+    // the workgroup's 4 waves take neighbouring parts
+    const int q = (int)part * 4 + wave, region = q / P, rp = q % P;
+    const int gx = ((int)tx * 2 + (region & 1)) * WW + (rp % cols) * RW + ray % RW;
+    const int gy = ((int)ty * 2 + (region >> 1)) * WH + (rp / cols) * RH + ray / RW;
+    const bool inside = gx < a.grid_w && gy < a.grid_h;
+    const int px = sparse ? judge_pixel(gx, a.stride, a.pix_block, a.pix_offset) : gx;
+    const int py = sparse ? judge_pixel(gy, a.stride, a.pix_block, a.pix_offset) : gy;
+    float4 e = make_float4(0.f, 0.f, 0.f, 0.f), l = e, res = e;
+    if (inside) {
+        const size_t pix = (size_t)py * a.w + px;
+        e = a.entry[pix];
+        l = a.exit[pix];
+    }
+    const bool hit = !is_background(e, l);
     RayCounters n;
-    uint32_t drained = 0;   // (lane 0) XCD queues seen empty
-    const uint32_t my_xcd = blockIdx.x % kXcds;
-    while (true) {
-        if (tid == 0) {
-            if (kXcdQueues) {
-                uint32_t t = total_tiles;
-                for (uint32_t k = 0; k < kXcds && t == total_tiles; ++k) {
-                    const uint32_t x = (my_xcd + k) % kXcds;
-                    if (drained & (1u << x)) continue;
-                    const uint32_t i = atomicAdd(counter + x * kCounterStride, 1u);
-                    if (i < xcd_tiles(x, total_tiles)) t = (x + kXcds * (i / kChunk)) * kChunk + i % kChunk;
-                    else drained |= 1u << x;
-                }
-                s_tile = t;
-            } else {
-                s_tile = atomicAdd(counter, 1u);
-            }
-        }
-        __syncthreads();   // also: every wave has finished the previous tile
-        const uint32_t tile = __builtin_amdgcn_readfirstlane(s_tile);
-        __syncthreads();   // s_tile is read before the next iteration writes it
-        if (tile >= total_tiles) break;
-        // job of this tile: last j with tile_start[j] <= tile
-        uint32_t lo = 0, hi = njobs;
-        while (hi - lo > 1) {
-            const uint32_t mid = (lo + hi) >> 1;
-            if (tile_start[mid] <= tile) lo = mid;
-            else hi = mid;
-        }
-        const int job = (int)__builtin_amdgcn_readfirstlane(lo);
-        const LearnedArgs& la = jobs[job];
-        const MarchArgs& a = la.m;
+    if (__syncthreads_or(hit)) {   // a workgroup of background pixels needs no tables
         // a job with a stepping table marches with learned stepping
-        const bool learned = la.table != nullptr;
-        if (job != cur_job) {
-            for (int i = tid; i < a.tf_width; i += 256) s_tf[i] = a.tf[i];
-            s_alpha[tid] = learned ? la.alpha_m[tid] : a.alpha_corr[tid];
-            __syncthreads();
-            cur_job = job;
-        }
-        // a job marches the pixels of its grid: the whole image, or (a
-        // judge's re-march: pix_block > 1) the sparse pixels judge_pixel
-        // places, written to out[gy * grid_w + gx]; their samples are not
-        // counted (the learned frame's statistics leave the judge out)
-        const bool sparse = a.pix_block > 1;
-        RayCounters uncounted;
-        RayCounters& nc = sparse ? uncounted : n;
-        const uint32_t lt = tile - tile_start[job];
-        const uint32_t tiles_x = (uint32_t)(a.grid_w + 2 * WW - 1) / (2 * WW);
-        uint32_t tx = lt % tiles_x, ty = lt / tiles_x;
-        if (kXcdQueues) block_tile(lt, tiles_x, (uint32_t)(a.grid_h + 2 * WH - 1) / (2 * WH), tx, ty);
-        const int gx = (int)tx * (2 * WW) + (wave & 1) * WW + (lane % WW);
-        const int gy = (int)ty * (2 * WH) + (wave >> 1) * WH + (lane / WW);
-        if (gx < a.grid_w && gy < a.grid_h) {
-            const int px = sparse ? judge_pixel(gx, a.stride, a.pix_block, a.pix_offset) : gx;
-            const int py = sparse ? judge_pixel(gy, a.stride, a.pix_block, a.pix_offset) : gy;
-            const size_t pix = (size_t)py * a.w + px;
-            const float4 e = a.entry[pix];
-            const float4 l = a.exit[pix];
-            float4 res = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (!is_background(e, l)) {
-                // WIDE: 64-bit record addressing for every job (a volume's
-                // records exceed 4 GiB); else 32-bit buffer offsets
-                if (learned) {
-                    unsigned long long ns = 0, nsh = 0;
-                    if (a.dtype == 0) {
-                        const CellFetch<uint8_t, WIDE> f = cell_fetch_of<uint8_t, WIDE>(a);
-                        res = learned_ray<uint8_t, WIDE, SHADE != 0>(la, f, s_tf, s_alpha, px, py, e, l, ns, nsh);
-                    } else {
-                        const CellFetch<uint16_t, WIDE> f = cell_fetch_of<uint16_t, WIDE>(a);
-                        res = learned_ray<uint16_t, WIDE, SHADE != 0>(la, f, s_tf, s_alpha, px, py, e, l, ns, nsh);
-                    }
-                    ++n.rays;
-                    n.samples += ns;
-                    n.fetched += ns;
-                    n.shaded += nsh;
-                } else if (a.dtype == 0) {
+        const bool learned = LEARNED && la.table != nullptr;
+        for (int k = tid; k < a.tf_width; k += 256) s_tf[k] = a.tf[k];
+        s_alpha[tid] = learned ? la.alpha_m[tid] : a.alpha_corr[tid];
+        __syncthreads();
+        if (hit) {
+            // WIDE: 64-bit record addressing for every job (a volume's
+            // records exceed 4 GiB); else 32-bit buffer offsets
+            if (LEARNED && learned) {
+                unsigned long long ns = 0, nsh = 0;
+                if (a.dtype == 0) {
                     const CellFetch<uint8_t, WIDE> f = cell_fetch_of<uint8_t, WIDE>(a);
-                    res = cell_ray<uint8_t, WIDE, SHADE, COUNT, K>(a, f, s_tf, s_alpha, nullptr, px, py, e, l, nc);
+                    res = learned_ray<uint8_t, WIDE, SHADE != 0, P>(la, f, s_tf, s_alpha, px, py, sub, e, l, ns, nsh);
                 } else {
                     const CellFetch<uint16_t, WIDE> f = cell_fetch_of<uint16_t, WIDE>(a);
-                    res = cell_ray<uint16_t, WIDE, SHADE, COUNT, K>(a, f, s_tf, s_alpha, nullptr, px, py, e, l, nc);
+                    res = learned_ray<uint16_t, WIDE, SHADE != 0, P>(la, f, s_tf, s_alpha, px, py, sub, e, l, ns,
+                                                                     nsh);
                 }
+                ++n.rays;
+                n.fetched += (uint32_t)ns;
+                n.shaded += (uint32_t)nsh;
+            } else if (a.dtype == 0) {
+                const CellFetch<uint8_t, WIDE> f = cell_fetch_of<uint8_t, WIDE>(a);
+                res = cell_ray<uint8_t, WIDE, SHADE, COUNT, P>(a, f, s_tf, s_alpha, px, py, sub, e, l, n);
+            } else {
+                const CellFetch<uint16_t, WIDE> f = cell_fetch_of<uint16_t, WIDE>(a);
+                res = cell_ray<uint16_t, WIDE, SHADE, COUNT, P>(a, f, s_tf, s_alpha, px, py, sub, e, l, n);
             }
-            a.out[(size_t)gy * a.grid_w + gx] = res;
         }
     }
-    if (COUNT) {
-        wave_add(counters + 0, n.rays);
-        wave_add(counters + 1, n.samples);
-        wave_add(counters + 2, n.fetched);
-        wave_add(counters + 3, n.shaded);
-        wave_add_max64(counters + 4, n.slots);
-        wave_add_max64(counters + 5, n.shade_slots);
-    }
+    if (inside && sub == 0) a.out[(size_t)gy * a.grid_w + gx] = res;
+    if (sparse) n = RayCounters();
+    if (COUNT) add_counters<P>(counters, n, sub == 0);
 }
 
-typedef void (*BatchKernel)(const LearnedArgs*, const uint32_t*, uint32_t, uint32_t, uint32_t*,
-                            unsigned long long*);
+typedef void (*BatchKernel)(const LearnedArgs*, const uint32_t*, uint32_t, uint32_t, unsigned long long*,
+                            uint32_t);
 
 template <bool WIDE, int SHADE, bool COUNT>
-BatchKernel pick_kernel(int tile, int k) {
-    if (k <= 2) {
-        if (tile == 0) return batch_kernel<WIDE, SHADE, COUNT, 2, 0>;
-        if (tile == 1) return batch_kernel<WIDE, SHADE, COUNT, 2, 1>;
-        return batch_kernel<WIDE, SHADE, COUNT, 2, 2>;
-    }
-    if (tile == 0) return batch_kernel<WIDE, SHADE, COUNT, 4, 0>;
-    if (tile == 1) return batch_kernel<WIDE, SHADE, COUNT, 4, 1>;
-    return batch_kernel<WIDE, SHADE, COUNT, 4, 2>;
+BatchKernel pick_kernel(int lanes, bool learned) {
+    if constexpr (SHADE < 2)   // no learned job shades exactly
+        if (learned) return lanes == 2 ? batch_kernel<WIDE, SHADE, COUNT, 2, true> : batch_kernel<WIDE, SHADE, COUNT, 4, true>;
+    if (lanes == 2) return batch_kernel<WIDE, SHADE, COUNT, 2, false>;
+    if (lanes == 4) return batch_kernel<WIDE, SHADE, COUNT, 4, false>;
+    return batch_kernel<WIDE, SHADE, COUNT, 16, false>;
 }
 
 template <bool WIDE>
-BatchKernel kernel_for_w(int shade, bool count, int tile, int k) {
-    if (shade == 2) return count ? pick_kernel<WIDE, 2, true>(tile, k) : pick_kernel<WIDE, 2, false>(tile, k);
-    if (shade == 1) return count ? pick_kernel<WIDE, 1, true>(tile, k) : pick_kernel<WIDE, 1, false>(tile, k);
-    return count ? pick_kernel<WIDE, 0, true>(tile, k) : pick_kernel<WIDE, 0, false>(tile, k);
+BatchKernel kernel_for_w(int shade, bool count, int lanes, bool learned) {
+    if (shade == 2) return count ? pick_kernel<WIDE, 2, true>(lanes, learned) : pick_kernel<WIDE, 2, false>(lanes, learned);
+    if (shade == 1) return count ? pick_kernel<WIDE, 1, true>(lanes, learned) : pick_kernel<WIDE, 1, false>(lanes, learned);
+    return count ? pick_kernel<WIDE, 0, true>(lanes, learned) : pick_kernel<WIDE, 0, false>(lanes, learned);
 }
 
-BatchKernel kernel_for(bool wide, int shade, bool count, int tile, int k) {
-    return wide ? kernel_for_w<true>(shade, count, tile, k) : kernel_for_w<false>(shade, count, tile, k);
+// Lanes per ray of a launch of `pixels` pixels whose finest step is `step`,
+// for the configuration's batch: as frame_lanes, with the lines where a launch
+// of many jobs fills the chip.  Start of the lines, 2 / 4 lanes in us: two
+// views of 390 K pixels 916 / 488, eleven of 5.7 M 1822 / 1772, 64 volumes of
+// 16.8 M unshaded 682 / 876, 12 views of 12.6 M with Phong 5995 / 7116.
+int batch_lanes(int batch, uint64_t pixels, float step, bool learned) {
+    if (!learned && (double)pixels * step <= 100.0) return 16;
+    if (pixels <= 1500000) return 4;
+    return pixels > 6000000 ? 2 : batch;
+}
+
+BatchKernel kernel_for(bool wide, int shade, bool count, int lanes, bool learned) {
+    return wide ? kernel_for_w<true>(shade, count, lanes, learned) : kernel_for_w<false>(shade, count, lanes, learned);
 }
 
 }  // namespace
@@ -231,7 +220,6 @@ struct hipdvr_batch {
     std::vector<uint32_t> order;           // caller's index of each launch position
     int shade = 0;                         // 0 none, 1 Phong, 2 exact Phong
     bool wide = false;                     // some volume's cell records exceed 4 GiB
-    int sms = 0;
     // per brick size: device brick tables per job and the jobs' arguments
     // (march arguments, plus the stepping table of learned jobs)
     std::vector<void*> allocations;
@@ -253,13 +241,12 @@ struct hipdvr_batch {
     // re-march (its sparse grid, marched plainly into its sparse image),
     // then every job; its tile ranges per tile shape
     uint32_t n_ljobs = 0;
-    uint32_t* d_ltile_start[kTileShapes] = {nullptr, nullptr, nullptr};
-    uint32_t ltotal_tiles[kTileShapes] = {0, 0, 0};
+    uint32_t* d_ltile_start[kTileShapes] = {};
+    uint32_t ltotal_tiles[kTileShapes] = {};
     hipdvr::JudgeJob* d_judge = nullptr;
     uint32_t n_judge = 0;
-    uint32_t* d_tile_start[kTileShapes] = {nullptr, nullptr, nullptr};
-    uint32_t total_tiles[kTileShapes] = {0, 0, 0};
-    uint32_t* d_counter = nullptr;
+    uint32_t* d_tile_start[kTileShapes] = {};
+    uint32_t total_tiles[kTileShapes] = {};
     hipdvr_batch_config cfg{0, 4, 4, 0};
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
@@ -299,25 +286,24 @@ void validate_config(const hipdvr_batch_config& c) {
 void launch_batch(hipdvr_batch* b, bool count, bool learned = false) {
     hipStream_t st = ctx_stream(b->ctx);
     const int t = b->cfg.tile, bs = b->cfg.brick_log2 - 3;
-    BatchKernel k = kernel_for(b->wide, b->shade, count, t, b->cfg.batch);
-    int per_cu = 0;
-    hip_check(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)k, 256, 0), "occupancy query");
-    if (per_cu < 1) per_cu = 1;
-    // resident workgroups per CU: more rays in flight evict each other's cell
-    // records.  Default: at most five (64 uneven volumes, unshaded: 59,030
-    // frames/s at the occupancy limit, 63,436 at five, 62,716 at four), three
-    // when records need 64-bit addressing (8 GiB volume, 8 views of 4K with
-    // Phong: 234 ms at three against 277 ms at four)
-    const int cap = b->cfg.resident > 0 ? b->cfg.resident : (b->wide ? 3 : kMaxResidentPerCu);
-    if (per_cu > cap) per_cu = cap;
+    uint64_t pixels = 0;
+    float step = b->jobs[0].params.step;
+    for (const hipdvr_batch_job& j : b->jobs) {
+        pixels += (uint64_t)j.w * j.h;
+        step = std::min(step, j.params.step);
+    }
+    const int lanes = batch_lanes(b->cfg.batch, pixels, step, learned);
+    BatchKernel k = kernel_for(b->wide, b->shade, count, lanes, learned);
+    // a residency limit: dynamic LDS up to a share of the CU's 160 KiB
+    size_t pad = 0;
+    if (b->cfg.resident > 0 && kCuLds / b->cfg.resident > kMarchStaticLds)
+        pad = kCuLds / b->cfg.resident - kMarchStaticLds;
+    if (pad > kWorkgroupLds - kMarchStaticLds) pad = kWorkgroupLds - kMarchStaticLds;
     const uint32_t total = learned ? b->ltotal_tiles[t] : b->total_tiles[t];
-    uint32_t grid = (uint32_t)(b->sms * per_cu);
-    if (grid > total) grid = total ? total : 1;
-    hipLaunchKernelGGL(batch_reset_kernel, dim3(1), dim3(64), 0, st, b->d_counter);
-    hipLaunchKernelGGL(k, dim3(grid), dim3(256), 0, st,
+    hipLaunchKernelGGL(k, linear_grid(batch_grid(total, lanes)), dim3(256), pad, st,
                        (const LearnedArgs*)(learned ? b->d_largs[bs] : b->d_args[bs]),
                        (const uint32_t*)(learned ? b->d_ltile_start[t] : b->d_tile_start[t]),
-                       learned ? b->n_ljobs : (uint32_t)b->jobs.size(), total, b->d_counter, b->ctx->d_counters);
+                       learned ? b->n_ljobs : (uint32_t)b->jobs.size(), total, b->ctx->d_counters, (uint32_t)t);
     hip_check(hipGetLastError(), "batch launch");
 }
 
@@ -352,9 +338,6 @@ int hipdvr_batch_create(hipdvr_ctx* ctx, const hipdvr_batch_job* jobs, uint32_t 
         b->ctx = ctx;
         b->shade = shade;
         try {
-            int dev = 0;
-            hip_check(hipGetDevice(&dev), "hipGetDevice");
-            hip_check(hipDeviceGetAttribute(&b->sms, hipDeviceAttributeMultiprocessorCount, dev), "device attribute");
             // largest estimated cost first
             std::vector<uint32_t> order(n);
             std::iota(order.begin(), order.end(), 0u);
@@ -384,32 +367,17 @@ int hipdvr_batch_create(hipdvr_ctx* ctx, const hipdvr_batch_job* jobs, uint32_t 
                         nb[k] = (v->desc.dims[k] + (1u << bl) - 1) >> bl;
                         count *= nb[k];
                     }
-                    uint2* mm = dev_alloc<uint2>(b, count * sizeof(uint2));
-                    uint8_t* occ = dev_alloc<uint8_t>(b, count);
-                    const uint32_t words = (uint32_t)((count + 31) / 32);
-                    uint32_t* bits = dev_alloc<uint32_t>(b, (size_t)words * 4);
+                    // ranges, skip grid and its scratch
+                    uint2* mm = dev_alloc<uint2>(b, count * (sizeof(uint2) + 2));
+                    uint8_t* skip = (uint8_t*)(mm + count);
                     launch_brick_minmax(v, bl, nb, mm, st);
-                    OccArgs o;
-                    o.minmax = mm;
-                    o.occ = occ;
-                    o.count = count;
-                    o.dtype = v->desc.dtype;
-                    o.rwm_scale = v->desc.rwm_scale;
-                    o.rwm_offset = v->desc.rwm_offset;
-                    o.dom_lo = j.tf->domain_lo;
-                    o.dom_hi = j.tf->domain_hi;
-                    o.tf_width = (int32_t)j.tf->width;
-                    o.alpha_prefix = j.tf->d_alpha_prefix;
-                    o.bits = bits;
-                    launch_occupancy(o, st);
+                    launch_skip_grid(occupancy_args(v, j.tf, mm, count), nb, skip, skip + count, st);
                     MarchArgs& a = args[i].m;
                     fill_march_args(a, v, j.tf, &j.params, j.d_entry, j.d_exit, j.d_out, j.w, j.h, nullptr);
                     a.cells = v->d_cells;
-                    a.brick_log2 = bl;
-                    for (int k = 0; k < 3; ++k) a.nbricks[k] = nb[k];
-                    a.brick_occ = occ;
-                    a.occ_bits = bits;
-                    a.occ_words = words;
+                    a.skip = skip;
+                    a.skip_log2 = bl;
+                    for (int k = 0; k < 3; ++k) a.nskip[k] = nb[k];
                 }
                 b->d_args[bs] = dev_alloc<LearnedArgs>(b, n * sizeof(LearnedArgs));
                 hip_check(hipMemcpyAsync(b->d_args[bs], args.data(), n * sizeof(LearnedArgs), hipMemcpyHostToDevice,
@@ -422,7 +390,7 @@ int hipdvr_batch_create(hipdvr_ctx* ctx, const hipdvr_batch_job* jobs, uint32_t 
                 const uint32_t tw = 2 * wave_w(t), th = 2 * wave_h(t);
                 for (uint32_t i = 0; i < n; ++i) {
                     const uint64_t tiles = (uint64_t)((b->jobs[i].w + tw - 1) / tw) * ((b->jobs[i].h + th - 1) / th);
-                    if (start[i] + tiles > 0xfffffff0ull) fail(HIPDVR_ERR_UNSUPPORTED, "batch too large");
+                    if (start[i] + tiles > kMaxTiles) fail(HIPDVR_ERR_UNSUPPORTED, "batch too large");
                     start[i + 1] = start[i] + (uint32_t)tiles;
                 }
                 b->total_tiles[t] = start[n];
@@ -431,7 +399,6 @@ int hipdvr_batch_create(hipdvr_ctx* ctx, const hipdvr_batch_job* jobs, uint32_t 
                           "upload");
                 hip_check(hipStreamSynchronize(st), "hipStreamSynchronize");
             }
-            b->d_counter = dev_alloc<uint32_t>(b, kXcds * kCounterStride * 4);
             b->learned.assign(n, nullptr);
             b->plain_learned.assign(n, 0);
             hip_check(hipGetLastError(), "batch setup");
@@ -544,7 +511,7 @@ int hipdvr_batch_autotune(hipdvr_batch* b, uint32_t reps, hipdvr_batch_config* b
             return ms / (float)reps;
         };
         try {
-            for (int t = 0; t < kTileShapes; ++t)
+            for (int t = 0; t < 3; ++t)
                 for (int bl = 3; bl <= 5; ++bl)
                     for (int k : {2, 4}) {
                         const float ms = time_config(hipdvr_batch_config{t, bl, k, 0});
@@ -681,7 +648,7 @@ int hipdvr_batch_set_learned(hipdvr_batch* b, hipdvr_learned* const* learned, ui
             for (uint32_t k = 0; k < nl; ++k) {
                 const MarchArgs& m = ljobs[0][k].m;
                 const uint64_t tiles = (uint64_t)((m.grid_w + tw - 1) / tw) * ((m.grid_h + th - 1) / th);
-                if (lstart[t][k] + tiles > 0xfffffff0ull) fail(HIPDVR_ERR_UNSUPPORTED, "batch too large");
+                if (lstart[t][k] + tiles > kMaxTiles) fail(HIPDVR_ERR_UNSUPPORTED, "batch too large");
                 lstart[t][k + 1] = lstart[t][k] + (uint32_t)tiles;
             }
         }
@@ -736,7 +703,7 @@ int hipdvr_batch_launch_learned(hipdvr_batch* b, hipdvr_learned_stats* stats) {
         const bool timed = ctx_timing_start(b->ctx);
         if (!b->d_largs[0]) fail(HIPDVR_ERR_INVALID, "hipdvr_batch_set_learned has not been called");
         // 1. the judges' plain re-marches of the learned views' sparse pixels
-        //    and every job, learned or plain, in one persistent launch
+        //    and every job, learned or plain, in one launch
         launch_batch(b, count, true);
         if (any) {
             // 2. the judges of all learned views in one launch, then per
@@ -749,7 +716,7 @@ int hipdvr_batch_launch_learned(hipdvr_batch* b, hipdvr_learned_stats* stats) {
                 MarchArgs fb = b->h_args[bs][i].m;
                 fb.counters = nullptr;
                 fb.cond_flag = b->d_flag[i];
-                launch_march_cell(fb, fb.dtype, shade, false, j.volume->cells_wide, default_batch(shade), st);
+                launch_march_cell(fb, fb.dtype, shade, false, j.volume->cells_wide, 0, st);
             }
         }
         hip_check(hipGetLastError(), "batched learned launch");

@@ -73,19 +73,42 @@ __host__ __device__ constexpr uint32_t cell_axis_mask(int i) {
     return m << 3;
 }
 
+// Product of two numbers below 2^24 (full rate on the VALU, a quarter of it
+// for 32-bit factors).  Brick numbers stay below it: a volume's records are
+// capped at 96 GiB, 2^18 bricks of 512 KiB, and its 8^3 skip bricks at 2^24.
+__host__ __device__ __forceinline__ uint32_t cell_mul24(uint32_t a, uint32_t b) {
+#ifdef __HIP_DEVICE_COMPILE__
+    return __umul24(a, b);
+#else
+    return a * b;
+#endif
+}
+
 // Record index of cell lo (nbx, nby: bricks along x and y).
 template <typename off_t>
 __host__ __device__ __forceinline__ off_t cell_index(const uint32_t lo[3], uint32_t nbx, uint32_t nby) {
-    uint32_t g[3], local = 0;
+    constexpr uint32_t S = kCellBrickLog2 + 1;   // voxels per brick edge, log2
+    const uint32_t brick = cell_mul24(cell_mul24(lo[2] >> S, nby) + (lo[1] >> S), nbx) + (lo[0] >> S);
+    uint32_t local = 0;
+    if (kCellMorton) {
 #pragma unroll
-    for (int i = 0; i < 3; ++i) {
-        g[i] = lo[i] >> 1;
-        const uint32_t o = g[i] & kCellBrickMask;
-        local |= (kCellMorton ? cell_spread(o) << (3 + i) : o << (3 + i * kCellBrickLog2)) | ((lo[i] & 1u) << i);
+        for (int i = 0; i < 3; ++i)
+            local |= (cell_spread((lo[i] >> 1) & kCellBrickMask) << (3 + i)) | ((lo[i] & 1u) << i);
+    } else {
+        // the axes' group bits side by side and the parities below them, each
+        // merged by a bit-field insert: what a shift leaves of a coordinate
+        // above or below its field is overwritten by its neighbour's
+        const uint32_t bits = kCellBrickLog2;
+        const uint32_t m0 = (1u << (3 + bits)) - 1, m1 = (1u << (3 + 2 * bits)) - 1, m2 = (1u << (3 + 3 * bits)) - 1;
+        uint32_t v = lo[0] << 2;
+        v = (v & m0) | ((lo[1] << (2 + bits)) & ~m0);
+        v = (v & m1) | ((lo[2] << (2 + 2 * bits)) & ~m1);
+        v = (lo[0] & 1u) | (v & ~1u);
+        v = ((lo[1] << 1) & 2u) | (v & ~2u);
+        v = ((lo[2] << 2) & 4u) | (v & ~4u);
+        local = v & m2;
     }
-    const uint32_t brick = ((g[2] >> kCellBrickLog2) * nby + (g[1] >> kCellBrickLog2)) * nbx +
-                           (g[0] >> kCellBrickLog2);
-    return ((off_t)brick << kCellBrickRecLog2) + (off_t)local;
+    return ((off_t)brick << kCellBrickRecLog2) | (off_t)local;
 }
 
 // Records of the cells lo - e_i and lo + e_i from the record index `own` of

@@ -50,7 +50,8 @@ void launch_trace(const LearnedArgs& la, float* err, unsigned int* visits, hipSt
 void launch_targets(const float* err, const unsigned int* visits, const float* feat, uint32_t rows,
                     float tau_skip, float tau_step, float* out_x, float* out_t, unsigned int* count,
                     uint32_t capacity, hipStream_t st);
-void launch_learned(const LearnedArgs& la, bool phong, bool count, bool wide, hipStream_t st);
+// lanes per ray: 2 or 4
+void launch_learned(const LearnedArgs& la, bool phong, bool count, bool wide, int lanes, hipStream_t st);
 
 // For batched launches (batch.hip): the judge's sparse grid of a w x h image
 // (host arithmetic), the options with their defaults, the stepping fields of

@@ -215,8 +215,6 @@ struct hipdvr_learned {
     bool gains = true;               // the prepared table departs from the plain march
     float4* d_sparse = nullptr;      // sparse plain image
     size_t sparse_cap = 0;
-    float4* d_seg = nullptr;         // its ray segments
-    size_t seg_cap = 0;
     float* d_sse = nullptr;
     int* d_flag = nullptr;
     unsigned int* d_count = nullptr;
@@ -278,14 +276,6 @@ SparseGrid sparse_grid(hipdvr_learned* l, uint32_t w, uint32_t h, uint32_t strid
         hip_check(hipMalloc((void**)&l->d_sparse, need), "hipMalloc(sparse)");
         l->sparse_cap = need;
     }
-    const size_t seg = sparse_segment_bytes((uint32_t)g.w * (uint32_t)g.h);
-    if (seg > l->seg_cap) {
-        if (l->d_seg) (void)hipFree(l->d_seg);
-        l->d_seg = nullptr;
-        l->seg_cap = 0;
-        hip_check(hipMalloc((void**)&l->d_seg, seg), "hipMalloc(sparse segments)");
-        l->seg_cap = seg;
-    }
     return g;
 }
 
@@ -301,7 +291,9 @@ void launch_sparse(hipdvr_learned* l, hipdvr_volume* vol, const hipdvr_tf* tf, c
     sp.stride = (int32_t)g.stride;
     sp.pix_block = (int32_t)g.block;
     sp.pix_offset = (int32_t)g.offs;
-    launch_sparse_remarch(sp, vol->desc.dtype, shade, vol->cells_wide, l->d_seg, st);
+    // 1/64 of the rays: sixteen lanes each, so that the longest one does not
+    // outlast the learned march beside it
+    launch_march_cell(sp, vol->desc.dtype, shade, false, vol->cells_wide, 8, st);
 }
 
 void free_learned(hipdvr_learned* l) {
@@ -318,7 +310,6 @@ void free_learned(hipdvr_learned* l) {
     (void)hipFree(l->d_nz_prefix);
     (void)hipFree(l->d_alpha_m);
     (void)hipFree(l->d_sparse);
-    (void)hipFree(l->d_seg);
     (void)hipFree(l->d_sse);
     (void)hipFree(l->d_flag);
     (void)hipFree(l->d_count);
@@ -581,7 +572,7 @@ int hipdvr_render_learned_device(hipdvr_learned* l, const hipdvr_tf* tf, const f
         ctx_set_device(l->ctx);
         hipStream_t st = ctx_stream(l->ctx);
         hipdvr_volume* vol = const_cast<hipdvr_volume*>(l->vol);
-        ensure_occupancy(l->ctx, vol, tf);
+        ensure_skip(l->ctx, vol, tf);
         const SparseGrid sg = sparse_grid(l, w, h, (uint32_t)opts.remarch_stride);
         const uint32_t stride = sg.stride, offs = sg.offs;
         const int swc = sg.w, shc = sg.h;
@@ -597,7 +588,7 @@ int hipdvr_render_learned_device(hipdvr_learned* l, const hipdvr_tf* tf, const f
             ensure_cells(vol, st);
             MarchArgs pa;
             fill_march_args(pa, vol, tf, prm, d_entry, d_exit, d_out, w, h, count ? l->ctx->d_counters : nullptr);
-            launch_march_cell(pa, vol->desc.dtype, shade, count, vol->cells_wide, default_batch(shade), st);
+            launch_march_cell(pa, vol->desc.dtype, shade, count, vol->cells_wide, 0, st);
             hip_check(hipGetLastError(), "learned render launch");
             if (timed0) ctx_timing_stop(l->ctx);
             if (count) {
@@ -622,7 +613,7 @@ int hipdvr_render_learned_device(hipdvr_learned* l, const hipdvr_tf* tf, const f
         LearnedArgs la;
         fill_learned_args(la, l, tf, prm, d_entry, d_exit, d_out, w, h);
         la.m.cells = vol->d_cells;
-        launch_learned(la, phong, count, vol->cells_wide, st);
+        launch_learned(la, phong, count, vol->cells_wide, frame_lanes(prm->batch, (uint64_t)w * h, prm->step), st);
         hip_check(hipStreamWaitEvent(st, l->join, 0), "hipStreamWaitEvent");
         // 3. judge: flag = PSNR below the floor
         const float mse_max = powf(10.f, -opts.psnr_floor / 10.f);
@@ -633,7 +624,7 @@ int hipdvr_render_learned_device(hipdvr_learned* l, const hipdvr_tf* tf, const f
         MarchArgs fb;
         fill_march_args(fb, vol, tf, prm, d_entry, d_exit, d_out, w, h, nullptr);
         fb.cond_flag = l->d_flag;
-        launch_march_cell(fb, vol->desc.dtype, shade, false, vol->cells_wide, default_batch(shade), st);
+        launch_march_cell(fb, vol->desc.dtype, shade, false, vol->cells_wide, 0, st);
         hip_check(hipGetLastError(), "learned render launch");
         if (timed) ctx_timing_stop(l->ctx);
         if (count) {
@@ -684,7 +675,7 @@ int hipdvr_learned_sparse_remarch(hipdvr_learned* l, const hipdvr_tf* tf, const 
         ctx_set_device(l->ctx);
         hipStream_t st = ctx_stream(l->ctx);
         hipdvr_volume* vol = const_cast<hipdvr_volume*>(l->vol);
-        ensure_occupancy(l->ctx, vol, tf);
+        ensure_skip(l->ctx, vol, tf);
         ensure_cells(vol, st);
         const SparseGrid g = sparse_grid(l, w, h, (uint32_t)opts.remarch_stride);
         const int shade = prm->shading == HIPDVR_SHADE_PHONG ? (prm->exact_shading ? 2 : 1) : 0;

@@ -409,57 +409,71 @@ void launch_targets(const float* err, const unsigned int* visits, const float* f
                        tau_skip, tau_step, out_x, out_t, count, capacity);
 }
 
-template <typename T, bool WIDE, bool PHONG, bool COUNT>
-__global__ __launch_bounds__(256) void learned_kernel(const LearnedArgs la) {
-    __shared__ uint32_t s_tf[kMaxTfWidth];
-    __shared__ float s_alpha[256];   // opacity correction of the base step
+// Tiles and lanes as march_cell_kernel.
+template <typename T, bool WIDE, bool PHONG, bool COUNT, int P>
+__global__ __launch_bounds__(256, PHONG ? 5 : 6) void learned_kernel(const LearnedArgs la) {
     const MarchArgs& a = la.m;
-    for (int i = threadIdx.x; i < a.tf_width; i += 256) s_tf[i] = a.tf[i];
-    s_alpha[threadIdx.x] = la.alpha_m[threadIdx.x];
-    __syncthreads();
     const uint32_t tiles_x = (a.w + 15) / 16;
     const uint32_t tiles_y = (a.h + 15) / 16;
+    const uint32_t block = linear_block(), slot = block / kXcds, part = slot % P;
     uint32_t tile_x, tile_y;   // XCD-compact tile order (xcd_tile)
-    const bool has_tile = xcd_tile(blockIdx.x, tiles_x, tiles_y, tile_x, tile_y);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int px = (int)tile_x * 16 + (wave & 1) * 8 + (lane & 7);
-    const int py = (int)tile_y * 16 + (wave >> 1) * 8 + (lane >> 3);
-    const CellFetch<T, WIDE> f = cell_fetch_of<T, WIDE>(a);
+    if (!xcd_tile((slot / P) * kXcds + block % kXcds, tiles_x, tiles_y, tile_x, tile_y)) return;
+    __shared__ uint32_t s_tf[kMaxTfWidth];
+    __shared__ float s_alpha[256];   // opacity correction of the base step
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, ray = lane / P, sub = lane % P;
+    constexpr int RW = ray_w<P>(), RH = ray_h<P>(), PX = 16 / (2 * RW);
+    const int px = (int)tile_x * 16 + ((int)(part % PX) * 2 + (wave & 1)) * RW + ray % RW;
+    const int py = (int)tile_y * 16 + ((int)(part / PX) * 2 + (wave >> 1)) * RH + ray / RW;
+    const bool inside = px < a.w && py < a.h;
+    const size_t pix = (size_t)py * a.w + px;
+    float4 e = make_float4(0.f, 0.f, 0.f, 0.f), l = e, res = e;
+    if (inside) {
+        e = a.entry[pix];
+        l = a.exit[pix];
+    }
+    const bool hit = !is_background(e, l);
     unsigned long long n_samples = 0, n_shaded = 0;
-    if (has_tile && px < a.w && py < a.h) {
-        const size_t pix = (size_t)py * a.w + px;
-        const float4 e = a.entry[pix], l = a.exit[pix];
-        float4 res = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (!is_background(e, l)) res = learned_ray<T, WIDE, PHONG>(la, f, s_tf, s_alpha, px, py, e, l, n_samples, n_shaded);
-        a.out[pix] = res;
+    if (__syncthreads_or(hit)) {
+        for (int i = threadIdx.x; i < a.tf_width; i += 256) s_tf[i] = a.tf[i];
+        s_alpha[threadIdx.x] = la.alpha_m[threadIdx.x];
+        __syncthreads();
+        const CellFetch<T, WIDE> f = cell_fetch_of<T, WIDE>(a);
+        if (hit)
+            res = learned_ray<T, WIDE, PHONG, P>(la, f, s_tf, s_alpha, px, py, sub, e, l, n_samples, n_shaded);
     }
+    if (inside && sub == 0) a.out[pix] = res;
     if (COUNT) {
-        wave_add(a.counters + 1, n_samples);
-        wave_add(a.counters + 3, n_shaded);
+        wave_add(a.counters + 1, sub == 0 ? n_samples : 0);
+        wave_add(a.counters + 3, sub == 0 ? n_shaded : 0);
     }
 }
 
-template <typename T, bool WIDE>
-static void launch_learned_t(const LearnedArgs& la, bool phong, bool count, dim3 grid, hipStream_t st) {
+template <typename T, bool WIDE, int P>
+static void launch_learned_t(const LearnedArgs& la, bool phong, bool count, hipStream_t st) {
+    const dim3 grid = linear_grid((uint64_t)xcd_tile_grid((la.m.w + 15) / 16, (la.m.h + 15) / 16) * P);
     if (phong) {
-        if (count) hipLaunchKernelGGL((learned_kernel<T, WIDE, true, true>), grid, dim3(256), 0, st, la);
-        else hipLaunchKernelGGL((learned_kernel<T, WIDE, true, false>), grid, dim3(256), 0, st, la);
+        if (count) hipLaunchKernelGGL((learned_kernel<T, WIDE, true, true, P>), grid, dim3(256), 0, st, la);
+        else hipLaunchKernelGGL((learned_kernel<T, WIDE, true, false, P>), grid, dim3(256), 0, st, la);
     } else {
-        const size_t shm = unshaded_dyn_lds(0);   // five workgroups per CU
-        if (count) hipLaunchKernelGGL((learned_kernel<T, WIDE, false, true>), grid, dim3(256), shm, st, la);
-        else hipLaunchKernelGGL((learned_kernel<T, WIDE, false, false>), grid, dim3(256), shm, st, la);
+        if (count) hipLaunchKernelGGL((learned_kernel<T, WIDE, false, true, P>), grid, dim3(256), 0, st, la);
+        else hipLaunchKernelGGL((learned_kernel<T, WIDE, false, false, P>), grid, dim3(256), 0, st, la);
     }
 }
 
-void launch_learned(const LearnedArgs& la, bool phong, bool count, bool wide, hipStream_t st) {
-    const dim3 grid(xcd_tile_grid((la.m.w + 15) / 16, (la.m.h + 15) / 16));
+template <int P>
+static void launch_learned_p(const LearnedArgs& la, bool phong, bool count, bool wide, hipStream_t st) {
     if (la.u16) {
-        if (wide) launch_learned_t<uint16_t, true>(la, phong, count, grid, st);
-        else launch_learned_t<uint16_t, false>(la, phong, count, grid, st);
+        if (wide) launch_learned_t<uint16_t, true, P>(la, phong, count, st);
+        else launch_learned_t<uint16_t, false, P>(la, phong, count, st);
     } else {
-        if (wide) launch_learned_t<uint8_t, true>(la, phong, count, grid, st);
-        else launch_learned_t<uint8_t, false>(la, phong, count, grid, st);
+        if (wide) launch_learned_t<uint8_t, true, P>(la, phong, count, st);
+        else launch_learned_t<uint8_t, false, P>(la, phong, count, st);
     }
+}
+
+void launch_learned(const LearnedArgs& la, bool phong, bool count, bool wide, int lanes, hipStream_t st) {
+    if (lanes <= 2) launch_learned_p<2>(la, phong, count, wide, st);
+    else launch_learned_p<4>(la, phong, count, wide, st);
 }
 
 // ---------------------------------------------------------------------------

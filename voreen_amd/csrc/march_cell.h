@@ -1,5 +1,5 @@
 // march_cell.h -- device code of the cell-record ray march, shared by the
-// per-frame kernel (march_cell.hip) and the batched persistent kernel
+// per-frame kernel (march_cell.hip) and the batched kernel
 // (batch.hip).
 //
 // The record of cell (x, y, z) holds the eight voxels of its trilinear
@@ -17,9 +17,9 @@
 // the reference-layout kernel (march_ref.hip, restating
 // CPURaycaster::directRendering, cpuraycaster.cpp:210-326), so the image is
 // bit-identical to it, shaded or not.  Empty-space skipping is the exact
-// brick fast-forward of the bricked kernel; the samples after a non-empty
-// sample are fetched K at a time (their loads in flight together) and
-// composited in order; a sample fetched past early termination is dropped.
+// fast-forward of the bricked kernel over the skip grid (volume.h); P lanes
+// march a ray together, one sample each, and composite in order; a sample
+// fetched past early termination is dropped.
 #pragma once
 
 #include <type_traits>
@@ -170,8 +170,8 @@ __device__ __forceinline__ void cell_gradient(const CellFetch<T, WIDE>& f, const
     }
 }
 
-// Interior central differences from the cell records: when every axis has
-// u_i in [1, dim_i - 3) and a proper fraction, the six lookups at +-1 voxel
+// Interior central differences from the cell records at unclamped voxel
+// position u: when every axis has u_i in [1, dim_i - 3) and a proper fraction, the six lookups at +-1 voxel
 // have the sample's own weights p, and their footprints are the sample's
 // corner planes plus the outer planes lo-1 and lo+2 (records of the cells
 // lo -+ e_i).  Equal to the six-lookup form up to float rounding (for the
@@ -184,15 +184,14 @@ __device__ __forceinline__ void cell_gradient(const CellFetch<T, WIDE>& f, const
 // cell_layout.h).  Returns false (and leaves gr) outside the interior.
 template <typename T, bool WIDE>
 __device__ __forceinline__ bool cell_gradient_interior(const CellFetch<T, WIDE>& f, const MarchArgs& a,
-                                                       const float s[3],
+                                                       const float u[3],
                                                        const typename CellFetch<T, WIDE>::rec_t& rec,
                                                        typename CellFetch<T, WIDE>::off_t own, const float p[3],
                                                        float gr[3]) {
     typedef typename CellFetch<T, WIDE>::off_t off_t;
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
-        const float u = (a.fdims[i] * s[i]) + (-0.5f);
-        if (!(u >= 1.0f) || !(u + 3.0f < a.fdims[i]) || !(p[i] > 0.0f)) return false;
+        if (!(u[i] >= 1.0f) || !(u[i] + 3.0f < a.fdims[i]) || !(p[i] > 0.0f)) return false;
     }
     off_t nb[6];
 #pragma unroll
@@ -244,175 +243,270 @@ __device__ __forceinline__ bool cell_gradient_interior(const CellFetch<T, WIDE>&
     return true;
 }
 
-// Per-ray counters of a march (COUNT builds).
+// Counters of a lane (COUNT builds); a lane marches few enough samples for 32
+// bits, the sums over the launch have 64.
 struct RayCounters {
-    unsigned long long rays = 0, samples = 0, fetched = 0, shaded = 0, slots = 0, shade_slots = 0;
+    uint32_t rays = 0, skipped = 0, fetched = 0, shaded = 0, passes = 0, shade_passes = 0;
 };
 
-// Occupancy bit words staged in LDS by the per-frame kernel up to this count
-// (4 KiB: 32768 bricks, e.g. 512^3 at 16^3 bricks).
-constexpr uint32_t kMaxLdsOccWords = 1024;
+// Adds a lane's counters to the launch's, the wavefront marching 64 / P rays
+// with P lanes each (every lane of a ray holds its counts).  Slots: samples
+// its rays could have taken, a skipped sample counting as one.
+template <int P>
+__device__ __forceinline__ void add_counters(unsigned long long* c, const RayCounters& n, bool own) {
+    wave_add(c + 0, own ? n.rays : 0);
+    wave_add(c + 1, own ? n.skipped + n.fetched : 0);
+    wave_add(c + 2, own ? n.fetched : 0);
+    wave_add(c + 3, own ? n.shaded : 0);
+    wave_add_max64(c + 4, n.passes * P + n.skipped, 64 / P);
+    wave_add_max64(c + 5, n.shade_passes * P, 64 / P);
+}
 
-// One ray of the cell march from entry point e to exit point l (neither the
-// background): returns the composited RGBA.  SHADE: 0 none, 1 Phong with the
-// interior gradient and the hardware-approximate lighting terms (within the
-// oracle's tolerance), 2 Phong bit-identical to the reference-layout kernel.  s_tf / s_alpha are the TF and
-// the opacity-correction table in LDS; a may live in kernel arguments or in
-// global memory (batched launches).
+// Lanes per ray.  P neighbouring lanes of a wavefront (1, 2, 4, 8 or 16)
+// march one ray together: in every pass lane `sub` of the ray fetches,
+// classifies and shades sample `sub` of the next P, and all P lanes then
+// composite the P results in order, so each lane holds the ray's state and
+// every branch of the ray is taken by its P lanes alike.  The results equal
+// the one-lane march bit for bit.  A ray is one dependent chain of memory
+// round trips and several hundred instructions per pass; P lanes cut it P
+// times, and neighbouring lanes read neighbouring samples, mostly of one
+// record group, in one load.  sub_value reads lane j's value (a move within
+// the VALU, no LDS).  What that gives is in kernels.h (frame_lanes); with six
+// wavefronts per SIMD, which one sample per lane leaves the registers for,
+// 512^3 / 1024^2 with Phong went from 1.04 ms (two samples in flight in one
+// lane, four wavefronts) to 0.68.
+template <int CTRL>
+__device__ __forceinline__ float dpp_move(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+// value of lane j of the row of 16
+__device__ __forceinline__ float row_value(float v, int j) {
+    switch (j) {
+        case 0: return dpp_move<0x150>(v);
+        case 1: return dpp_move<0x151>(v);
+        case 2: return dpp_move<0x152>(v);
+        case 3: return dpp_move<0x153>(v);
+        case 4: return dpp_move<0x154>(v);
+        case 5: return dpp_move<0x155>(v);
+        case 6: return dpp_move<0x156>(v);
+        case 7: return dpp_move<0x157>(v);
+        case 8: return dpp_move<0x158>(v);
+        case 9: return dpp_move<0x159>(v);
+        case 10: return dpp_move<0x15a>(v);
+        case 11: return dpp_move<0x15b>(v);
+        case 12: return dpp_move<0x15c>(v);
+        case 13: return dpp_move<0x15d>(v);
+        case 14: return dpp_move<0x15e>(v);
+        default: return dpp_move<0x15f>(v);
+    }
+}
+template <int P>
+__device__ __forceinline__ float sub_value(float v, int j) {
+    static_assert(P == 1 || P == 2 || P == 4 || P == 8 || P == 16, "lanes per ray");
+    if (P == 1) return v;
+    if (P == 2) return j == 0 ? dpp_move<0xA0>(v) : dpp_move<0xF5>(v);   // quad permutations
+    if (P == 4) return j == 0 ? dpp_move<0x00>(v) : j == 1 ? dpp_move<0x55>(v) : j == 2 ? dpp_move<0xAA>(v)
+                                                                                       : dpp_move<0xFF>(v);
+    if (P == 8) return (threadIdx.x & 8) ? row_value(v, j + 8) : row_value(v, j);
+    return row_value(v, j);
+}
+template <int P>
+__device__ __forceinline__ uint32_t sub_value(uint32_t v, int j) {
+    return __float_as_uint(sub_value<P>(__uint_as_float(v), j));
+}
+
+// Counts one sample of a pass (COUNT builds): cj its opacity (-1: past the
+// ray's end), A the ray's before it.
+template <int SHADE>
+__device__ __forceinline__ void count_sample(RayCounters& n, float cj, float A) {
+    const bool on = cj >= 0.0f && A < kErtOpacity;
+    n.fetched += on ? 1 : 0;
+    if (SHADE) n.shaded += on && cj > 0.0f ? 1 : 0;
+}
+
+// The place of a wavefront's rays in the image: 64 / P rays, ray_w<P>() wide.
+template <int P>
+__host__ __device__ constexpr int ray_w() { return P <= 2 ? 8 : (P <= 8 ? 4 : 2); }
+template <int P>
+__host__ __device__ constexpr int ray_h() { return 64 / P / ray_w<P>(); }
+
 // The sample loop of one ray from state (t, loop, r, g, bb, A) up to sample
-// index cap (exclusive) or the ray's end; returns true when the ray is
-// finished (past tend, or terminated early).
-template <typename T, bool WIDE, int SHADE, bool COUNT, int K>
-__device__ __forceinline__ bool cell_march(const MarchArgs& a, const CellFetch<T, WIDE>& f, const uint32_t* s_tf,
-                                           const float* s_alpha, const uint32_t* s_occ, int px, int py,
-                                           const float first[3], const float dir[3], float tend, int cap, float& t,
-                                           int& loop, float& r, float& g, float& bb, float& A, RayCounters& n) {
+// index cap (exclusive) or the ray's end.  SHADE: 0 none, 1 Phong with the
+// interior gradient and the hardware-approximate lighting terms (within the
+// oracle's tolerance), 2 Phong bit-identical to the reference-layout kernel.
+// s_tf / s_alpha are the TF and the opacity-correction table in LDS; a may
+// live in kernel arguments or in global memory (batched launches).  `sub` is
+// this lane's place among the ray's P lanes.
+//
+// The skip grid is asked only after a pass that composited nothing: inside
+// visible matter there is nothing to skip, and the grid's byte is a memory
+// round trip ahead of the sample's own.
+template <typename T, bool WIDE, int SHADE, bool COUNT, int P>
+__device__ __forceinline__ void cell_march(const MarchArgs& a, const CellFetch<T, WIDE>& f, const uint32_t* s_tf,
+                                           const float* s_alpha, int px, int py, int sub, const float first[3],
+                                           const float dir[3], float tend, int cap, float& t, int& loop, float& r,
+                                           float& g, float& bb, float& A, RayCounters& n) {
     typedef typename CellFetch<T, WIDE>::rec_t rec_t;
-    const uint32_t bl = a.brick_log2;
-    const uint32_t nbx = a.nbricks[0], nbxy = a.nbricks[0] * a.nbricks[1];
+    const uint32_t bl = a.skip_log2;
     uint32_t cur_brick = 0xffffffffu;
-    bool cur_occ = false;
+    uint32_t empty = 0;   // the skip grid's entry of the current brick
     float t_lim = 0.0f;
+    bool probe = true;
     // reciprocals for the empty-brick bound (a bound with a 0.05-voxel
     // margin needs no correctly rounded quotient); an axis with |dir| below
     // 1e-30 cannot move 0.05 voxel within a ray and bounds nothing
     float rdir[3], rfd[3];
+    // a degenerate ray (its direction or start is not a number): the clamps
+    // below map its positions into the volume, its intensities are NaN
+    bool nan_ray = false;
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
         rdir[i] = fabsf(dir[i]) < 1e-30f ? 0.0f : __builtin_amdgcn_rcpf(dir[i]);
         rfd[i] = __builtin_amdgcn_rcpf(a.fdims[i]);
+        nan_ray = nan_ray || !(fabsf(dir[i]) < INFINITY) || first[i] != first[i];
     }
     bool finished = false;
     while (!finished && loop < cap) {
-        const float s[3] = {first[0] + t * dir[0], first[1] + t * dir[1], first[2] + t * dir[2]};
-        float vp[3];
+        // this lane's sample and the next pass's first
+        float tm = t, t_next = t;
 #pragma unroll
-        for (int i = 0; i < 3; ++i) vp[i] = tex_to_voxel(s[i], a.fdims[i], a.fdm1[i]);
-        const uint32_t brick = (((uint32_t)vp[2] >> bl) * nbxy) + (((uint32_t)vp[1] >> bl) * nbx) +
-                               ((uint32_t)vp[0] >> bl);
-        if (brick != cur_brick) {
-            cur_brick = brick;
-            // occupancy bits staged in LDS when they fit, else the byte table
-            cur_occ = s_occ ? ((s_occ[brick >> 5] >> (brick & 31)) & 1u) != 0 : a.brick_occ[brick] != 0;
-            if (!cur_occ) t_lim = empty_brick_limit_rcp(a, first, rdir, rfd, vp, bl);
+        for (int j = 1; j < P; ++j) {
+            t_next = t_next + a.step;
+            tm = sub == j ? t_next : tm;
         }
-        if (!cur_occ) {
-            // every sample at t' < t_lim lies in this empty brick: only
-            // the count and the float sequence t += step remain
-            ++n.samples;
-            if (COUNT) ++n.slots;
-            {
-                // most of the run in closed form; the last steps below take
-                // the reference's float sequence step by step
-                float d = 0.0f;
-                const int j = closed_form_steps(t, a.step, fminf(t_lim, tend), cap - loop, d);
-                if (j > 0) {
-                    t = t + (float)j * d;
-                    loop += j;
-                    n.samples += (unsigned long long)j;
-                    if (COUNT) n.slots += (unsigned long long)j;
-                }
-            }
-            float tn = t + a.step;
-            while (tn < t_lim && !(tn > tend) && loop + 1 < cap) {
-                t = tn;
-                ++loop;
-                ++n.samples;
-                if (COUNT) ++n.slots;
-                tn = t + a.step;
-            }
-            ++loop;
-            t = tn;
-            finished = t > tend;
-            continue;
-        }
-        // K samples t, t+step, ... (each within the ray and the cap);
-        // all loads issued before the first is composited
-        float tk[K], pk[K][3];
-        rec_t rk[K];
-        typename CellFetch<T, WIDE>::off_t ik[K];
-        bool valid[K];
-        {
-            float tt = t;
+        t_next = t_next + a.step;
+        float s[3], u[3], vp[3];
+        uint32_t lo[3];
 #pragma unroll
-            for (int k = 0; k < K; ++k) {
-                valid[k] = (k == 0) || (valid[k - 1] && !(tt > tend) && loop + k < cap);
-                tk[k] = tt;
-                if (valid[k]) {
-                    float sk[3];
-                    if (k == 0) {
-                        sk[0] = s[0];
-                        sk[1] = s[1];
-                        sk[2] = s[2];
-                    } else {
-                        sk[0] = first[0] + tt * dir[0];
-                        sk[1] = first[1] + tt * dir[1];
-                        sk[2] = first[2] + tt * dir[2];
+        for (int i = 0; i < 3; ++i) {
+            s[i] = first[i] + tm * dir[i];
+            u[i] = (a.fdims[i] * s[i]) + (-0.5f);
+            vp[i] = __builtin_amdgcn_fmed3f(u[i], 0.0f, a.fdm1[i]);   // tex_to_voxel of a number
+            lo[i] = (uint32_t)vp[i];                                  // <= dims - 1
+        }
+        if (probe) {
+            uint32_t b[3];
+#pragma unroll
+            for (int i = 0; i < 3; ++i) b[i] = sub_value<P>(lo[i], 0) >> bl;   // the pass's first sample
+            const uint32_t brick = cell_mul24(cell_mul24(b[2], a.nskip[1]) + b[1], a.nskip[0]) + b[0];
+            if (brick != cur_brick) {
+                cur_brick = brick;
+                empty = a.skip[brick];
+                if (empty) t_lim = empty_box_limit_rcp(a.nskip, first, rdir, rfd, b, bl, empty);
+            }
+            if (empty) {
+                // every sample at t' < t_lim lies in empty bricks: only the
+                // count and the float sequence t += step remain
+                const int loop0 = loop;
+                {
+                    // most of the run in closed form; the last steps below
+                    // take the reference's float sequence step by step
+                    float d = 0.0f;
+                    const int j = closed_form_steps(t, a.step, fminf(t_lim, tend), cap - loop, d);
+                    if (j > 0) {
+                        t = t + (float)j * d;
+                        loop += j;
                     }
-                    ik[k] = cell_of<T, WIDE>(f, a, sk, pk[k]);
-                    rk[k] = f.load(ik[k]);
                 }
-                tt = tt + a.step;
+                float tn = t + a.step;
+                while (tn < t_lim && !(tn > tend) && loop + 1 < cap) {
+                    t = tn;
+                    ++loop;
+                    tn = t + a.step;
+                }
+                ++loop;
+                t = tn;
+                finished = t > tend;
+                if (COUNT) n.skipped += (uint32_t)(loop - loop0);
+                continue;
             }
         }
+        // ca: the sample's corrected opacity; -1 past the ray's end or the cap
+        float ca = -1.0f, col[3] = {0.f, 0.f, 0.f};
+        if (sub == 0 || (!(tm > tend) && loop + sub < cap)) {
+            float p[3];
 #pragma unroll
-        for (int k = 0; k < K; ++k) {
-            if (!valid[k] || finished) break;
-            bool shade_now = false;
-            ++loop;
-            ++n.samples;
-            ++n.fetched;
+            for (int i = 0; i < 3; ++i) p[i] = vp[i] - floorf(vp[i]);
+            const typename CellFetch<T, WIDE>::off_t own = f.index(lo);
+            const rec_t rec = f.load(own);
             float v[8];
-            CellRecord<T>::unpack(rk[k], v);
-            const float inten = trilerp(v, pk[k]);
+            CellRecord<T>::unpack(rec, v);
+            const float inten = nan_ray ? NAN : trilerp(v, p);
             const uint32_t c8 = s_tf[tf_index(inten, a)];
-            const float ca = s_alpha[c8 >> 24];
+            ca = s_alpha[c8 >> 24];
             if (ca > 0.0f) {
-                float col[3] = {byte_norm(c8 & 0xffu), byte_norm((c8 >> 8) & 0xffu),
-                                byte_norm((c8 >> 16) & 0xffu)};
+                col[0] = byte_norm(c8 & 0xffu);
+                col[1] = byte_norm((c8 >> 8) & 0xffu);
+                col[2] = byte_norm((c8 >> 16) & 0xffu);
                 if (SHADE) {
-                    shade_now = true;
-                    const float tt = tk[k];
-                    const float ss[3] = {first[0] + tt * dir[0], first[1] + tt * dir[1],
-                                         first[2] + tt * dir[2]};
-                    float gr[3];
-                    if (tt == 0.0f) clip_border_gradient(a, px, py, ss, dir, gr);
-                    else if (SHADE == 2) cell_gradient<T, WIDE>(f, a, ss, gr);
-                    else if (!cell_gradient_interior<T, WIDE>(f, a, ss, rk[k], ik[k], pk[k], gr))
-                        cell_gradient<T, WIDE, true>(f, a, ss, gr);
-                    float pos[3];
+                    float gr[3], pos[3];
+                    if (tm == 0.0f) clip_border_gradient(a, px, py, s, dir, gr);
+                    else if (SHADE == 2 || nan_ray) cell_gradient<T, WIDE>(f, a, s, gr);
+                    else if (!cell_gradient_interior<T, WIDE>(f, a, u, rec, own, p, gr))
+                        cell_gradient<T, WIDE, true>(f, a, s, gr);
+                    if (SHADE == 2) {
 #pragma unroll
-                    for (int i = 0; i < 3; ++i)
-                        pos[i] = (((ss[i] * a.fdims[i]) - 0.5f) * a.spacing[i]) + a.offset[i];
-                    if (SHADE == 2) shade_model(a, gr, pos, col);
-                    else phong_fast(a, gr, pos, col);
-                    ++n.shaded;
+                        for (int i = 0; i < 3; ++i)
+                            pos[i] = (((s[i] * a.fdims[i]) - 0.5f) * a.spacing[i]) + a.offset[i];
+                        shade_model(a, gr, pos, col);
+                    } else {
+#pragma unroll
+                        for (int i = 0; i < 3; ++i) pos[i] = __builtin_fmaf(u[i], a.spacing[i], a.offset[i]);
+                        phong_fast(a, gr, pos, col);
+                    }
                 }
-                const float wgt = (1.0f - A) * ca;
-                r = r + wgt * col[0];
-                g = g + wgt * col[1];
-                bb = bb + wgt * col[2];
-                A = A + (1.0f - A) * ca;
             }
-            if (COUNT) {
-                ++n.slots;
-                n.shade_slots += (__ballot(shade_now) != 0ull) ? 1 : 0;
-            }
-            if (A >= kErtOpacity) {
-                A = 1.0f;
-                finished = true;
-            }
-            t = tk[k] + a.step;
-            finished = finished || (t > tend);
         }
+        if (COUNT) {
+            ++n.passes;
+            if (SHADE) n.shade_passes += (__ballot(ca > 0.0f) != 0ull) ? 1 : 0;
+        }
+        // the ray's lanes composite the pass's samples in order.  A terminated
+        // ray has A = 1, so later samples weigh zero and a sample of alpha 0
+        // changes nothing: no branches, unless a colour is not a finite
+        // number (degenerate lighting), which a zero weight would not keep out
+        const float A0 = A;
+        if (SHADE && __any(!(fabsf((col[0] + col[1]) + col[2]) < INFINITY))) {
+#pragma unroll
+            for (int j = 0; j < P; ++j) {
+                const float cj = sub_value<P>(ca, j);
+                const float c0 = sub_value<P>(col[0], j), c1 = sub_value<P>(col[1], j), c2 = sub_value<P>(col[2], j);
+                if (COUNT) count_sample<SHADE>(n, cj, A);
+                if (cj > 0.0f && A < kErtOpacity) {
+                    const float wgt = (1.0f - A) * cj;
+                    r = r + wgt * c0;
+                    g = g + wgt * c1;
+                    bb = bb + wgt * c2;
+                    A = A + wgt;
+                    A = A >= kErtOpacity ? 1.0f : A;
+                }
+            }
+        } else {
+            const float cz = fmaxf(ca, 0.0f);
+#pragma unroll
+            for (int j = 0; j < P; ++j) {
+                if (COUNT) count_sample<SHADE>(n, sub_value<P>(ca, j), A);
+                const float wgt = (1.0f - A) * sub_value<P>(cz, j);
+                r = r + wgt * sub_value<P>(col[0], j);
+                g = g + wgt * sub_value<P>(col[1], j);
+                bb = bb + wgt * sub_value<P>(col[2], j);
+                A = A + wgt;
+                A = A >= kErtOpacity ? 1.0f : A;
+            }
+        }
+        probe = A == A0;
+        loop += P;
+        t = t_next;
+        finished = A >= kErtOpacity || t > tend;
     }
-    return finished;
 }
 
-template <typename T, bool WIDE, int SHADE, bool COUNT, int K>
+// One ray of the cell march from entry point e to exit point l (neither the
+// background): returns the composited RGBA (in each of the ray's P lanes).
+template <typename T, bool WIDE, int SHADE, bool COUNT, int P>
 __device__ __forceinline__ float4 cell_ray(const MarchArgs& a, const CellFetch<T, WIDE>& f, const uint32_t* s_tf,
-                                           const float* s_alpha, const uint32_t* s_occ, int px, int py, float4 e,
-                                           float4 l, RayCounters& n) {
+                                           const float* s_alpha, int px, int py, int sub, float4 e, float4 l,
+                                           RayCounters& n) {
     ++n.rays;
     const float first[3] = {e.x, e.y, e.z};
     const float last[3] = {l.x, l.y, l.z};
@@ -420,8 +514,8 @@ __device__ __forceinline__ float4 cell_ray(const MarchArgs& a, const CellFetch<T
     const float tend = ray_setup(first, last, a.step, dir);
     float t = 0.0f, r = 0.f, g = 0.f, bb = 0.f, A = 0.f;
     int loop = 0;   // samples taken (the reference loop counter)
-    cell_march<T, WIDE, SHADE, COUNT, K>(a, f, s_tf, s_alpha, s_occ, px, py, first, dir, tend, a.loop_cap, t, loop, r,
-                                         g, bb, A, n);
+    cell_march<T, WIDE, SHADE, COUNT, P>(a, f, s_tf, s_alpha, px, py, sub, first, dir, tend, a.loop_cap, t, loop, r, g,
+                                         bb, A, n);
     return make_float4(r, g, bb, A);
 }
 

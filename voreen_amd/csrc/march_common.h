@@ -35,6 +35,11 @@ struct MarchArgs {
     const uint8_t* brick_occ;   // per-brick occupancy (1 = may hold alpha > 0) for this TF
     const uint32_t* occ_bits;   // the same occupancy, one bit per brick (bit b&31 of word b>>5)
     uint32_t occ_words;
+    // skip grid of the cell kernels (volume.h): per brick of 2^skip_log2
+    // voxels 0 (may hold alpha > 0) or the Chebyshev distance in bricks to
+    // the nearest such brick, at most kSkipReach
+    const uint8_t* skip;
+    uint32_t skip_log2, nskip[3];
     uint32_t dims[3];
     uint32_t nbricks[3];
     uint32_t brick_log2;
@@ -506,14 +511,37 @@ __device__ __forceinline__ float empty_brick_limit_rcp(const MarchArgs& a, const
     return tl;
 }
 
-// 64-lane maximum of a per-lane counter, times 64, added once per wavefront.
-__device__ __forceinline__ void wave_add_max64(unsigned long long* dst, unsigned long long v) {
+// empty_brick_limit_rcp for the box of bricks within d - 1 bricks (all empty)
+// of brick b, on a grid of nb bricks; selects instead of branches, since the
+// lanes of a wavefront face different ways.
+__device__ __forceinline__ float empty_box_limit_rcp(const uint32_t nb[3], const float first[3], const float rdir[3],
+                                                     const float rfd[3], const uint32_t b[3], uint32_t bl,
+                                                     uint32_t d) {
+    float tl = INFINITY;
+    const float B = (float)(1u << bl);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        const bool up = rdir[i] > 0.0f;
+        const int face = up ? (int)(b[i] + d) : (int)(b[i] + 1) - (int)d;
+        // inside the grid, and the axis moves (rdir 0: it bounds nothing)
+        const bool bounds = (up ? face < (int)nb[i] : face > 0) && rdir[i] != 0.0f;
+        const float vb = __builtin_fmaf((float)face, B, up ? 0.45f : 0.55f);   // face -+ 0.05 voxel, + 0.5
+        const float te = __builtin_fmaf(vb, rfd[i], -first[i]) * rdir[i];
+        tl = bounds ? fminf(tl, te) : tl;
+    }
+    return tl;
+}
+
+// 64-lane maximum of a per-lane counter, times `times` (the wavefront's rays),
+// added once per wavefront.
+__device__ __forceinline__ void wave_add_max64(unsigned long long* dst, unsigned long long v,
+                                               unsigned long long times = 64ull) {
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) {
         const unsigned long long o = __shfl_xor(v, off, 64);
         v = o > v ? o : v;
     }
-    if ((threadIdx.x & 63) == 0 && v) atomicAdd(dst, 64ull * v);
+    if ((threadIdx.x & 63) == 0 && v) atomicAdd(dst, times * v);
 }
 
 // 64-lane sum of a per-lane counter; lane 0 adds it to the global counter.
@@ -536,16 +564,22 @@ __host__ __device__ inline int judge_pixel(int g, int stride, int block, int off
 // regions, each XCD region kXcdRegionW x kXcdRegionH tiles; the i-th
 // workgroup of XCD x marches tile i of XCD region x of chip region
 // i / (W*H), chip regions from the middle of the image out (center_out).
-// So the rays one XCD has in flight lie in one compact region and share its
-// L2, and the 8 XCDs march neighbouring regions, so the rays in flight on
-// the chip cover one compact image area and share the Infinity Cache.  Measured on 512^3 / 1024^2 with
-// Phong: plain dispatch order 1.90 ms; each XCD on 2x2-tile blocks taken in
-// turn 1.79 ms; XCD regions of 4x4 tiles 1.74 ms, 8x4 1.73 ms, 8x8 1.79
-// ms, 16x8 (chip regions as wide as the image) 2.74 ms; one contiguous
-// image band per XCD 2.74 ms.  On 128^3 / 256^2 (16 x 16 tiles) the 2x2
-// blocks keep all XCDs busy (51,220 frames/s against 46,139 with regions).
+// So the rays one XCD has in flight lie in a few compact regions and share its
+// L2, and the 8 XCDs march neighbouring regions, so the rays in flight on the
+// chip cover one compact image area and share the Infinity Cache.  XCD regions
+// of 2x2 tiles, four lanes per ray, Phong: 512^3 / 1024^2 679 us, 256^3 / 512^2
+// 270 us, 1024^3 / 3840x2160 6.52 ms; 4x2 tiles 708, 281, 6.60; 2x1 675, 271,
+// 6.45; 8x4 tiles (five waves per SIMD) 823, 364, 7.02: the smaller region
+// spreads the long rays over the XCDs, which cannot take each other's tiles.
+// On 128^3 / 256^2 (16 x 16 tiles) the 2x2 blocks below keep all XCDs busy.
 constexpr uint32_t kXcds = 8;
-constexpr uint32_t kXcdRegionW = 8, kXcdRegionH = 4;
+constexpr uint32_t kXcdRegionW = 2, kXcdRegionH = 2;
+// XCD x takes region (x + kXcdTurnX * i + kXcdTurnY * j) % 8 of the chip region
+// in column i and row j of that order: along rows and along columns each XCD
+// meets every place of a chip region equally often.  With one fixed place per
+// XCD, the XCDs whose columns held the long rays had up to twice the others'
+// work and marched alone for the last 40% of a frame.
+constexpr uint32_t kXcdTurnX = 5, kXcdTurnY = 3;
 constexpr uint32_t kChipRegionW = 4 * kXcdRegionW, kChipRegionH = 2 * kXcdRegionH;
 // Images smaller than one chip region would leave XCDs without tiles; there
 // each XCD takes 2x2-tile blocks in turn instead (block b % 8 of every
@@ -572,14 +606,23 @@ __host__ __device__ inline uint32_t xcd_tile_grid(uint32_t tiles_x, uint32_t til
 // The k-th of n rows (or columns) of chip regions, from the middle out:
 // c, c + 1, c - 1, c + 2, ... (c = (n - 1) / 2), then the rest of the longer
 // side.  Long rays through the middle of the volume start first and the
-// cheap edges fill the end of the launch (1.74 -> 1.71 ms on 512^3 / 1024^2
-// with Phong), while the regions in flight stay next to each other.
+// cheap edges fill the end of the launch, while the regions in flight stay
+// next to each other.
 __device__ __forceinline__ uint32_t center_out(uint32_t k, uint32_t n) {
     const uint32_t c = (n - 1) / 2;   // c rows below the middle one, n - 1 - c >= c above
     if (k == 0) return c;
     if (k <= 2 * c) return (k & 1) ? c + (k + 1) / 2 : c - (k + 1) / 2;
     return c + (k - c);
 }
+
+// A launch of `blocks` workgroups as rows of at most 2^20 of them (one
+// dimension of a launch holds 2^32 work items), a whole number of rounds over
+// the XCDs, and a workgroup's number in it.
+inline dim3 linear_grid(uint64_t blocks) {
+    const uint64_t row = 1ull << 20;
+    return blocks <= row ? dim3((unsigned)blocks) : dim3((unsigned)row, (unsigned)((blocks + row - 1) / row));
+}
+__device__ __forceinline__ uint32_t linear_block() { return blockIdx.y * gridDim.x + blockIdx.x; }
 
 // Tile (tx, ty) of workgroup b; false for a workgroup with no tile.
 __device__ __forceinline__ bool xcd_tile(uint32_t b, uint32_t tiles_x, uint32_t tiles_y, uint32_t& tx,
@@ -591,8 +634,9 @@ __device__ __forceinline__ bool xcd_tile(uint32_t b, uint32_t tiles_x, uint32_t 
         const uint32_t cx_n = (tiles_x + kChipRegionW - 1) / kChipRegionW;
         const uint32_t cy_n = (tiles_y + kChipRegionH - 1) / kChipRegionH;
         const uint32_t cx = center_out(chip % cx_n, cx_n), cy = center_out(chip / cx_n, cy_n);
-        tx = cx * kChipRegionW + (xcd % 4) * kXcdRegionW + j % kXcdRegionW;
-        ty = cy * kChipRegionH + (xcd / 4) * kXcdRegionH + j / kXcdRegionW;
+        const uint32_t r = (xcd + kXcdTurnX * (chip % cx_n) + kXcdTurnY * (chip / cx_n)) % kXcds;
+        tx = cx * kChipRegionW + (r % 4) * kXcdRegionW + j % kXcdRegionW;
+        ty = cy * kChipRegionH + (r / 4) * kXcdRegionH + j / kXcdRegionW;
     } else {
         constexpr uint32_t S = kXcdBlock * kXcdBlock;
         const uint32_t block = (slot / S) * kXcds + xcd, j = slot % S;

@@ -41,6 +41,14 @@
 
 namespace hipdvr {
 
+// Occupancy bit words staged in LDS up to this count (4 KiB: 32768 bricks,
+// e.g. 512^3 at 16^3 bricks).
+constexpr uint32_t kMaxLdsOccWords = 1024;
+
+struct SlabCounters {
+    unsigned long long rays = 0, samples = 0, fetched = 0, shaded = 0, slots = 0, shade_slots = 0;
+};
+
 constexpr int kSlabLog2 = 3;                  // S = 8 planes per slab
 constexpr int kSlab = 1 << kSlabLog2;
 // LDS voxels of the staged box: 24 KiB for either voxel type (12288 uint16
@@ -273,7 +281,7 @@ struct SlabRay {
 template <typename T, int SHADE, bool COUNT>
 __device__ __forceinline__ int slab_march(const MarchArgs& a, const SlabReader<T>& rd, const uint32_t* s_tf,
                                           const float* s_alpha, const uint32_t* s_occ, int d, int slab,
-                                          SlabRay& ray, RayCounters& n) {
+                                          SlabRay& ray, SlabCounters& n) {
     const uint32_t bl = a.brick_log2;
     const uint32_t nbx = a.nbricks[0], nbxy = a.nbricks[0] * a.nbricks[1];
     const int cap = a.loop_cap;

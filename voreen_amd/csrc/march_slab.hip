@@ -107,7 +107,7 @@ __global__ __launch_bounds__(256) void march_slab_kernel(const MarchArgs a, cons
     const int gy = (int)tile_y * 16 + (wave >> 1) * 8 + (lane >> 3);
     const int px = gx * a.stride + a.pix_offset, py = gy * a.stride + a.pix_offset;
     const bool inside = (gx < a.grid_w) && (gy < a.grid_h) && (px < a.w) && (py < a.h);
-    RayCounters n;
+    SlabCounters n;
     SlabRay ray;
     ray.active = false;
     ray.r = ray.g = ray.b = ray.A = 0.f;

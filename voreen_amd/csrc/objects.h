@@ -38,7 +38,9 @@ void validate_params(const hipdvr_params* p, const hipdvr_tf* tf);
 void fill_march_args(MarchArgs& a, const hipdvr_volume* vol, const hipdvr_tf* tf, const hipdvr_params* p,
                      const float* d_entry, const float* d_exit, float* d_out, uint32_t w, uint32_t h,
                      unsigned long long* counters);
+OccArgs occupancy_args(const hipdvr_volume* vol, const hipdvr_tf* tf, const uint2* minmax, uint64_t count);
 void ensure_occupancy(hipdvr_ctx* ctx, hipdvr_volume* vol, const hipdvr_tf* tf);
+void ensure_skip(hipdvr_ctx* ctx, hipdvr_volume* vol, const hipdvr_tf* tf);
 // Opacity-corrected 2D table for this step on the device (host powf, as
 // cpuraycaster.cpp:289 evaluates it per sample).
 void ensure_tf2d(hipdvr_tf* tf, float step, hipStream_t st);

@@ -15,8 +15,9 @@ namespace hipdvr {
 // second increment to equal the first.  Returns a number of steps j >= 0 that
 // may be taken as t + j*d: every t_k, k <= j, stays below bound and within
 // cap_left - 1 steps, with margins of a few steps for the float estimates
-// (the two step counts are formed with one reciprocal of d: within 1 ulp of
-// the quotients, well inside the margins for counts up to 10^6).
+// (the two step counts are formed with one reciprocal of d, on the device the
+// hardware's: within 2 ulp of the quotients, well inside the margins for
+// counts up to 10^6).
 // The product and the sum are exact because t + j*d < 2^(e+1) lies on the
 // binade's ulp grid.
 __host__ __device__ inline int closed_form_steps(float t, float step, float bound, int cap_left, float& d) {
@@ -25,7 +26,11 @@ __host__ __device__ inline int closed_form_steps(float t, float step, float boun
     d = (t + step) - t;
     const float t1 = t + d;
     if (((t1 + step) - t1) != d) return 0;
+#ifdef __HIP_DEVICE_COMPILE__
+    const float rd = __builtin_amdgcn_rcpf(d);
+#else
     const float rd = 1.0f / d;
+#endif
     const float room = (B - step - t) * rd;     // steps k with t_k + step < B: k < room
     const float est = (bound - t) * rd;         // steps k with t_k < bound: k < est
     if (!(room > 6.0f) || !(est > 6.0f)) return 0;

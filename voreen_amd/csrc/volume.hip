@@ -91,6 +91,71 @@ __global__ __launch_bounds__(256) void minmax_kernel(const T* __restrict__ src, 
     }
 }
 
+// Ranges of 8^3 bricks (plus the upper one-voxel apron): a workgroup takes 32
+// bricks of a brick row, lane i the voxels of column 256*bx + i over the 9 x 9
+// rows (coalesced; the last column of the apron by one more load of lane 0's
+// wave), then one lane per brick folds its 9 columns from LDS.  Each voxel is
+// read 1.27 times.
+template <typename T>
+__global__ __launch_bounds__(256) void minmax8_kernel(const T* __restrict__ src, uint2* __restrict__ mm, uint32_t X,
+                                                      uint32_t Y, uint32_t Z, uint32_t nbx, uint32_t nby,
+                                                      uint32_t groups_x, uint64_t groups) {
+    __shared__ uint32_t s_lo[257], s_hi[257];
+    for (uint64_t gr = blockIdx.x; gr < groups; gr += gridDim.x) {
+        const uint32_t gx = (uint32_t)(gr % groups_x);
+        const uint64_t row = gr / groups_x;
+        const uint32_t by = (uint32_t)(row % nby), bz = (uint32_t)(row / nby);
+        for (uint32_t c = threadIdx.x; c < 257; c += 256) {
+            const uint32_t xc = gx * 256 + c, x = xc < X ? xc : X - 1;
+            uint32_t lo = 0xffffffffu, hi = 0;
+            for (uint32_t dz = 0; dz < 9; ++dz) {
+                const uint32_t zc = bz * 8 + dz, z = zc < Z ? zc : Z - 1;
+#pragma unroll
+                for (uint32_t dy = 0; dy < 9; ++dy) {
+                    const uint32_t yc = by * 8 + dy, y = yc < Y ? yc : Y - 1;
+                    const uint32_t v = src[((uint64_t)z * Y + y) * X + x];
+                    lo = v < lo ? v : lo;
+                    hi = v > hi ? v : hi;
+                }
+            }
+            s_lo[c] = lo;
+            s_hi[c] = hi;
+        }
+        __syncthreads();
+        const uint32_t bx = gx * 32 + threadIdx.x;
+        if (threadIdx.x < 32 && bx < nbx) {
+            uint32_t lo = 0xffffffffu, hi = 0;
+            for (uint32_t k = 0; k < 9; ++k) {
+                const uint32_t l2 = s_lo[threadIdx.x * 8 + k], h2 = s_hi[threadIdx.x * 8 + k];
+                lo = l2 < lo ? l2 : lo;
+                hi = h2 > hi ? h2 : hi;
+            }
+            mm[((uint64_t)bz * nby + by) * nbx + bx] = make_uint2(lo, hi);
+        }
+        __syncthreads();   // the columns are rewritten for the next group
+    }
+}
+
+// Ranges of bricks of 8 * 2^s voxels per edge from those of the 8^3 bricks
+// (the apron of the last child is the brick's).
+__global__ __launch_bounds__(256) void minmax_fold_kernel(const uint2* __restrict__ mm8, uint2* __restrict__ mm,
+                                                          uint32_t n8x, uint32_t n8y, uint32_t n8z, uint32_t s,
+                                                          uint32_t nbx, uint32_t nby, uint64_t count) {
+    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+    for (uint64_t b = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; b < count; b += stride) {
+        const uint32_t bx = (uint32_t)(b % nbx), by = (uint32_t)((b / nbx) % nby), bz = (uint32_t)(b / nbx / nby);
+        uint32_t lo = 0xffffffffu, hi = 0;
+        for (uint32_t z = bz << s; z < ((bz + 1) << s) && z < n8z; ++z)
+            for (uint32_t y = by << s; y < ((by + 1) << s) && y < n8y; ++y)
+                for (uint32_t x = bx << s; x < ((bx + 1) << s) && x < n8x; ++x) {
+                    const uint2 v = mm8[((uint64_t)z * n8y + y) * n8x + x];
+                    lo = v.x < lo ? v.x : lo;
+                    hi = v.y > hi ? v.y : hi;
+                }
+        mm[b] = make_uint2(lo, hi);
+    }
+}
+
 // One lane per record: the 8 footprint voxels of cell (x, y, z), clamped.
 // Records in the order of cell_layout.h; cells of the padding hold zeros.
 template <typename T>
@@ -137,9 +202,12 @@ void build_layouts(hipdvr_volume* v, hipStream_t st) {
                        (const T*)v->d_linear, (T*)v->d_tiled, X, Y, Z, v->nblocks[0], v->nblocks[1],
                        total);
     hip_check(hipGetLastError(), "tile kernel launch");
-    hipLaunchKernelGGL(minmax_kernel<T>, dim3(stride_grid(v->brick_count, 1)), dim3(256), 0, st,
-                       (const T*)v->d_linear, v->d_minmax, X, Y, Z, v->desc.brick_log2,
-                       v->nbricks[0], v->nbricks[1], v->brick_count);
+    const uint32_t gx = (v->nskip[0] + 31) / 32;
+    const uint64_t groups = (uint64_t)gx * v->nskip[1] * v->nskip[2];
+    hipLaunchKernelGGL(minmax8_kernel<T>, dim3(stride_grid(groups, 1)), dim3(256), 0, st, (const T*)v->d_linear,
+                       v->d_minmax8, X, Y, Z, v->nskip[0], v->nskip[1], gx, groups);
+    hip_check(hipGetLastError(), "min/max kernel launch");
+    launch_brick_minmax(v, v->desc.brick_log2, v->nbricks, v->d_minmax, st);
     hip_check(hipGetLastError(), "min/max kernel launch");
 }
 
@@ -155,10 +223,8 @@ __device__ __forceinline__ int map_index(float n, const OccArgs& a) {
     return idx < 0 ? 0 : (idx > w1 ? w1 : idx);
 }
 
-__global__ __launch_bounds__(256) void occupancy_kernel(const OccArgs a) {
-    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= a.count) return;
-    const uint2 mm = a.minmax[i];
+// Whether a brick of raw range mm may hold alpha > 0.
+__device__ __forceinline__ bool brick_occupied(const OccArgs& a, uint2 mm) {
     const float n0 = norm_raw(mm.x, a.dtype) - 1e-5f;
     const float n1 = norm_raw(mm.y, a.dtype) + 1e-5f;
     int i0 = map_index(n0, a), i1 = map_index(n1, a);
@@ -169,7 +235,55 @@ __global__ __launch_bounds__(256) void occupancy_kernel(const OccArgs a) {
     }
     i0 = i0 > 0 ? i0 - 1 : 0;
     i1 = i1 < a.tf_width - 1 ? i1 + 1 : a.tf_width - 1;
-    a.occ[i] = (a.alpha_prefix[i1 + 1] - a.alpha_prefix[i0]) != 0u ? 1 : 0;
+    return (a.alpha_prefix[i1 + 1] - a.alpha_prefix[i0]) != 0u;
+}
+
+__global__ __launch_bounds__(256) void occupancy_kernel(const OccArgs a) {
+    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < a.count) a.occ[i] = brick_occupied(a, a.minmax[i]) ? 1 : 0;
+}
+
+// The skip grid in three passes, one per axis: the Chebyshev distance to the
+// nearest occupied brick is the minimum over k of max(|k|, distance within
+// the row k bricks away), taken axis after axis.  Pass 1 classifies 256
+// bricks of an x row and their neighbours into LDS and writes the distance
+// within the row.
+__global__ __launch_bounds__(256) void skip_x_kernel(const OccArgs a, uint8_t* __restrict__ out, uint32_t nbx,
+                                                     uint32_t parts, uint64_t groups) {
+    constexpr int R = (int)kSkipReach;
+    __shared__ uint8_t s_occ[256 + 2 * R];
+    for (uint64_t gr = blockIdx.x; gr < groups; gr += gridDim.x) {
+        const uint64_t row = gr / parts;
+        const int x0 = (int)(gr % parts) * 256;
+        const uint2* mm = a.minmax + row * nbx;
+        for (int i = (int)threadIdx.x; i < 256 + 2 * R; i += 256) {
+            const int x = x0 + i - R;
+            s_occ[i] = x >= 0 && x < (int)nbx && brick_occupied(a, mm[x]) ? 1 : 0;
+        }
+        __syncthreads();
+        const int x = x0 + (int)threadIdx.x;
+        if (x < (int)nbx) {
+            int d = 0;
+            while (d < R && !s_occ[threadIdx.x + R - d] && !s_occ[threadIdx.x + R + d]) ++d;
+            out[row * nbx + x] = (uint8_t)d;
+        }
+        __syncthreads();   // the classes are rewritten for the next group
+    }
+}
+
+// Passes 2 and 3: n bricks along the axis, `stride` bytes apart.
+__global__ __launch_bounds__(256) void skip_axis_kernel(const uint8_t* __restrict__ in, uint8_t* __restrict__ out,
+                                                        uint64_t stride, uint32_t n, uint64_t count) {
+    const uint64_t step = (uint64_t)gridDim.x * blockDim.x;
+    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < count; i += step) {
+        const int c = (int)((i / stride) % n);
+        int d = in[i];
+        for (int k = 1; k < d; ++k) {
+            if (c - k >= 0) d = min(d, max(k, (int)in[i - (uint64_t)k * stride]));
+            if (c + k < (int)n) d = min(d, max(k, (int)in[i + (uint64_t)k * stride]));
+        }
+        out[i] = (uint8_t)d;
+    }
 }
 
 __global__ __launch_bounds__(256) void occupancy_bits_kernel(const uint8_t* __restrict__ occ,
@@ -188,6 +302,17 @@ void launch_occupancy(const OccArgs& a, hipStream_t st) {
     const uint64_t words = (a.count + 31) / 32;
     hipLaunchKernelGGL(occupancy_bits_kernel, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, st, a.occ, a.bits,
                        a.count);
+}
+
+void launch_skip_grid(const OccArgs& a, const uint32_t nb[3], uint8_t* skip, uint8_t* scratch, hipStream_t st) {
+    const uint64_t count = (uint64_t)nb[0] * nb[1] * nb[2];
+    const uint32_t parts = (nb[0] + 255) / 256;
+    const uint64_t groups = (uint64_t)parts * nb[1] * nb[2];
+    hipLaunchKernelGGL(skip_x_kernel, dim3(stride_grid(groups, 1)), dim3(256), 0, st, a, skip, nb[0], parts, groups);
+    hipLaunchKernelGGL(skip_axis_kernel, dim3(stride_grid(count)), dim3(256), 0, st, (const uint8_t*)skip, scratch,
+                       (uint64_t)nb[0], nb[1], count);
+    hipLaunchKernelGGL(skip_axis_kernel, dim3(stride_grid(count)), dim3(256), 0, st, (const uint8_t*)scratch, skip,
+                       (uint64_t)nb[0] * nb[1], nb[2], count);
 }
 
 hipdvr_volume* volume_create(hipdvr_ctx* ctx, hipStream_t st, const hipdvr_volume_desc* d,
@@ -211,7 +336,9 @@ hipdvr_volume* volume_create(hipdvr_ctx* ctx, hipStream_t st, const hipdvr_volum
         v->nbricks[i] = (d->dims[i] + (1u << bl) - 1) >> bl;
         v->tiled_elems *= v->nblocks[i];
         v->brick_count *= v->nbricks[i];
+        v->nskip[i] = (d->dims[i] + (1u << kSkipLog2) - 1) >> kSkipLog2;
     }
+    v->skip_count = (uint64_t)v->nskip[0] * v->nskip[1] * v->nskip[2];
     v->desc.dtype = d->dtype;
     v->desc.rwm_scale = d->rwm_scale;
     v->desc.rwm_offset = d->rwm_offset;
@@ -221,10 +348,18 @@ hipdvr_volume* volume_create(hipdvr_ctx* ctx, hipStream_t st, const hipdvr_volum
     try {
         hip_check(hipMalloc(&v->d_linear, bytes), "hipMalloc(volume)");
         hip_check(hipMalloc(&v->d_tiled, v->tiled_elems * vsz), "hipMalloc(tiled volume)");
-        hip_check(hipMalloc((void**)&v->d_minmax, v->brick_count * sizeof(uint2)), "hipMalloc(minmax)");
-        hip_check(hipMalloc((void**)&v->d_occ, v->brick_count), "hipMalloc(occupancy)");
+        // the brick tables in one allocation: ranges of the volume's bricks and
+        // of the 8^3 bricks, occupancy bits and bytes, skip grid and scratch
         v->occ_words = (uint32_t)((v->brick_count + 31) / 32);
-        hip_check(hipMalloc((void**)&v->d_occ_bits, (size_t)v->occ_words * 4), "hipMalloc(occupancy bits)");
+        const size_t mm = v->brick_count * sizeof(uint2), mm8 = v->skip_count * sizeof(uint2);
+        const size_t words = ((size_t)v->occ_words * 4 + 7) & ~(size_t)7;
+        char* p = nullptr;
+        hip_check(hipMalloc((void**)&p, mm + mm8 + words + v->brick_count + 2 * v->skip_count), "hipMalloc(bricks)");
+        v->d_minmax = (uint2*)p;
+        v->d_minmax8 = (uint2*)(p + mm);
+        v->d_occ_bits = (uint32_t*)(p + mm + mm8);
+        v->d_occ = (uint8_t*)(p + mm + mm8 + words);
+        v->d_skip = v->d_occ + v->brick_count;
         hip_check(hipMemcpyAsync(v->d_linear, voxels, bytes,
                                  on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, st),
                   "volume upload");
@@ -286,6 +421,11 @@ void volume_raw_minmax(const hipdvr_volume* v, hipStream_t st, uint32_t out[2]) 
 void launch_brick_minmax(const hipdvr_volume* v, uint32_t bl, const uint32_t nb[3], uint2* out, hipStream_t st) {
     const uint32_t X = v->desc.dims[0], Y = v->desc.dims[1], Z = v->desc.dims[2];
     const uint64_t count = (uint64_t)nb[0] * nb[1] * nb[2];
+    if (bl >= kSkipLog2) {
+        hipLaunchKernelGGL(minmax_fold_kernel, dim3(stride_grid(count)), dim3(256), 0, st, (const uint2*)v->d_minmax8,
+                           out, v->nskip[0], v->nskip[1], v->nskip[2], bl - kSkipLog2, nb[0], nb[1], count);
+        return;
+    }
     const dim3 grid(stride_grid(count, 1));
     if (v->desc.dtype == HIPDVR_U8)
         hipLaunchKernelGGL(minmax_kernel<uint8_t>, grid, dim3(256), 0, st, (const uint8_t*)v->d_linear, out, X, Y,
@@ -331,9 +471,7 @@ void volume_destroy(hipdvr_volume* v) {
     if (v->d_cells) (void)hipFree(v->d_cells);
     if (v->d_linear) (void)hipFree(v->d_linear);
     if (v->d_tiled) (void)hipFree(v->d_tiled);
-    if (v->d_minmax) (void)hipFree(v->d_minmax);
-    if (v->d_occ) (void)hipFree(v->d_occ);
-    if (v->d_occ_bits) (void)hipFree(v->d_occ_bits);
+    if (v->d_minmax) (void)hipFree(v->d_minmax);   // and the tables behind it
     if (v->d_grad) (void)hipFree(v->d_grad);
     delete v;
 }

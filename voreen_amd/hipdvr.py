@@ -746,7 +746,7 @@ def learned_sparse_dims(w, h, remarch_stride=0):
 
 
 class Batch:
-    """Many volumes in one persistent launch (include/hipdvr_batch.h).
+    """Many volumes in one launch (include/hipdvr_batch.h).
     jobs: sequence of (volume, tf, d_entry, d_exit, d_out, w, h, params)."""
 
     def __init__(self, ctx, jobs):
