@@ -7,6 +7,7 @@
 // message is kept per context.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 #include <utility>
 #include <cmath>
@@ -36,11 +37,6 @@ int guarded(hipdvr_ctx* ctx, F&& f) {
 }
 
 void set_device(hipdvr_ctx* ctx) { hip_check(hipSetDevice(ctx->device), "hipSetDevice"); }
-
-uint64_t next_serial() {
-    static std::atomic<uint64_t> s{1};
-    return s.fetch_add(1);
-}
 
 uint64_t fbits(float f) {
     uint32_t u;
@@ -101,6 +97,11 @@ struct MappingKey {
 
 }  // namespace
 
+uint64_t next_serial() {
+    static std::atomic<uint64_t> s{1};
+    return s.fetch_add(1);
+}
+
 OccArgs occupancy_args(const hipdvr_volume* vol, const hipdvr_tf* tf, const uint2* minmax, uint64_t count) {
     OccArgs o;
     o.minmax = minmax;
@@ -114,6 +115,7 @@ OccArgs occupancy_args(const hipdvr_volume* vol, const hipdvr_tf* tf, const uint
     o.dom_hi = tf->domain_hi;
     o.tf_width = (int32_t)tf->width;
     o.alpha_prefix = tf->d_alpha_prefix;
+    o.pair_reach = nullptr;
     return o;
 }
 
@@ -131,14 +133,26 @@ void ensure_occupancy(hipdvr_ctx* ctx, hipdvr_volume* vol, const hipdvr_tf* tf) 
     std::memcpy(vol->occ_key, key.k, sizeof key.k);
 }
 
-// The same for the skip grid of the cell kernels.
-void ensure_skip(hipdvr_ctx* ctx, hipdvr_volume* vol, const hipdvr_tf* tf) {
+// The same for the skip grid of the cell kernels; iso for kSkipIso.
+void ensure_skip(hipdvr_ctx* ctx, hipdvr_volume* vol, const hipdvr_tf* tf, SkipRule rule, float iso) {
     const MappingKey key(vol, tf);
-    if (std::memcmp(key.k, vol->skip_key, sizeof key.k) == 0) return;
-    launch_skip_grid(occupancy_args(vol, tf, vol->d_minmax8, vol->skip_count), vol->nskip, vol->d_skip,
-                     vol->d_skip + vol->skip_count, ctx->stream);
+    uint64_t k[5];
+    std::memcpy(k, key.k, sizeof key.k);
+    if (rule == kSkipPairs) k[0] = tf->preint_serial;
+    k[4] = ((uint64_t)rule << 32) | (rule == kSkipIso ? fbits(iso) : 0);
+    if (std::memcmp(k, vol->skip_key, sizeof k) == 0) return;
+    OccArgs o = occupancy_args(vol, tf, vol->d_minmax8, vol->skip_count);
+    if (rule == kSkipIso) {
+        launch_iso_prefix(tf->d_rgba, tf->width, iso, vol->d_band, ctx->stream);
+        o.alpha_prefix = vol->d_band;
+    } else if (rule == kSkipPairs) {
+        launch_pair_reach(tf->d_preint, tf->preint_n, vol->d_band, ctx->stream);
+        o.tf_width = (int32_t)tf->preint_n;
+        o.pair_reach = vol->d_band;
+    }
+    launch_skip_grid(o, vol->nskip, vol->d_skip, vol->d_skip + vol->skip_count, ctx->stream);
     hip_check(hipGetLastError(), "skip grid kernel launch");
-    std::memcpy(vol->skip_key, key.k, sizeof key.k);
+    std::memcpy(vol->skip_key, k, sizeof k);
 }
 
 // Opacity correction per alpha byte: cpuraycaster.cpp:291 with the TF colour
@@ -194,6 +208,7 @@ void fill_march_args(MarchArgs& a, const hipdvr_volume* vol, const hipdvr_tf* tf
     a.occ_words = vol->occ_words;
     a.brick_log2 = v.brick_log2;
     a.skip = vol->d_skip;
+    a.skip_minmax = vol->d_minmax8;
     a.skip_log2 = kSkipLog2;
     for (int i = 0; i < 3; ++i) {
         a.dims[i] = v.dims[i];
@@ -298,9 +313,7 @@ void render_device_impl(hipdvr_ctx* ctx, const hipdvr_volume* vol, const hipdvr_
     const bool other_gradient = p->gradient != HIPDVR_GRADIENT_CENTRAL &&
                                 (phong || p->compositing == HIPDVR_COMPOSITE_FHN);
     int kernel = p->kernel;
-    // the skipping kernels drop samples, which the pre-integrated mode cannot
-    // (its lookup pairs every sample with the previous one); the cell records
-    // serve the linear filter
+    // the cell records serve the linear filter and central differences
     const bool modes = p->compositing != HIPDVR_COMPOSITE_DVR;
     if (modes && kernel != HIPDVR_KERNEL_AUTO && kernel != HIPDVR_KERNEL_REFERENCE)
         fail(HIPDVR_ERR_UNSUPPORTED, "compositing modes other than DVR run on the reference kernel");
@@ -315,6 +328,21 @@ void render_device_impl(hipdvr_ctx* ctx, const hipdvr_volume* vol, const hipdvr_
         else if (p->shading == HIPDVR_SHADE_NONE || p->shading == HIPDVR_SHADE_PHONG) kernel = HIPDVR_KERNEL_BRICKED;
         else kernel = HIPDVR_KERNEL_REFERENCE;
     }
+    hipdvr_volume* mvol = const_cast<hipdvr_volume*>(vol);
+    // The other modes and the pre-integrated classification march the cell
+    // records as well (march_cell_modes.hip), with the same results in less
+    // time than the reference-layout kernels at every size measured (there).
+    // Those stay for the volumes whose records do not fit, and while the
+    // stream is captured: a graph would replay without the skip grid of its
+    // mapping.
+    bool cell_modes = p->kernel == HIPDVR_KERNEL_AUTO && kernel == HIPDVR_KERNEL_REFERENCE && !other_gradient &&
+                      p->filter == HIPDVR_FILTER_LINEAR && p->classification != HIPDVR_CLASS_TF2D &&
+                      (modes || p->classification == HIPDVR_CLASS_PREINT) && cells_allowed(vol);
+    if (cell_modes) {
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        cell_modes = hipStreamIsCapturing(ctx->stream, &cs) == hipSuccess && cs == hipStreamCaptureStatusNone &&
+                     try_cells(mvol, ctx->stream);
+    }
     const bool cell = kernel == HIPDVR_KERNEL_CELL;
     const bool slab = kernel == HIPDVR_KERNEL_SLAB;
     if ((kernel == HIPDVR_KERNEL_BRICKED || cell || slab) && p->classification != HIPDVR_CLASS_TF)
@@ -323,7 +351,6 @@ void render_device_impl(hipdvr_ctx* ctx, const hipdvr_volume* vol, const hipdvr_
         fail(HIPDVR_ERR_UNSUPPORTED, "the cell and slab kernels support the linear filter only");
     if (kernel == HIPDVR_KERNEL_BRICKED && p->shading != HIPDVR_SHADE_NONE && p->shading != HIPDVR_SHADE_PHONG)
         fail(HIPDVR_ERR_UNSUPPORTED, "the bricked kernel shades with Phong only");
-    hipdvr_volume* mvol = const_cast<hipdvr_volume*>(vol);
     if (p->classification == HIPDVR_CLASS_TF2D) {
         hipdvr_tf* mtf = const_cast<hipdvr_tf*>(tf);
         ensure_tf2d(mtf, p->step, ctx->stream);
@@ -335,9 +362,25 @@ void render_device_impl(hipdvr_ctx* ctx, const hipdvr_volume* vol, const hipdvr_
         ensure_cells(mvol, ctx->stream);
         a.cells = mvol->d_cells;
     }
+    if (cell_modes) {
+        a.cells = mvol->d_cells;
+        const VolumeDesc& v = vol->desc;
+        const float longest = (float)std::max(v.dims[0], std::max(v.dims[1], v.dims[2]));
+        if (modes) {
+            // the counters hold every sample that a light would have reached
+            const bool band = p->compositing == HIPDVR_COMPOSITE_ISO && !(count && phong);
+            ensure_skip(ctx, mvol, tf, band ? kSkipIso : kSkipAlpha, p->iso_value);
+        } else if (p->step * longest <= 7.5f) {
+            ensure_skip(ctx, mvol, tf, kSkipPairs);
+        } else {
+            a.skip = nullptr;   // a sample's predecessor may lie two bricks back
+        }
+    }
     if (count) hip_check(hipEventRecord(ctx->ev0, ctx->stream), "hipEventRecord");
     const bool timed = ctx_timing_start(ctx);
-    if (modes) {
+    if (cell_modes) {
+        launch_march_cell_modes(a, vol->desc.dtype, mvol->cells_wide, !modes, phong, count, p->batch, ctx->stream);
+    } else if (modes) {
         launch_march_modes(a, vol->desc.dtype, p->filter, phong, ctx->stream);
     } else if (kernel == HIPDVR_KERNEL_REFERENCE) {
         launch_march_ref(a, vol->desc.dtype, p->filter, p->classification, phong, count, ctx->stream);
@@ -617,6 +660,7 @@ int hipdvr_tf_set_preint(hipdvr_tf* tf, const float* table, uint32_t n) {
             tf->d_preint = nullptr;
             tf->preint_n = 0;
         }
+        tf->preint_serial = next_serial();
         const size_t bytes = (size_t)n * n * sizeof(float4);
         hip_check(hipMalloc((void**)&tf->d_preint, bytes), "hipMalloc(preint)");
         hip_check(hipMemcpy(tf->d_preint, table, bytes, hipMemcpyHostToDevice), "preint upload");

@@ -30,6 +30,12 @@ void launch_march_fast(const MarchArgs& a, int dtype, int filter, bool phong, bo
 // grid's pixels are placed by judge_pixel (a.pix_block; 1 for a whole frame).
 void launch_march_cell(const MarchArgs& a, int dtype, int shade, bool count, bool wide, int batch,
                        hipStream_t st);
+// The other compositing modes (preint false) or the pre-integrated
+// classification on the cell records, linear filter and central differences:
+// the reference-layout kernels' results bit for bit.  Without a.skip nothing
+// is skipped.
+void launch_march_cell_modes(const MarchArgs& a, int dtype, bool wide, bool preint, bool shaded, bool count, int batch,
+                             hipStream_t st);
 // Lanes per ray of a frame (march_cell.h) for hipdvr_params::batch: 1 and 2
 // two, 4 four, 8 sixteen; 0 by the grid's size.  A frame of few rays waits
 // for their chains, a frame of many for issue slots, of which more lanes per

@@ -330,6 +330,28 @@ __host__ __device__ constexpr int ray_w() { return P <= 2 ? 8 : (P <= 8 ? 4 : 2)
 template <int P>
 __host__ __device__ constexpr int ray_h() { return 64 / P / ray_w<P>(); }
 
+// Takes the run of samples that starts at (t, loop) and lies before t_lim, the
+// ray's end and the cap: (t, loop) becomes its last sample, the next sample's
+// t is returned.  bound = fminf(t_lim, tend).
+__device__ __forceinline__ float skip_run(float step, float bound, float t_lim, float tend, int cap, float& t,
+                                          int& loop) {
+    // most of the run in closed form; the last steps below take the
+    // reference's float sequence step by step
+    float d = 0.0f;
+    const int j = closed_form_steps(t, step, bound, cap - loop, d);
+    if (j > 0) {
+        t = t + (float)j * d;
+        loop += j;
+    }
+    float tn = t + step;
+    while (tn < t_lim && !(tn > tend) && loop + 1 < cap) {
+        t = tn;
+        ++loop;
+        tn = t + step;
+    }
+    return tn;
+}
+
 // The sample loop of one ray from state (t, loop, r, g, bb, A) up to sample
 // index cap (exclusive) or the ray's end.  SHADE: 0 none, 1 Phong with the
 // interior gradient and the hardware-approximate lighting terms (within the
@@ -398,22 +420,7 @@ __device__ __forceinline__ void cell_march(const MarchArgs& a, const CellFetch<T
                 // every sample at t' < t_lim lies in empty bricks: only the
                 // count and the float sequence t += step remain
                 const int loop0 = loop;
-                {
-                    // most of the run in closed form; the last steps below
-                    // take the reference's float sequence step by step
-                    float d = 0.0f;
-                    const int j = closed_form_steps(t, a.step, fminf(t_lim, tend), cap - loop, d);
-                    if (j > 0) {
-                        t = t + (float)j * d;
-                        loop += j;
-                    }
-                }
-                float tn = t + a.step;
-                while (tn < t_lim && !(tn > tend) && loop + 1 < cap) {
-                    t = tn;
-                    ++loop;
-                    tn = t + a.step;
-                }
+                const float tn = skip_run(a.step, fminf(t_lim, tend), t_lim, tend, cap, t, loop);
                 ++loop;
                 t = tn;
                 finished = t > tend;

@@ -39,6 +39,7 @@ struct MarchArgs {
     // voxels 0 (may hold alpha > 0) or the Chebyshev distance in bricks to
     // the nearest such brick, at most kSkipReach
     const uint8_t* skip;
+    const uint2* skip_minmax;   // raw value range of every brick of the skip grid
     uint32_t skip_log2, nskip[3];
     uint32_t dims[3];
     uint32_t nbricks[3];

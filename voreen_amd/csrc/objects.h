@@ -20,6 +20,7 @@ struct hipdvr_tf {
     std::vector<uint8_t> host_rgba;
     float4* d_preint = nullptr;
     uint32_t preint_n = 0;
+    uint64_t preint_serial = 0;      // of the table, as serial
     // 2D TF (hipdvr_tf2d_create): float RGBA table, its domains, and the
     // opacity-corrected copy on the device for the step it was made for
     bool is2d = false;
@@ -40,7 +41,9 @@ void fill_march_args(MarchArgs& a, const hipdvr_volume* vol, const hipdvr_tf* tf
                      unsigned long long* counters);
 OccArgs occupancy_args(const hipdvr_volume* vol, const hipdvr_tf* tf, const uint2* minmax, uint64_t count);
 void ensure_occupancy(hipdvr_ctx* ctx, hipdvr_volume* vol, const hipdvr_tf* tf);
-void ensure_skip(hipdvr_ctx* ctx, hipdvr_volume* vol, const hipdvr_tf* tf);
+void ensure_skip(hipdvr_ctx* ctx, hipdvr_volume* vol, const hipdvr_tf* tf, SkipRule rule = kSkipAlpha,
+                 float iso = 0.0f);
+uint64_t next_serial();   // of objects and tables, never the same twice
 // Opacity-corrected 2D table for this step on the device (host powf, as
 // cpuraycaster.cpp:289 evaluates it per sample).
 void ensure_tf2d(hipdvr_tf* tf, float step, hipStream_t st);

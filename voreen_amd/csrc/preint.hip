@@ -159,5 +159,6 @@ extern "C" int hipdvr_tf_preint_device(hipdvr_tf* tf, const hipdvr_tf_key* keys,
         if (tf->d_preint) (void)hipFree(tf->d_preint);
         tf->d_preint = d_tab;
         tf->preint_n = n;
+        tf->preint_serial = next_serial();
     });
 }

@@ -47,6 +47,11 @@ namespace hipdvr {
 
 constexpr uint32_t kSkipLog2 = 3;    // 8^3 voxels
 constexpr uint32_t kSkipReach = 15;
+constexpr uint32_t kBandWords = 4100;
+// Which samples a skip grid may leave out: those of TF alpha 0; those whose
+// alpha lies outside the isosurface band; those whose pre-integrated entry
+// (with any predecessor from a neighbouring brick) has alpha 0.
+enum SkipRule { kSkipAlpha = 0, kSkipIso = 1, kSkipPairs = 2 };
 
 struct VolumeDesc {
     uint32_t dims[3];
@@ -76,7 +81,8 @@ struct hipdvr_volume {
     uint8_t* d_skip = nullptr;       // skip grid for the last TF mapping, and as many bytes of scratch
     uint32_t nskip[3] = {0, 0, 0};   // 8^3 bricks per axis
     uint64_t skip_count = 0;
-    uint64_t skip_key[4] = {0, 0, 0, 0};
+    uint64_t skip_key[5] = {0, 0, 0, 0, 0};
+    uint32_t* d_band = nullptr;      // [kBandWords] table of the skip grid's rule (SkipRule)
     void* d_cells = nullptr;         // cell records (null until first use)
     uint64_t cell_bytes = 0;
     bool cells_wide = false;         // more than 2^32 - 256 bytes: 64-bit addressing
@@ -101,6 +107,8 @@ void launch_brick_minmax(const hipdvr_volume* vol, uint32_t bl, const uint32_t n
 // Raw minimum and maximum voxel of the whole volume (synchronous).
 void volume_raw_minmax(const hipdvr_volume* vol, hipStream_t st, uint32_t out[2]);
 // Build the cell records if they are not there yet (synchronous).
+// try_cells: false, and no error, where there is no memory for them.
+bool try_cells(hipdvr_volume* vol, hipStream_t st);
 void ensure_cells(hipdvr_volume* vol, hipStream_t st);
 
 // Per-brick occupancy for a TF mapping: a brick is empty when no TF entry
@@ -115,10 +123,20 @@ struct OccArgs {
     int32_t tf_width;
     const uint32_t* alpha_prefix;   // [w+1]: number of non-zero alpha bytes in [0, i)
     uint32_t* bits;                 // [ceil(count/32)] occupancy bits (written after occ)
+    // kSkipPairs: indices are those of a table of tf_width entries a side;
+    // the square of indices [i, pair_reach[i] - 1] holds no entry of alpha > 0,
+    // and a brick is judged by the range over its 3^3 neighbourhood, which
+    // holds a sample's predecessor as well
+    const uint32_t* pair_reach;
 };
 void launch_occupancy(const OccArgs& a, hipStream_t st);
 // Skip grid (see above) of nb bricks from the ranges in a (a.occ and a.bits
 // unused); scratch holds as many bytes as the grid.
 void launch_skip_grid(const OccArgs& a, const uint32_t nb[3], uint8_t* skip, uint8_t* scratch, hipStream_t st);
+// prefix[i]: number of entries in [0, i) of the width entries of rgba whose
+// alpha is not 0 and within 0.02 of iso (the ISO compositing's test).
+void launch_iso_prefix(const uint32_t* rgba, uint32_t width, float iso, uint32_t* prefix, hipStream_t st);
+// reach of an n x n pre-integration table (OccArgs::pair_reach).
+void launch_pair_reach(const float4* table, uint32_t n, uint32_t* reach, hipStream_t st);
 
 }  // namespace hipdvr

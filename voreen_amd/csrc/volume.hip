@@ -223,11 +223,12 @@ __device__ __forceinline__ int map_index(float n, const OccArgs& a) {
     return idx < 0 ? 0 : (idx > w1 ? w1 : idx);
 }
 
-// Whether a brick of raw range mm may hold alpha > 0.
-__device__ __forceinline__ bool brick_occupied(const OccArgs& a, uint2 mm) {
+// Table indices that samples of raw range mm may take, one more to each side.
+__device__ __forceinline__ void index_range(const OccArgs& a, uint2 mm, int& i0, int& i1) {
     const float n0 = norm_raw(mm.x, a.dtype) - 1e-5f;
     const float n1 = norm_raw(mm.y, a.dtype) + 1e-5f;
-    int i0 = map_index(n0, a), i1 = map_index(n1, a);
+    i0 = map_index(n0, a);
+    i1 = map_index(n1, a);
     if (i0 > i1) {
         const int t = i0;
         i0 = i1;
@@ -235,6 +236,12 @@ __device__ __forceinline__ bool brick_occupied(const OccArgs& a, uint2 mm) {
     }
     i0 = i0 > 0 ? i0 - 1 : 0;
     i1 = i1 < a.tf_width - 1 ? i1 + 1 : a.tf_width - 1;
+}
+
+// Whether a brick of raw range mm may hold alpha > 0.
+__device__ __forceinline__ bool brick_occupied(const OccArgs& a, uint2 mm) {
+    int i0, i1;
+    index_range(a, mm, i0, i1);
     return (a.alpha_prefix[i1 + 1] - a.alpha_prefix[i0]) != 0u;
 }
 
@@ -243,14 +250,33 @@ __global__ __launch_bounds__(256) void occupancy_kernel(const OccArgs a) {
     if (i < a.count) a.occ[i] = brick_occupied(a, a.minmax[i]) ? 1 : 0;
 }
 
+// The same for the pairs of a pre-integration table: brick (x, y, z) of the
+// grid nb.
+__device__ __forceinline__ bool brick_pairs_occupied(const OccArgs& a, const uint32_t nb[3], uint32_t x, uint32_t y,
+                                                     uint32_t z) {
+    uint32_t lo = 0xffffffffu, hi = 0;
+    for (uint32_t k = z > 0 ? z - 1 : 0; k <= z + 1 && k < nb[2]; ++k)
+        for (uint32_t j = y > 0 ? y - 1 : 0; j <= y + 1 && j < nb[1]; ++j)
+            for (uint32_t i = x > 0 ? x - 1 : 0; i <= x + 1 && i < nb[0]; ++i) {
+                const uint2 v = a.minmax[((uint64_t)k * nb[1] + j) * nb[0] + i];
+                lo = v.x < lo ? v.x : lo;
+                hi = v.y > hi ? v.y : hi;
+            }
+    int i0, i1;
+    index_range(a, make_uint2(lo, hi), i0, i1);
+    return a.pair_reach[i0] <= (uint32_t)i1;
+}
+
 // The skip grid in three passes, one per axis: the Chebyshev distance to the
 // nearest occupied brick is the minimum over k of max(|k|, distance within
 // the row k bricks away), taken axis after axis.  Pass 1 classifies 256
 // bricks of an x row and their neighbours into LDS and writes the distance
 // within the row.
+template <bool PAIRS>
 __global__ __launch_bounds__(256) void skip_x_kernel(const OccArgs a, uint8_t* __restrict__ out, uint32_t nbx,
-                                                     uint32_t parts, uint64_t groups) {
+                                                     uint32_t nby, uint32_t nbz, uint32_t parts, uint64_t groups) {
     constexpr int R = (int)kSkipReach;
+    const uint32_t nb[3] = {nbx, nby, nbz};
     __shared__ uint8_t s_occ[256 + 2 * R];
     for (uint64_t gr = blockIdx.x; gr < groups; gr += gridDim.x) {
         const uint64_t row = gr / parts;
@@ -258,7 +284,12 @@ __global__ __launch_bounds__(256) void skip_x_kernel(const OccArgs a, uint8_t* _
         const uint2* mm = a.minmax + row * nbx;
         for (int i = (int)threadIdx.x; i < 256 + 2 * R; i += 256) {
             const int x = x0 + i - R;
-            s_occ[i] = x >= 0 && x < (int)nbx && brick_occupied(a, mm[x]) ? 1 : 0;
+            bool occ = x >= 0 && x < (int)nbx;
+            if (occ) {
+                if constexpr (PAIRS) occ = brick_pairs_occupied(a, nb, x, (uint32_t)(row % nby), (uint32_t)(row / nby));
+                else occ = brick_occupied(a, mm[x]);
+            }
+            s_occ[i] = occ ? 1 : 0;
         }
         __syncthreads();
         const int x = x0 + (int)threadIdx.x;
@@ -286,6 +317,83 @@ __global__ __launch_bounds__(256) void skip_axis_kernel(const uint8_t* __restric
     }
 }
 
+// One workgroup: inclusive scan of v over its 1024 lanes (s: 1024 words).
+template <bool MIN>
+__device__ __forceinline__ uint32_t block_scan(uint32_t v, uint32_t* s) {
+    const int tid = threadIdx.x;
+    s[tid] = v;
+    __syncthreads();
+    for (int off = 1; off < 1024; off <<= 1) {
+        const uint32_t o = tid >= off ? s[tid - off] : (MIN ? 0xffffffffu : 0u);
+        __syncthreads();
+        v = MIN ? (o < v ? o : v) : v + o;
+        s[tid] = v;
+        __syncthreads();
+    }
+    return v;
+}
+
+// One workgroup, four entries per lane: width <= 4096.
+__global__ __launch_bounds__(1024) void iso_prefix_kernel(const uint32_t* __restrict__ rgba, uint32_t width, float iso,
+                                                          uint32_t* __restrict__ prefix) {
+    __shared__ uint32_t s[1024];
+    uint32_t c[4], sum = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) {
+        const uint32_t i = threadIdx.x * 4 + k;
+        const float al = i < width ? VoxNorm<uint8_t>::apply(rgba[i] >> 24) : 0.0f;
+        sum += al > 0.0f && al >= iso - 0.02f && al <= iso + 0.02f ? 1 : 0;
+        c[k] = sum;
+    }
+    const uint32_t before = block_scan<false>(sum, s) - sum;
+    if (threadIdx.x == 0) prefix[0] = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k)
+        if (threadIdx.x * 4 + k < width) prefix[threadIdx.x * 4 + k + 1] = before + c[k];
+}
+
+// Block i: the smallest j >= i whose entry (i, j) or (j, i) has alpha > 0 (n:
+// none), from i upward, so a table that is mostly visible is hardly read.
+__global__ __launch_bounds__(256) void pair_first_kernel(const float4* __restrict__ table, uint32_t n,
+                                                         uint32_t* __restrict__ first) {
+    __shared__ uint32_t s_min[4];
+    const uint32_t i = blockIdx.x;
+    uint32_t found = n;
+    for (uint32_t j0 = i; j0 < n; j0 += 256) {
+        const uint32_t j = j0 + threadIdx.x;
+        bool hit = false;
+        if (j < n) hit = !(table[(size_t)i * n + j].w <= 0.0f) || !(table[(size_t)j * n + i].w <= 0.0f);
+        const unsigned long long b = __ballot(hit);
+        if ((threadIdx.x & 63) == 0) s_min[threadIdx.x >> 6] = b ? j + (uint32_t)__builtin_ctzll(b) : n;
+        __syncthreads();
+        for (int w = 3; w >= 0; --w) found = s_min[w] < found ? s_min[w] : found;
+        __syncthreads();
+        if (found < n) break;
+    }
+    if (threadIdx.x == 0) first[i] = found;
+}
+
+// One workgroup: reach[i] = minimum of first over [i, n), in place, n <= 4096
+// (entries beyond i's square have a first beyond it as well).
+__global__ __launch_bounds__(1024) void pair_reach_kernel(uint32_t* __restrict__ first, uint32_t n) {
+    __shared__ uint32_t s[1024];
+    uint32_t c[4], m = 0xffffffffu;
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) {   // from the table's end
+        const uint32_t r = threadIdx.x * 4 + k;
+        const uint32_t v = r < n ? first[n - 1 - r] : 0xffffffffu;
+        m = v < m ? v : m;
+        c[k] = m;
+    }
+    block_scan<true>(m, s);
+    const uint32_t before = threadIdx.x > 0 ? s[threadIdx.x - 1] : 0xffffffffu;
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) {
+        const uint32_t r = threadIdx.x * 4 + k;
+        if (r < n) first[n - 1 - r] = before < c[k] ? before : c[k];
+    }
+}
+
 __global__ __launch_bounds__(256) void occupancy_bits_kernel(const uint8_t* __restrict__ occ,
                                                              uint32_t* __restrict__ bits, uint64_t count) {
     const uint64_t w = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -308,11 +416,25 @@ void launch_skip_grid(const OccArgs& a, const uint32_t nb[3], uint8_t* skip, uin
     const uint64_t count = (uint64_t)nb[0] * nb[1] * nb[2];
     const uint32_t parts = (nb[0] + 255) / 256;
     const uint64_t groups = (uint64_t)parts * nb[1] * nb[2];
-    hipLaunchKernelGGL(skip_x_kernel, dim3(stride_grid(groups, 1)), dim3(256), 0, st, a, skip, nb[0], parts, groups);
+    if (a.pair_reach)
+        hipLaunchKernelGGL(skip_x_kernel<true>, dim3(stride_grid(groups, 1)), dim3(256), 0, st, a, skip, nb[0], nb[1],
+                           nb[2], parts, groups);
+    else
+        hipLaunchKernelGGL(skip_x_kernel<false>, dim3(stride_grid(groups, 1)), dim3(256), 0, st, a, skip, nb[0], nb[1],
+                           nb[2], parts, groups);
     hipLaunchKernelGGL(skip_axis_kernel, dim3(stride_grid(count)), dim3(256), 0, st, (const uint8_t*)skip, scratch,
                        (uint64_t)nb[0], nb[1], count);
     hipLaunchKernelGGL(skip_axis_kernel, dim3(stride_grid(count)), dim3(256), 0, st, (const uint8_t*)scratch, skip,
                        (uint64_t)nb[0] * nb[1], nb[2], count);
+}
+
+void launch_iso_prefix(const uint32_t* rgba, uint32_t width, float iso, uint32_t* prefix, hipStream_t st) {
+    hipLaunchKernelGGL(iso_prefix_kernel, dim3(1), dim3(1024), 0, st, rgba, width, iso, prefix);
+}
+
+void launch_pair_reach(const float4* table, uint32_t n, uint32_t* reach, hipStream_t st) {
+    hipLaunchKernelGGL(pair_first_kernel, dim3(n), dim3(256), 0, st, table, n, reach);
+    hipLaunchKernelGGL(pair_reach_kernel, dim3(1), dim3(1024), 0, st, reach, n);
 }
 
 hipdvr_volume* volume_create(hipdvr_ctx* ctx, hipStream_t st, const hipdvr_volume_desc* d,
@@ -354,12 +476,16 @@ hipdvr_volume* volume_create(hipdvr_ctx* ctx, hipStream_t st, const hipdvr_volum
         const size_t mm = v->brick_count * sizeof(uint2), mm8 = v->skip_count * sizeof(uint2);
         const size_t words = ((size_t)v->occ_words * 4 + 7) & ~(size_t)7;
         char* p = nullptr;
-        hip_check(hipMalloc((void**)&p, mm + mm8 + words + v->brick_count + 2 * v->skip_count), "hipMalloc(bricks)");
+        hip_check(hipMalloc((void**)&p, mm + mm8 + words + v->brick_count + 2 * v->skip_count +
+                                              kBandWords * 4 + 4),
+                  "hipMalloc(bricks)");
         v->d_minmax = (uint2*)p;
         v->d_minmax8 = (uint2*)(p + mm);
         v->d_occ_bits = (uint32_t*)(p + mm + mm8);
         v->d_occ = (uint8_t*)(p + mm + mm8 + words);
         v->d_skip = v->d_occ + v->brick_count;
+        const size_t band = mm + mm8 + words + v->brick_count + 2 * v->skip_count;
+        v->d_band = (uint32_t*)(p + ((band + 3) & ~(size_t)3));
         hip_check(hipMemcpyAsync(v->d_linear, voxels, bytes,
                                  on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, st),
                   "volume upload");
@@ -441,13 +567,18 @@ uint64_t cell_record_bytes(const hipdvr_volume* v) {
 
 bool cells_allowed(const hipdvr_volume* v) { return cell_record_bytes(v) <= kMaxCellBytes; }
 
-void ensure_cells(hipdvr_volume* v, hipStream_t st) {
-    if (v->d_cells) return;
+bool try_cells(hipdvr_volume* v, hipStream_t st) {
+    if (v->d_cells) return true;
     const uint64_t bytes = cell_record_bytes(v);
-    if (bytes > kMaxCellBytes) fail(HIPDVR_ERR_UNSUPPORTED, "cell records of this volume exceed the size limit");
+    if (bytes > kMaxCellBytes) return false;
     const uint64_t total = bytes / (v->desc.dtype == HIPDVR_U8 ? 8 : 16);
     void* p = nullptr;
-    hip_check(hipMalloc(&p, bytes), "hipMalloc(cell records)");
+    const hipError_t e0 = hipMalloc(&p, bytes);
+    if (e0 == hipErrorOutOfMemory) {
+        (void)hipGetLastError();   // not left for the next call
+        return false;
+    }
+    hip_check(e0, "hipMalloc(cell records)");
     const dim3 grid(stride_grid(total));
     if (v->desc.dtype == HIPDVR_U8)
         hipLaunchKernelGGL(cells_kernel<uint8_t>, grid, dim3(256), 0, st, (const uint8_t*)v->d_linear, p,
@@ -464,6 +595,13 @@ void ensure_cells(hipdvr_volume* v, hipStream_t st) {
     v->d_cells = p;
     v->cell_bytes = bytes;
     v->cells_wide = bytes > 0xffffff00ull;
+    return true;
+}
+
+void ensure_cells(hipdvr_volume* v, hipStream_t st) {
+    if (v->d_cells) return;
+    if (!cells_allowed(v)) fail(HIPDVR_ERR_UNSUPPORTED, "cell records of this volume exceed the size limit");
+    if (!try_cells(v, st)) hip_check(hipErrorOutOfMemory, "hipMalloc(cell records)");
 }
 
 void volume_destroy(hipdvr_volume* v) {
