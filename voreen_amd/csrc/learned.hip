@@ -23,6 +23,7 @@ struct hipdvr_mlp {
     float* d_m = nullptr;        // Adam moments
     float* d_v = nullptr;
     float* d_grad = nullptr;
+    float* d_partial = nullptr;  // gradient sums per workgroup; d_loss and dev.frag lie behind
     float* d_loss = nullptr;
     MlpDevParams dev{};
     int step = 0;
@@ -38,11 +39,11 @@ void free_mlp(hipdvr_mlp* m) {
     (void)hipFree(m->d_m);
     (void)hipFree(m->d_v);
     (void)hipFree(m->d_grad);
-    (void)hipFree(m->d_loss);
     (void)hipFree(m->dev.w1);
     (void)hipFree(m->dev.w2);
     (void)hipFree(m->dev.w3);
     (void)hipFree(m->dev.b);
+    (void)hipFree(m->d_partial);
     delete m;
 }
 
@@ -70,7 +71,11 @@ int hipdvr_mlp_create(hipdvr_ctx* ctx, uint64_t seed, hipdvr_mlp** out) {
             hip_check(hipMalloc((void**)&m->d_m, pb), "hipMalloc(mlp)");
             hip_check(hipMalloc((void**)&m->d_v, pb), "hipMalloc(mlp)");
             hip_check(hipMalloc((void**)&m->d_grad, pb + 64), "hipMalloc(mlp)");
-            hip_check(hipMalloc((void**)&m->d_loss, 64), "hipMalloc(mlp)");
+            const size_t sums = (size_t)kMlpGradBlocks * kMlpPartial;
+            hip_check(hipMalloc((void**)&m->d_partial, (sums + 16) * sizeof(float) + kMlpFrag * sizeof(short)),
+                      "hipMalloc(mlp)");
+            m->d_loss = m->d_partial + sums;
+            m->dev.frag = (short*)(m->d_loss + 16);
             hip_check(hipMalloc((void**)&m->dev.w1, kMlpIn * kMlpHidden * 2), "hipMalloc(mlp)");
             hip_check(hipMalloc((void**)&m->dev.w2, kMlpHidden * kMlpHidden * 2), "hipMalloc(mlp)");
             hip_check(hipMalloc((void**)&m->dev.w3, kMlpHidden * 16 * 2), "hipMalloc(mlp)");
@@ -151,7 +156,8 @@ int hipdvr_mlp_gradient(hipdvr_mlp* m, const float* d_x, const float* d_t, uint3
     return ctx_guarded(m->ctx, [&] {
         if (!d_x || !d_t || !grad_out || rows == 0) fail(HIPDVR_ERR_INVALID, "bad arguments");
         ctx_set_device(m->ctx);
-        launch_mlp_grad(m->dev, d_x, d_t, rows, m->d_grad, m->d_loss, ctx_stream(m->ctx));
+        const uint32_t blocks = launch_mlp_grad(m->dev, d_x, d_t, rows, m->d_partial, ctx_stream(m->ctx));
+        launch_mlp_sum(m->d_partial, blocks, m->d_grad, m->d_loss, ctx_stream(m->ctx));
         hip_check(hipGetLastError(), "mlp grad launch");
         hip_check(hipMemcpyAsync(grad_out, m->d_grad, kMlpParams * sizeof(float), hipMemcpyDeviceToHost,
                                  ctx_stream(m->ctx)), "grad download");
@@ -170,10 +176,10 @@ int hipdvr_mlp_train_step(hipdvr_mlp* m, const float* d_x, const float* d_t, uin
         if (!d_x || !d_t || rows == 0 || !(lr > 0.f)) fail(HIPDVR_ERR_INVALID, "bad arguments");
         ctx_set_device(m->ctx);
         hipStream_t st = ctx_stream(m->ctx);
-        launch_mlp_grad(m->dev, d_x, d_t, rows, m->d_grad, m->d_loss, st);
+        const uint32_t blocks = launch_mlp_grad(m->dev, d_x, d_t, rows, m->d_partial, st);
         m->step += 1;
-        launch_mlp_adam(m->d_master, m->d_m, m->d_v, m->d_grad, lr, m->step, st);
-        launch_mlp_pack(m->d_master, m->dev, st);
+        launch_mlp_update(m->d_partial, blocks, m->d_grad, m->d_loss, m->d_master, m->d_m, m->d_v, m->dev, lr, m->step,
+                          st);
         hip_check(hipGetLastError(), "mlp train launch");
         if (loss_out) {
             hip_check(hipMemcpyAsync(loss_out, m->d_loss, sizeof(float), hipMemcpyDeviceToHost, st),

@@ -9,7 +9,7 @@
 //
 // Parameters (FP32 master copy, flat): W1[16][64] b1[64] W2[64][64] b2[64]
 // W3[64][2] b3[2]; the kernels read BF16 copies of W1, W2, W3 (W3 padded to
-// 64x16 with zero columns) made by mlp_pack after every update.
+// 64x16 with zero columns) that every update writes with the master (pack_param).
 //
 // Loss per row (targets t0 in {0,1}, t1 in [0,3], weight t2):
 //   BCE-with-logits(y0, t0) + t2 * (y1 - t1)^2, averaged over the batch.
@@ -29,14 +29,8 @@ __device__ __forceinline__ short f2bf(float x) {
 }
 __device__ __forceinline__ float bf2f(short b) { return __uint_as_float(((uint32_t)(uint16_t)b) << 16); }
 
-// GELU (erf form) and its derivative.
+// GELU (erf form).
 __device__ __forceinline__ float gelu(float x) { return 0.5f * x * (1.0f + erff(x * 0.70710678118654752f)); }
-__device__ __forceinline__ float gelu_grad(float x) {
-    const float cdf = 0.5f * (1.0f + erff(x * 0.70710678118654752f));
-    const float pdf = 0.39894228040143268f * expf(-0.5f * x * x);
-    return cdf + x * pdf;
-}
-
 __device__ __forceinline__ f4 mfma(s4 a, s4 b, f4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
 }
@@ -54,10 +48,6 @@ struct WaveTile {
     short x[16 * kMlpIn];       // input rows (bf16)
     short h1[16 * kMlpHidden];  // GELU(z1) (bf16)
     short h2[16 * kMlpHidden];  // GELU(z2) (bf16)
-    float z1[16 * kMlpHidden];
-    float z2[16 * kMlpHidden];
-    float dz[16 * kMlpHidden];  // dZ2, then dZ1
-    float dy[16 * 2];
 };
 
 __device__ void load_shared(MlpShared& sh, const MlpDevParams& p) {
@@ -88,7 +78,6 @@ __device__ void tile_forward(const MlpShared& sh, WaveTile& t, f4& y) {
         for (int i = 0; i < 4; ++i) {
             const int row = kq + i, col = nt * 16 + n0;
             const float z = acc[i] + sh.b1[col];
-            t.z1[row * kMlpHidden + col] = z;
             t.h1[row * kMlpHidden + col] = f2bf(gelu(z));
         }
     }
@@ -108,7 +97,6 @@ __device__ void tile_forward(const MlpShared& sh, WaveTile& t, f4& y) {
         for (int i = 0; i < 4; ++i) {
             const int row = kq + i, col = nt * 16 + n0;
             const float z = acc[i] + sh.b2[col];
-            t.z2[row * kMlpHidden + col] = z;
             t.h2[row * kMlpHidden + col] = f2bf(gelu(z));
         }
     }
@@ -161,190 +149,262 @@ __global__ __launch_bounds__(256) void mlp_forward_kernel(MlpDevParams p, const 
     }
 }
 
-// Forward + backward over the batch; accumulates dL/dparam (FP32) into grad
-// and the summed loss into loss[0].  Each wavefront keeps its weight-gradient
-// partial sums in accumulator registers over its tiles and adds them to
-// global memory once.
-__global__ __launch_bounds__(256) void mlp_grad_kernel(MlpDevParams p, const float* __restrict__ x,
-                                                       const float* __restrict__ tgt, uint32_t rows,
-                                                       float inv_batch, float* __restrict__ grad,
-                                                       float* __restrict__ loss) {
-    __shared__ MlpShared sh;
-    __shared__ WaveTile tiles[4];
-    load_shared(sh, p);
-    __syncthreads();
+// Value of lane j of the lane's row of 16.
+template <int J>
+__device__ __forceinline__ float row_lane(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + J, 0xf, 0xf, true));
+}
+
+// GELU of z rounded to BF16, and its derivative (one erf for both).
+__device__ __forceinline__ short gelu_both(float z, float& grad) {
+    const float e = 1.0f + erff(z * 0.70710678118654752f);
+    const float pdf = 0.39894228040143268f * expf(-0.5f * z * z);
+    grad = 0.5f * e + z * pdf;
+    return f2bf(0.5f * z * e);
+}
+
+// Forward + backward over the batch: the workgroup's sums of dL/dparam and of
+// the loss.
+//
+// A tile of 16 rows is a chain of small products and GELUs (a batch has only a
+// few tiles per compute unit), so its length bounds the kernel: the four
+// wavefronts share each tile, wavefront w the hidden units 16w .. 16w+15.
+// In the accumulator layout a lane holds four rows of one unit, which is also
+// the operand layout of the products over rows (dW1, dW2): those operands, the
+// weights (packed in operand order), z's derivatives and the sums stay in
+// registers, and only h1, h2 and dZ2 pass through LDS.  The sums are stored
+// per workgroup and added by the update kernel.  8192 rows: 14 us; with one
+// atomic addition per wavefront and parameter and a tile per wavefront 51.
+constexpr int kRowPad = kMlpHidden + 8;   // shorts: 8-byte reads down the rows meet no bank twice
+
+__global__ __launch_bounds__(256) void mlp_grad_kernel(const MlpDevParams p, const float* __restrict__ x,
+                                                       const float* __restrict__ tgt, uint32_t rows, float inv_batch,
+                                                       float* __restrict__ partial) {
+    __shared__ __align__(8) short s_h1[16 * kRowPad], s_h2[16 * kRowPad], s_dz[16 * kRowPad];
+    __shared__ s4 s_dzf[4][64];   // dZ2 as the operand of dW2
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int n0 = lane & 15, kq = (lane >> 4) * 4;
-    WaveTile& t = tiles[wave];
-    f4 gw2[4][4], gw1[4];
-    for (int a = 0; a < 4; ++a) {
-        gw1[a] = f4{0.f, 0.f, 0.f, 0.f};
-        for (int b = 0; b < 4; ++b) gw2[a][b] = f4{0.f, 0.f, 0.f, 0.f};
+    const int n0 = lane & 15, kg = lane >> 4, kq = kg * 4, col = wave * 16 + n0;
+    const s4* frag = (const s4*)p.frag;
+    const s4 w1 = frag[wave * 64 + lane];
+    s4 w2[4], w2t[4], w3[4];
+#pragma unroll
+    for (int kc = 0; kc < 4; ++kc) {
+        w2[kc] = frag[256 + (wave * 4 + kc) * 64 + lane];
+        w2t[kc] = frag[256 + 1024 + (wave * 4 + kc) * 64 + lane];
+        w3[kc] = s4{0, 0, 0, 0};
+        if (n0 < kMlpOut) w3[kc] = frag[256 + 2048 + (kc * 4 + kg) * kMlpOut + n0];
     }
-    float gw3[2] = {0.f, 0.f};     // lane = hidden unit k: dW3[k][0..1]
-    float gb1 = 0.f, gb2 = 0.f;    // lane = hidden unit
-    float gb3[2] = {0.f, 0.f};
-    float lsum = 0.f;
+    const float b1 = p.b[col], b2 = p.b[kMlpHidden + col], b3 = n0 < kMlpOut ? p.b[2 * kMlpHidden + n0] : 0.f;
+    const float w30 = bf2f(p.w3[col * 16]), w31 = bf2f(p.w3[col * 16 + 1]);
+    const f4 zero = {0.f, 0.f, 0.f, 0.f};
+    f4 gw1 = zero, gw2[4] = {zero, zero, zero, zero};
+    float gb1 = 0.f, gb2 = 0.f, gb3 = 0.f, gw3[2] = {0.f, 0.f}, lsum = 0.f;
     const uint32_t ntiles = (rows + 15) / 16;
-    for (uint32_t tile = blockIdx.x * 4 + wave; tile < ntiles; tile += gridDim.x * 4) {
-        tile_load_x(t, x, tile * 16, rows);
-        f4 y;
-        tile_forward(sh, t, y);
-        // dL/dy
+    for (uint32_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+        s4 xa, xt;   // rows as the operand of layer 1, and of dW1
+        float t0[4], t2[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t ra = tile * 16 + n0, rt = tile * 16 + kq + i;
+            xa[i] = f2bf(ra < rows ? x[(size_t)ra * kMlpIn + kq + i] : 0.f);
+            xt[i] = f2bf(rt < rows ? x[(size_t)rt * kMlpIn + n0] : 0.f);
+            t0[i] = t2[i] = 0.f;
+            if (n0 < kMlpOut && rt < rows) {
+                t0[i] = tgt[(size_t)rt * kMlpTargets + n0];
+                t2[i] = tgt[(size_t)rt * kMlpTargets + 2];
+            }
+        }
+        s4 h1, h2;
+        float g1[4], g2[4];
+        f4 acc = mfma(xa, w1, zero);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            h1[i] = gelu_both(acc[i] + b1, g1[i]);
+            s_h1[(kq + i) * kRowPad + col] = h1[i];
+        }
+        __syncthreads();
+        acc = zero;
+#pragma unroll
+        for (int kc = 0; kc < 4; ++kc) acc = mfma(*(const s4*)&s_h1[n0 * kRowPad + kc * 16 + kq], w2[kc], acc);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            h2[i] = gelu_both(acc[i] + b2, g2[i]);
+            s_h2[(kq + i) * kRowPad + col] = h2[i];
+        }
+        __syncthreads();
+        acc = zero;   // every wavefront takes the two outputs
+#pragma unroll
+        for (int kc = 0; kc < 4; ++kc) acc = mfma(*(const s4*)&s_h2[n0 * kRowPad + kc * 16 + kq], w3[kc], acc);
+        float d[4] = {0.f, 0.f, 0.f, 0.f};   // dL/dy: lanes 0 and 1 of a row of 16
         if (n0 < kMlpOut)
+#pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const uint32_t r = tile * 16 + kq + i;
-                float d = 0.f;
-                if (r < rows) {
-                    const float* tr = tgt + (size_t)r * kMlpTargets;
-                    if (n0 == 0) {
-                        const float s = 1.f / (1.f + expf(-y[i]));
-                        d = s - tr[0];
-                        lsum += fmaxf(y[i], 0.f) - y[i] * tr[0] + log1pf(expf(-fabsf(y[i])));
-                    } else {
-                        const float e = y[i] - tr[1];
-                        d = 2.f * tr[2] * e;
-                        lsum += tr[2] * e * e;
-                    }
+                const float y = acc[i] + b3;
+                if (tile * 16 + kq + i >= rows) continue;
+                if (n0 == 0) {
+                    const float s = 1.f / (1.f + expf(-y));
+                    d[i] = s - t0[i];
+                    lsum += fmaxf(y, 0.f) - y * t0[i] + log1pf(expf(-fabsf(y)));
+                } else {
+                    const float e = y - t0[i];
+                    d[i] = 2.f * t2[i] * e;
+                    lsum += t2[i] * e * e;
                 }
-                t.dy[(kq + i) * 2 + n0] = d * inv_batch;
+                d[i] = d[i] * inv_batch;
+                gb3 += d[i];
             }
-        __builtin_amdgcn_s_waitcnt(0);
-        __builtin_amdgcn_wave_barrier();
-        // layer 3 gradients (K = 2: scalar); lane = hidden unit k
-        {
-            const int k = lane;
-            const float w30 = bf2f(sh.w3[k * 16 + 0]), w31 = bf2f(sh.w3[k * 16 + 1]);
-            for (int r = 0; r < 16; ++r) {
-                const float d0 = t.dy[r * 2], d1 = t.dy[r * 2 + 1];
-                const float h = bf2f(t.h2[r * kMlpHidden + k]);
-                gw3[0] += h * d0;
-                gw3[1] += h * d1;
-                const float dh = d0 * w30 + d1 * w31;
-                const float dz = dh * gelu_grad(t.z2[r * kMlpHidden + k]);
-                t.dz[r * kMlpHidden + k] = dz;
-                gb2 += dz;
-            }
-            if (lane < 2)
-                for (int r = 0; r < 16; ++r) gb3[lane] += t.dy[r * 2 + lane];
+        s4 dz2;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float d0 = row_lane<0>(d[i]), d1 = row_lane<1>(d[i]);
+            const float h = bf2f(h2[i]);
+            gw3[0] += h * d0;
+            gw3[1] += h * d1;
+            const float dz = (d0 * w30 + d1 * w31) * g2[i];
+            gb2 += dz;
+            dz2[i] = f2bf(dz);
+            s_dz[(kq + i) * kRowPad + col] = dz2[i];
         }
-        __builtin_amdgcn_s_waitcnt(0);
-        __builtin_amdgcn_wave_barrier();
+        s_dzf[wave][lane] = dz2;
+        __syncthreads();
         // dW2[k][j] += sum_r h1[r][k] dz2[r][j]   (M = k, N = j, K = r)
-        for (int mt = 0; mt < 4; ++mt) {
-            s4 a;
-            for (int i = 0; i < 4; ++i) a[i] = t.h1[(kq + i) * kMlpHidden + mt * 16 + n0];
-            for (int nt = 0; nt < 4; ++nt) {
-                s4 b;
-                for (int i = 0; i < 4; ++i) b[i] = f2bf(t.dz[(kq + i) * kMlpHidden + nt * 16 + n0]);
-                gw2[mt][nt] = mfma(a, b, gw2[mt][nt]);
-            }
-        }
+#pragma unroll
+        for (int nt = 0; nt < 4; ++nt) gw2[nt] = mfma(h1, s_dzf[nt][lane], gw2[nt]);
         // dH1[r][k] = sum_j dz2[r][j] W2[k][j]   (M = r, N = k, K = j)
-        f4 dh1[4];
-        for (int nt = 0; nt < 4; ++nt) {
-            f4 acc = {0.f, 0.f, 0.f, 0.f};
-            for (int kc = 0; kc < 4; ++kc) {
-                s4 a, b;
-                for (int i = 0; i < 4; ++i) {
-                    a[i] = f2bf(t.dz[n0 * kMlpHidden + kc * 16 + kq + i]);
-                    b[i] = sh.w2[(nt * 16 + n0) * kMlpHidden + kc * 16 + kq + i];
-                }
-                acc = mfma(a, b, acc);
-            }
-            dh1[nt] = acc;
+        acc = zero;
+#pragma unroll
+        for (int kc = 0; kc < 4; ++kc) acc = mfma(*(const s4*)&s_dz[n0 * kRowPad + kc * 16 + kq], w2t[kc], acc);
+        s4 dz1;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float dz = acc[i] * g1[i];
+            gb1 += dz;
+            dz1[i] = f2bf(dz);
         }
-        __builtin_amdgcn_s_waitcnt(0);
-        __builtin_amdgcn_wave_barrier();
-        // dZ1 = dH1 * gelu'(z1)
-        for (int nt = 0; nt < 4; ++nt)
-            for (int i = 0; i < 4; ++i) {
-                const int row = kq + i, col = nt * 16 + n0;
-                t.dz[row * kMlpHidden + col] = dh1[nt][i] * gelu_grad(t.z1[row * kMlpHidden + col]);
-            }
-        __builtin_amdgcn_s_waitcnt(0);
-        __builtin_amdgcn_wave_barrier();
-        for (int r = 0; r < 16; ++r) gb1 += t.dz[r * kMlpHidden + lane];
         // dW1[f][k] += sum_r x[r][f] dz1[r][k]   (M = f, N = k, K = r)
-        {
-            s4 a;
-            for (int i = 0; i < 4; ++i) a[i] = t.x[(kq + i) * kMlpIn + n0];
-            for (int nt = 0; nt < 4; ++nt) {
-                s4 b;
-                for (int i = 0; i < 4; ++i) b[i] = f2bf(t.dz[(kq + i) * kMlpHidden + nt * 16 + n0]);
-                gw1[nt] = mfma(a, b, gw1[nt]);
-            }
-        }
-        __builtin_amdgcn_s_waitcnt(0);
-        __builtin_amdgcn_wave_barrier();
+        gw1 = mfma(xt, dz1, gw1);
+        // the next tile writes s_h1, s_h2 and s_dz one barrier or more after
+        // this tile's last read of each
     }
-    // flush this wavefront's partial sums
-    float* gW1 = grad;
-    float* gB1 = grad + kMlpIn * kMlpHidden;
+    // sums over the four groups of rows
+    auto over_groups = [](float v) {
+        v += __shfl_xor(v, 16, 64);
+        return v + __shfl_xor(v, 32, 64);
+    };
+    gb1 = over_groups(gb1);
+    gb2 = over_groups(gb2);
+    gb3 = over_groups(gb3);
+    gw3[0] = over_groups(gw3[0]);
+    gw3[1] = over_groups(gw3[1]);
+    for (int off = 32; off > 0; off >>= 1) lsum += __shfl_xor(lsum, off, 64);
+    float* gW1 = partial + (size_t)blockIdx.x * kMlpPartial;
+    float* gB1 = gW1 + kMlpIn * kMlpHidden;
     float* gW2 = gB1 + kMlpHidden;
     float* gB2 = gW2 + kMlpHidden * kMlpHidden;
     float* gW3 = gB2 + kMlpHidden;
     float* gB3 = gW3 + kMlpHidden * kMlpOut;
-    for (int nt = 0; nt < 4; ++nt)
-        for (int i = 0; i < 4; ++i)
-            atomicAdd(&gW1[(kq + i) * kMlpHidden + nt * 16 + n0], gw1[nt][i]);
-    for (int mt = 0; mt < 4; ++mt)
-        for (int nt = 0; nt < 4; ++nt)
-            for (int i = 0; i < 4; ++i)
-                atomicAdd(&gW2[(mt * 16 + kq + i) * kMlpHidden + nt * 16 + n0], gw2[mt][nt][i]);
-    atomicAdd(&gB1[lane], gb1);
-    atomicAdd(&gB2[lane], gb2);
-    atomicAdd(&gW3[lane * kMlpOut + 0], gw3[0]);
-    atomicAdd(&gW3[lane * kMlpOut + 1], gw3[1]);
-    if (lane < 2) atomicAdd(&gB3[lane], gb3[lane]);
-    for (int off = 32; off > 0; off >>= 1) lsum += __shfl_xor(lsum, off, 64);
-    if (lane == 0) atomicAdd(loss, lsum * inv_batch);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        gW1[(kq + i) * kMlpHidden + col] = gw1[i];
+#pragma unroll
+        for (int nt = 0; nt < 4; ++nt) gW2[(wave * 16 + kq + i) * kMlpHidden + nt * 16 + n0] = gw2[nt][i];
+    }
+    if (kg == 0) {
+        gB1[col] = gb1;
+        gB2[col] = gb2;
+        gW3[col * kMlpOut] = gw3[0];
+        gW3[col * kMlpOut + 1] = gw3[1];
+        if (wave == 0 && n0 < kMlpOut) gB3[n0] = gb3;
+        if (wave == 0 && n0 == 0) gB3[kMlpOut] = lsum * inv_batch;
+    }
 }
 
-// Adam step on the FP32 master parameters.
-__global__ void mlp_adam_kernel(float* __restrict__ w, float* __restrict__ m, float* __restrict__ v,
-                                const float* __restrict__ g, int n, float lr, float b1, float b2,
-                                float eps, float c1, float c2) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float gi = g[i];
+// Writes parameter i's packed copies: FP32 biases, BF16 weights row by row
+// (W3 padded to 16 columns) and in operand order: of the K x N matrix a
+// product multiplies by, tile (nt, kc) of 16 x 16 holds for lane n + 16*(k/4)
+// elements k%4 (W1; W2; W2 transposed, for dH1; W3's two columns).
+__device__ __forceinline__ void pack_param(int i, float w, const MlpDevParams& p) {
+    constexpr int H = kMlpHidden;
+    auto tile = [](int k, int n) { return (((n >> 4) * 4 + (k >> 4)) * 64 + ((k >> 2) & 3) * 16 + (n & 15)) * 4 + (k & 3); };
+    if (i < kMlpIn * H) {
+        const int k = i / H, n = i % H;
+        p.w1[i] = f2bf(w);
+        p.frag[((n >> 4) * 64 + (k >> 2) * 16 + (n & 15)) * 4 + (k & 3)] = f2bf(w);
+        return;
+    }
+    i -= kMlpIn * H;
+    if (i < H) {
+        p.b[i] = w;
+        return;
+    }
+    i -= H;
+    if (i < H * H) {
+        const int k = i / H, n = i % H;
+        p.w2[i] = f2bf(w);
+        p.frag[kMlpIn * H + tile(k, n)] = f2bf(w);
+        p.frag[kMlpIn * H + H * H + tile(n, k)] = f2bf(w);
+        return;
+    }
+    i -= H * H;
+    if (i < H) {
+        p.b[H + i] = w;
+        return;
+    }
+    i -= H;
+    if (i < H * kMlpOut) {
+        const int k = i / kMlpOut, n = i % kMlpOut;
+        p.w3[k * 16 + n] = f2bf(w);
+        p.frag[kMlpIn * H + 2 * H * H + ((k >> 2) * kMlpOut + n) * 4 + (k & 3)] = f2bf(w);
+        return;
+    }
+    p.b[2 * H + i - H * kMlpOut] = w;
+}
+
+// Sums the workgroups' gradients, 32 parameters per workgroup, eight lanes to
+// a parameter; ADAM: the step on the FP32 master parameters and the packed
+// copies with it.  One launch (4.7 us) for what were two fills, the step and the
+// packing (18 us); it reads the partial sums once (5.5 MB at 256 workgroups).
+template <bool ADAM>
+__global__ __launch_bounds__(256) void mlp_update_kernel(const float* __restrict__ partial, uint32_t blocks,
+                                                         float* __restrict__ grad, float* __restrict__ loss,
+                                                         float* __restrict__ w, float* __restrict__ m,
+                                                         float* __restrict__ v, const MlpDevParams p, float lr,
+                                                         float b1, float b2, float eps, float c1, float c2) {
+    __shared__ float s_sum[8][32];
+    const int c = threadIdx.x & 31, part = threadIdx.x >> 5, i = blockIdx.x * 32 + c;
+    float sum = 0.f;
+    if (i <= kMlpParams)
+#pragma unroll 8
+        for (uint32_t b = part; b < blocks; b += 8) sum += partial[(size_t)b * kMlpPartial + i];
+    s_sum[part][c] = sum;
+    __syncthreads();
+    if (part != 0 || i > kMlpParams) return;
+    float gi = s_sum[0][c];
+#pragma unroll
+    for (int k = 1; k < 8; ++k) gi += s_sum[k][c];
+    if (i == kMlpParams) {
+        *loss = gi;
+        return;
+    }
+    grad[i] = gi;
+    if (!ADAM) return;
     const float mi = b1 * m[i] + (1.f - b1) * gi;
     const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
     m[i] = mi;
     v[i] = vi;
-    w[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+    const float wi = w[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+    w[i] = wi;
+    pack_param(i, wi, p);
 }
 
-// FP32 master -> BF16 weights (W3 padded to 16 columns) + FP32 biases.
 __global__ void mlp_pack_kernel(const float* __restrict__ w, MlpDevParams p) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const float* W1 = w;
-    const float* B1 = W1 + kMlpIn * kMlpHidden;
-    const float* W2 = B1 + kMlpHidden;
-    const float* B2 = W2 + kMlpHidden * kMlpHidden;
-    const float* W3 = B2 + kMlpHidden;
-    const float* B3 = W3 + kMlpHidden * kMlpOut;
-    if (i < kMlpIn * kMlpHidden) p.w1[i] = f2bf(W1[i]);
-    if (i < kMlpHidden * kMlpHidden) p.w2[i] = f2bf(W2[i]);
-    if (i < kMlpHidden * 16) {
-        const int k = i / 16, j = i % 16;
-        p.w3[i] = j < kMlpOut ? f2bf(W3[k * kMlpOut + j]) : (short)0;
-    }
-    if (i < kMlpHidden) {
-        p.b[i] = B1[i];
-        p.b[kMlpHidden + i] = B2[i];
-    }
-    if (i < kMlpOut) p.b[2 * kMlpHidden + i] = B3[i];
-}
-
-__global__ void zero_f32_kernel(float* p, int n) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = 0.f;
+    if (i < kMlpHidden * 16 && i % 16 >= kMlpOut) p.w3[i] = 0;
+    if (i < kMlpParams) pack_param(i, w[i], p);
 }
 
 void launch_mlp_pack(const float* master, const MlpDevParams& p, hipStream_t st) {
-    hipLaunchKernelGGL(mlp_pack_kernel, dim3((kMlpHidden * kMlpHidden + 255) / 256), dim3(256), 0, st,
-                       master, p);
+    hipLaunchKernelGGL(mlp_pack_kernel, dim3((kMlpParams + 255) / 256), dim3(256), 0, st, master, p);
 }
 
 void launch_mlp_forward(const MlpDevParams& p, const float* x, uint32_t rows, float* y, hipStream_t st) {
@@ -355,24 +415,26 @@ void launch_mlp_forward(const MlpDevParams& p, const float* x, uint32_t rows, fl
     hipLaunchKernelGGL(mlp_forward_kernel, dim3(blocks), dim3(256), 0, st, p, x, rows, y);
 }
 
-void launch_mlp_grad(const MlpDevParams& p, const float* x, const float* tgt, uint32_t rows,
-                     float* grad, float* loss, hipStream_t st) {
-    hipLaunchKernelGGL(zero_f32_kernel, dim3((kMlpParams + 1 + 255) / 256), dim3(256), 0, st, grad,
-                       kMlpParams);
-    hipLaunchKernelGGL(zero_f32_kernel, dim3(1), dim3(64), 0, st, loss, 1);
+uint32_t launch_mlp_grad(const MlpDevParams& p, const float* x, const float* tgt, uint32_t rows, float* partial,
+                         hipStream_t st) {
     const uint32_t ntiles = (rows + 15) / 16;
-    uint32_t blocks = (ntiles + 3) / 4;
-    if (blocks > 256) blocks = 256;
-    if (blocks == 0) return;
-    hipLaunchKernelGGL(mlp_grad_kernel, dim3(blocks), dim3(256), 0, st, p, x, tgt, rows,
-                       1.0f / (float)rows, grad, loss);
+    const uint32_t blocks = ntiles < kMlpGradBlocks ? ntiles : kMlpGradBlocks;
+    if (blocks)
+        hipLaunchKernelGGL(mlp_grad_kernel, dim3(blocks), dim3(256), 0, st, p, x, tgt, rows, 1.0f / (float)rows, partial);
+    return blocks;
 }
 
-void launch_mlp_adam(float* w, float* m, float* v, const float* g, float lr, int step, hipStream_t st) {
+void launch_mlp_sum(const float* partial, uint32_t blocks, float* grad, float* loss, hipStream_t st) {
+    hipLaunchKernelGGL(mlp_update_kernel<false>, dim3((kMlpParams + 1 + 31) / 32), dim3(256), 0, st, partial, blocks, grad,
+                       loss, nullptr, nullptr, nullptr, MlpDevParams{}, 0.f, 0.f, 0.f, 0.f, 1.f, 1.f);
+}
+
+void launch_mlp_update(const float* partial, uint32_t blocks, float* grad, float* loss, float* w, float* m, float* v,
+                       const MlpDevParams& p, float lr, int step, hipStream_t st) {
     const float b1 = 0.9f, b2 = 0.999f;
     const float c1 = 1.f - powf(b1, (float)step), c2 = 1.f - powf(b2, (float)step);
-    hipLaunchKernelGGL(mlp_adam_kernel, dim3((kMlpParams + 255) / 256), dim3(256), 0, st, w, m, v, g,
-                       kMlpParams, lr, b1, b2, 1e-8f, c1, c2);
+    hipLaunchKernelGGL(mlp_update_kernel<true>, dim3((kMlpParams + 1 + 31) / 32), dim3(256), 0, st, partial, blocks, grad,
+                       loss, w, m, v, p, lr, b1, b2, 1e-8f, c1, c2);
 }
 
 }  // namespace hipdvr
