@@ -158,8 +158,8 @@ __global__ __launch_bounds__(256, SHADE == 2 ? 4 : (SHADE == 1 ? (LEARNED || COU
                                                                      nsh);
                 }
                 ++n.rays;
-                n.fetched += (uint32_t)ns;
-                n.shaded += (uint32_t)nsh;
+                n.fetched += sub == 0 ? (uint32_t)ns : 0;   // the ray's, counted by one lane
+                n.shaded += sub == 0 ? (uint32_t)nsh : 0;
             } else if (a.dtype == 0) {
                 const CellFetch<uint8_t, WIDE> f = cell_fetch_of<uint8_t, WIDE>(a);
                 res = cell_ray<uint8_t, WIDE, SHADE, COUNT, P>(a, f, s_tf, s_alpha, px, py, sub, e, l, n);

@@ -244,22 +244,42 @@ __device__ __forceinline__ bool cell_gradient_interior(const CellFetch<T, WIDE>&
 }
 
 // Counters of a lane (COUNT builds); a lane marches few enough samples for 32
-// bits, the sums over the launch have 64.
+// bits, the sums over the launch have 64.  rays, skipped and the passes are the
+// ray's, alike in its P lanes; fetched and shaded are the lane's own samples.
 struct RayCounters {
     uint32_t rays = 0, skipped = 0, fetched = 0, shaded = 0, passes = 0, shade_passes = 0;
 };
 
-// Adds a lane's counters to the launch's, the wavefront marching 64 / P rays
-// with P lanes each (every lane of a ray holds its counts).  Slots: samples
-// its rays could have taken, a skipped sample counting as one.
+// Adds the lanes' counters to the launch's, the wavefronts marching 64 / P rays
+// with P lanes each.  Slots: samples a wavefront's rays could have taken, a
+// skipped sample counting as one.  Every thread of a workgroup of 256 calls it:
+// the counters lie in one line, so a workgroup adds them with one instruction.
+// Counted 256^3 Phong frame, 512^2 with four lanes per ray: 559 us with an
+// atomic per wavefront and counter and samples counted by every lane of a ray,
+// 326 so (270 without counters).
 template <int P>
 __device__ __forceinline__ void add_counters(unsigned long long* c, const RayCounters& n, bool own) {
-    wave_add(c + 0, own ? n.rays : 0);
-    wave_add(c + 1, own ? n.skipped + n.fetched : 0);
-    wave_add(c + 2, own ? n.fetched : 0);
-    wave_add(c + 3, own ? n.shaded : 0);
-    wave_add_max64(c + 4, n.passes * P + n.skipped, 64 / P);
-    wave_add_max64(c + 5, n.shade_passes * P, 64 / P);
+    __shared__ uint32_t s_count[4][kNumCounters];
+    uint32_t v[kNumCounters] = {own ? n.rays : 0, (own ? n.skipped : 0) + n.fetched, n.fetched, n.shaded,
+                                n.passes * P + n.skipped, n.shade_passes * P};
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1)
+#pragma unroll
+        for (int k = 0; k < kNumCounters; ++k) {
+            const uint32_t o = __shfl_xor(v[k], off, 64);
+            v[k] = k < 4 ? v[k] + o : (o > v[k] ? o : v[k]);
+        }
+    if ((threadIdx.x & 63) == 0) {
+#pragma unroll
+        for (int k = 0; k < kNumCounters; ++k) s_count[threadIdx.x >> 6][k] = k < 4 ? v[k] : v[k] * (64 / P);
+    }
+    __syncthreads();
+    if (threadIdx.x < kNumCounters) {
+        unsigned long long sum = 0;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) sum += s_count[w][threadIdx.x];
+        if (sum) atomicAdd(c + threadIdx.x, sum);
+    }
 }
 
 // Lanes per ray.  P neighbouring lanes of a wavefront (1, 2, 4, 8 or 16)
@@ -315,13 +335,24 @@ __device__ __forceinline__ uint32_t sub_value(uint32_t v, int j) {
     return __float_as_uint(sub_value<P>(__uint_as_float(v), j));
 }
 
-// Counts one sample of a pass (COUNT builds): cj its opacity (-1: past the
-// ray's end), A the ray's before it.
-template <int SHADE>
-__device__ __forceinline__ void count_sample(RayCounters& n, float cj, float A) {
-    const bool on = cj >= 0.0f && A < kErtOpacity;
+// Counts this lane's sample of a pass (COUNT builds): ca its opacity (-1: past
+// the ray's end); A0 and A the ray's opacity before and after the pass.  Where
+// the ray ended in the pass, the samples up to the one that ended it count.
+template <int SHADE, int P>
+__device__ __forceinline__ void count_pass(RayCounters& n, float ca, float A0, float A, int sub) {
+    bool on = ca >= 0.0f;
+    if (A >= kErtOpacity) {
+        const float cz = fmaxf(ca, 0.0f);
+        float before = A0;
+#pragma unroll
+        for (int j = 0; j < P - 1; ++j) {
+            const float next = before + (1.0f - before) * sub_value<P>(cz, j);
+            before = j < sub ? next : before;
+        }
+        on = on && before < kErtOpacity;
+    }
     n.fetched += on ? 1 : 0;
-    if (SHADE) n.shaded += on && cj > 0.0f ? 1 : 0;
+    if (SHADE) n.shaded += on && ca > 0.0f ? 1 : 0;
 }
 
 // The place of a wavefront's rays in the image: 64 / P rays, ray_w<P>() wide.
@@ -478,7 +509,6 @@ __device__ __forceinline__ void cell_march(const MarchArgs& a, const CellFetch<T
             for (int j = 0; j < P; ++j) {
                 const float cj = sub_value<P>(ca, j);
                 const float c0 = sub_value<P>(col[0], j), c1 = sub_value<P>(col[1], j), c2 = sub_value<P>(col[2], j);
-                if (COUNT) count_sample<SHADE>(n, cj, A);
                 if (cj > 0.0f && A < kErtOpacity) {
                     const float wgt = (1.0f - A) * cj;
                     r = r + wgt * c0;
@@ -492,7 +522,6 @@ __device__ __forceinline__ void cell_march(const MarchArgs& a, const CellFetch<T
             const float cz = fmaxf(ca, 0.0f);
 #pragma unroll
             for (int j = 0; j < P; ++j) {
-                if (COUNT) count_sample<SHADE>(n, sub_value<P>(ca, j), A);
                 const float wgt = (1.0f - A) * sub_value<P>(cz, j);
                 r = r + wgt * sub_value<P>(col[0], j);
                 g = g + wgt * sub_value<P>(col[1], j);
@@ -501,6 +530,7 @@ __device__ __forceinline__ void cell_march(const MarchArgs& a, const CellFetch<T
                 A = A >= kErtOpacity ? 1.0f : A;
             }
         }
+        if (COUNT) count_pass<SHADE, P>(n, ca, A0, A, sub);
         probe = A == A0;
         loop += P;
         t = t_next;

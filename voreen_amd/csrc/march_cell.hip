@@ -10,7 +10,7 @@ namespace hipdvr {
 // A workgroup is 2x2 waves of ray_w<P>() x ray_h<P>() rays, P lanes per ray: a
 // P-th of a 16x16 pixel tile.
 template <typename T, bool WIDE, int SHADE, bool COUNT, int P>
-__global__ __launch_bounds__(256, SHADE == 2 ? 4 : (SHADE == 1 && COUNT ? 5 : 6)) void march_cell_kernel(const MarchArgs a, const uint32_t tiles_x,
+__global__ __launch_bounds__(256, SHADE == 2 ? 4 : 6) void march_cell_kernel(const MarchArgs a, const uint32_t tiles_x,
                                                          const uint32_t tiles_y) {
     // XCD-compact tile order (xcd_tile): each XCD marches one compact region
     // of tiles, the chip one compact image area; the P workgroups of a tile

@@ -311,11 +311,10 @@ __global__ __launch_bounds__(256, GRAD ? 4 : 6) void march_modes_cell_kernel(con
                         const float aj = sub_value<P>(m.alpha, j);
                         const float c[3] = {sub_value<P>(m.c[0], j), sub_value<P>(m.c[1], j), sub_value<P>(m.c[2], j)};
                         const float rj = PREINT ? 0.0f : sub_value<P>(m.rw, j);
-                        const uint32_t sj = COUNT && GRAD ? sub_value<P>((uint32_t)shaded, j) : 0;
                         if (!(aj >= -1.0f) || finished) continue;
-                        if (COUNT) {
+                        if (COUNT && sub == j) {
                             ++n.fetched;
-                            n.shaded += sj;
+                            n.shaded += shaded ? 1 : 0;
                         }
                         if (!(aj >= 0.0f)) continue;
                         probe = mip && skips;   // MIP: the bricks ahead may lie below the new maximum
