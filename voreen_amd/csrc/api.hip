@@ -135,26 +135,104 @@ void ensure_occupancy(hipdvr_ctx* ctx, hipdvr_volume* vol, const hipdvr_tf* tf) 
     std::memcpy(vol->occ_key, key.k, sizeof key.k);
 }
 
-// The same for the skip grid of the cell kernels; iso for kSkipIso.
-void ensure_skip(hipdvr_ctx* ctx, hipdvr_volume* vol, const hipdvr_tf* tf, SkipRule rule, float iso) {
+namespace {
+
+// Whether a graph is being captured from the context's stream.
+bool capturing(const hipdvr_ctx* ctx) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx->stream, &cs) == hipSuccess) return cs != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();   // not left for the next call
+    return false;
+}
+
+// Orders the context's stream (or, while that is captured, the caller) after
+// what the context submitted to `other` before it left it.
+void wait_left(hipdvr_ctx* ctx, hipStream_t other, bool on_host) {
+    for (const hipdvr_ctx::Left& l : ctx->left) {
+        if (l.stream != other) continue;
+        if (!on_host) {
+            hip_check(hipStreamWaitEvent(ctx->stream, l.event, 0), "hipStreamWaitEvent");
+        } else {
+            hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+            hip_check(hipThreadExchangeStreamCaptureMode(&mode), "hipThreadExchangeStreamCaptureMode");
+            const hipError_t e = hipEventSynchronize(l.event);
+            (void)hipThreadExchangeStreamCaptureMode(&mode);
+            hip_check(e, "hipEventSynchronize");
+        }
+        return;
+    }
+}
+
+// The context leaves its stream: an event behind what it submitted there.
+// Never fails: without an event, the device is waited for.
+void leave_stream(hipdvr_ctx* ctx) {
+    constexpr size_t kMaxLeft = 64;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    hipError_t e = hipStreamIsCapturing(ctx->stream, &cs);
+    if (e == hipSuccess && cs != hipStreamCaptureStatusNone) return;   // that work belongs to a graph
+    hipEvent_t ev = nullptr;
+    for (const hipdvr_ctx::Left& l : ctx->left)
+        if (l.stream == ctx->stream) ev = l.event;
+    if (e == hipSuccess && !ev) {
+        if (ctx->left.size() >= kMaxLeft) {
+            (void)hipEventSynchronize(ctx->left.front().event);
+            (void)hipEventDestroy(ctx->left.front().event);
+            ctx->left.erase(ctx->left.begin());
+        }
+        e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
+        if (e == hipSuccess) ctx->left.push_back({ctx->stream, ev});
+    }
+    if (e == hipSuccess) e = hipEventRecord(ev, ctx->stream);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        (void)hipDeviceSynchronize();
+        (void)hipGetLastError();
+    }
+}
+
+}  // namespace
+
+// The same for the skip grids of the cell kernels; iso for kSkipIso.
+const uint8_t* ensure_skip(hipdvr_ctx* ctx, hipdvr_volume* vol, const hipdvr_tf* tf, SkipRule rule, float iso) {
     const MappingKey key(vol, tf);
     uint64_t k[5];
     std::memcpy(k, key.k, sizeof key.k);
     if (rule == kSkipPairs) k[0] = tf->preint_serial;
     k[4] = ((uint64_t)rule << 32) | (rule == kSkipIso ? fbits(iso) : 0);
-    if (std::memcmp(k, vol->skip_key, sizeof k) == 0) return;
+    const hipStream_t st = ctx->stream;
+    const bool in_capture = capturing(ctx);
+    for (SkipGrid& g : vol->skips) {
+        if (g.in_graph || std::memcmp(k, g.key, sizeof k) != 0) continue;
+        if (std::find(g.streams.begin(), g.streams.end(), st) == g.streams.end()) {
+            wait_left(ctx, g.streams.front(), in_capture);
+            g.streams.push_back(st);
+        }
+        g.captured = g.captured || in_capture;
+        return g.d;
+    }
+    SkipGrid* g = nullptr;
+    for (SkipGrid& s : vol->skips)
+        if (!in_capture && s.rule == rule && !s.captured) g = &s;
+    if (!g) g = &add_skip_grid(vol, rule);
+    // after the frames that still read it
+    for (const hipStream_t s : g->streams)
+        if (s != st) wait_left(ctx, s, false);
+    std::memset(g->key, 0, sizeof g->key);
+    g->streams.assign(1, st);
+    g->captured = g->in_graph = in_capture;
     OccArgs o = occupancy_args(vol, tf, vol->d_minmax8, vol->skip_count);
     if (rule == kSkipIso) {
-        launch_iso_prefix(tf->d_rgba, tf->width, iso, vol->d_band, ctx->stream);
-        o.alpha_prefix = vol->d_band;
+        launch_iso_prefix(tf->d_rgba, tf->width, iso, g->d_band, st);
+        o.alpha_prefix = g->d_band;
     } else if (rule == kSkipPairs) {
-        launch_pair_reach(tf->d_preint, tf->preint_n, vol->d_band, ctx->stream);
+        launch_pair_reach(tf->d_preint, tf->preint_n, g->d_band, st);
         o.tf_width = (int32_t)tf->preint_n;
-        o.pair_reach = vol->d_band;
+        o.pair_reach = g->d_band;
     }
-    launch_skip_grid(o, vol->nskip, vol->d_skip, vol->d_skip + vol->skip_count, ctx->stream);
+    launch_skip_grid(o, vol->nskip, g->d, g->d + vol->skip_count, st);
     hip_check(hipGetLastError(), "skip grid kernel launch");
-    std::memcpy(vol->skip_key, k, sizeof k);
+    std::memcpy(g->key, k, sizeof k);
+    return g->d;
 }
 
 // Opacity correction per alpha byte: cpuraycaster.cpp:291 with the TF colour
@@ -209,7 +287,7 @@ void fill_march_args(MarchArgs& a, const hipdvr_volume* vol, const hipdvr_tf* tf
     a.occ_bits = vol->d_occ_bits;
     a.occ_words = vol->occ_words;
     a.brick_log2 = v.brick_log2;
-    a.skip = vol->d_skip;
+    a.skip = nullptr;   // ensure_skip
     a.skip_minmax = vol->d_minmax8;
     a.skip_log2 = kSkipLog2;
     for (int i = 0; i < 3; ++i) {
@@ -335,15 +413,12 @@ void render_device_impl(hipdvr_ctx* ctx, const hipdvr_volume* vol, const hipdvr_
     // records as well (march_cell_modes.hip), with the same results in less
     // time than the reference-layout kernels at every size measured (there).
     // Those stay for the volumes whose records do not fit, and while the
-    // stream is captured: a graph would replay without the skip grid of its
-    // mapping.
+    // stream is captured (records are built outside of a graph).
     bool cell_modes = p->kernel == HIPDVR_KERNEL_AUTO && kernel == HIPDVR_KERNEL_REFERENCE && !other_gradient &&
                       p->filter == HIPDVR_FILTER_LINEAR && p->classification != HIPDVR_CLASS_TF2D &&
                       (modes || p->classification == HIPDVR_CLASS_PREINT) && cells_allowed(vol);
     if (cell_modes) {
-        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-        cell_modes = hipStreamIsCapturing(ctx->stream, &cs) == hipSuccess && cs == hipStreamCaptureStatusNone &&
-                     try_cells(mvol, ctx->stream);
+        cell_modes = !capturing(ctx) && try_cells(mvol, ctx->stream);
     }
     const bool cell = kernel == HIPDVR_KERNEL_CELL;
     const bool slab = kernel == HIPDVR_KERNEL_SLAB;
@@ -360,7 +435,7 @@ void render_device_impl(hipdvr_ctx* ctx, const hipdvr_volume* vol, const hipdvr_
     }
     if (kernel == HIPDVR_KERNEL_BRICKED || slab) ensure_occupancy(ctx, mvol, tf);
     if (cell) {
-        ensure_skip(ctx, mvol, tf);
+        a.skip = ensure_skip(ctx, mvol, tf);
         ensure_cells(mvol, ctx->stream);
         a.cells = mvol->d_cells;
     }
@@ -371,11 +446,10 @@ void render_device_impl(hipdvr_ctx* ctx, const hipdvr_volume* vol, const hipdvr_
         if (modes) {
             // the counters hold every sample that a light would have reached
             const bool band = p->compositing == HIPDVR_COMPOSITE_ISO && !(count && phong);
-            ensure_skip(ctx, mvol, tf, band ? kSkipIso : kSkipAlpha, p->iso_value);
+            a.skip = ensure_skip(ctx, mvol, tf, band ? kSkipIso : kSkipAlpha, p->iso_value);
         } else if (p->step * longest <= 7.5f) {
-            ensure_skip(ctx, mvol, tf, kSkipPairs);
-        } else {
-            a.skip = nullptr;   // a sample's predecessor may lie two bricks back
+            // (beyond, a sample's predecessor may lie two bricks back)
+            a.skip = ensure_skip(ctx, mvol, tf, kSkipPairs);
         }
     }
     if (count) hip_check(hipEventRecord(ctx->ev0, ctx->stream), "hipEventRecord");
@@ -509,6 +583,7 @@ int hipdvr_destroy(hipdvr_ctx* ctx) {
     if (ctx->ev0) (void)hipEventDestroy(ctx->ev0);
     if (ctx->ev1) (void)hipEventDestroy(ctx->ev1);
     for (hipEvent_t e : ctx->tev) (void)hipEventDestroy(e);
+    for (const hipdvr_ctx::Left& l : ctx->left) (void)hipEventDestroy(l.event);
     if (ctx->own_stream) (void)hipStreamDestroy(ctx->own_stream);
     delete ctx;
     return HIPDVR_OK;
@@ -516,7 +591,12 @@ int hipdvr_destroy(hipdvr_ctx* ctx) {
 
 int hipdvr_set_stream(hipdvr_ctx* ctx, void* stream) {
     if (!ctx) return HIPDVR_ERR_INVALID;
-    ctx->stream = stream ? (hipStream_t)stream : ctx->own_stream;
+    const hipStream_t next = stream ? (hipStream_t)stream : ctx->own_stream;
+    if (next != ctx->stream) {
+        (void)hipSetDevice(ctx->device);
+        leave_stream(ctx);
+        ctx->stream = next;
+    }
     return HIPDVR_OK;
 }
 

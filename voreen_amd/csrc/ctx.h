@@ -28,6 +28,13 @@ struct hipdvr_ctx {
     float* d_stage = nullptr;
     float* h_stage = nullptr;
     size_t stage_bytes = 0;                      // each of the two, 3 images
+    // streams the context has left (hipdvr_set_stream), with an event behind
+    // the work it had submitted there
+    struct Left {
+        hipStream_t stream;
+        hipEvent_t event;
+    };
+    std::vector<Left> left;
 };
 
 namespace hipdvr {

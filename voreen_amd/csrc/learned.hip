@@ -286,12 +286,13 @@ SparseGrid sparse_grid(hipdvr_learned* l, uint32_t w, uint32_t h, uint32_t strid
 }
 
 // The plain re-march of the sparse pixels into d_out (g.w x g.h RGBA).
-void launch_sparse(hipdvr_learned* l, hipdvr_volume* vol, const hipdvr_tf* tf, const hipdvr_params* prm,
-                   const float* d_entry, const float* d_exit, uint32_t w, uint32_t h, const SparseGrid& g, int shade,
-                   float* d_out, hipStream_t st) {
+void launch_sparse(hipdvr_learned* l, hipdvr_volume* vol, const hipdvr_tf* tf, const uint8_t* skip,
+                   const hipdvr_params* prm, const float* d_entry, const float* d_exit, uint32_t w, uint32_t h,
+                   const SparseGrid& g, int shade, float* d_out, hipStream_t st) {
     MarchArgs sp;
     fill_march_args(sp, vol, tf, prm, d_entry, d_exit, d_out, w, h, nullptr);
     sp.cells = vol->d_cells;
+    sp.skip = skip;
     sp.grid_w = g.w;
     sp.grid_h = g.h;
     sp.stride = (int32_t)g.stride;
@@ -578,7 +579,7 @@ int hipdvr_render_learned_device(hipdvr_learned* l, const hipdvr_tf* tf, const f
         ctx_set_device(l->ctx);
         hipStream_t st = ctx_stream(l->ctx);
         hipdvr_volume* vol = const_cast<hipdvr_volume*>(l->vol);
-        ensure_skip(l->ctx, vol, tf);
+        const uint8_t* skip = ensure_skip(l->ctx, vol, tf);
         const SparseGrid sg = sparse_grid(l, w, h, (uint32_t)opts.remarch_stride);
         const uint32_t stride = sg.stride, offs = sg.offs;
         const int swc = sg.w, shc = sg.h;
@@ -594,6 +595,7 @@ int hipdvr_render_learned_device(hipdvr_learned* l, const hipdvr_tf* tf, const f
             ensure_cells(vol, st);
             MarchArgs pa;
             fill_march_args(pa, vol, tf, prm, d_entry, d_exit, d_out, w, h, count ? l->ctx->d_counters : nullptr);
+            pa.skip = skip;
             launch_march_cell(pa, vol->desc.dtype, shade, count, vol->cells_wide, 0, st);
             hip_check(hipGetLastError(), "learned render launch");
             if (timed0) ctx_timing_stop(l->ctx);
@@ -614,11 +616,12 @@ int hipdvr_render_learned_device(hipdvr_learned* l, const hipdvr_tf* tf, const f
         ensure_cells(vol, st);
         hip_check(hipEventRecord(l->fork, st), "hipEventRecord");
         hip_check(hipStreamWaitEvent(l->side, l->fork, 0), "hipStreamWaitEvent");
-        launch_sparse(l, vol, tf, prm, d_entry, d_exit, w, h, sg, shade, (float*)l->d_sparse, l->side);
+        launch_sparse(l, vol, tf, skip, prm, d_entry, d_exit, w, h, sg, shade, (float*)l->d_sparse, l->side);
         hip_check(hipEventRecord(l->join, l->side), "hipEventRecord");
         LearnedArgs la;
         fill_learned_args(la, l, tf, prm, d_entry, d_exit, d_out, w, h);
         la.m.cells = vol->d_cells;
+        la.m.skip = skip;
         // Two lanes per ray sooner than the plain frame: the passes that skip
         // bricks are taken by all lanes of a ray alike.  512^3, 1024^2 with a
         // trained network, frames/s with 1 / 2 / 4 lanes: 1040 / 1543 / 1261.
@@ -634,6 +637,7 @@ int hipdvr_render_learned_device(hipdvr_learned* l, const hipdvr_tf* tf, const f
         // 4. fallback: the plain frame, launched always, runs only if flagged
         MarchArgs fb;
         fill_march_args(fb, vol, tf, prm, d_entry, d_exit, d_out, w, h, nullptr);
+        fb.skip = skip;
         fb.cond_flag = l->d_flag;
         launch_march_cell(fb, vol->desc.dtype, shade, false, vol->cells_wide, 0, st);
         hip_check(hipGetLastError(), "learned render launch");
@@ -686,11 +690,11 @@ int hipdvr_learned_sparse_remarch(hipdvr_learned* l, const hipdvr_tf* tf, const 
         ctx_set_device(l->ctx);
         hipStream_t st = ctx_stream(l->ctx);
         hipdvr_volume* vol = const_cast<hipdvr_volume*>(l->vol);
-        ensure_skip(l->ctx, vol, tf);
+        const uint8_t* skip = ensure_skip(l->ctx, vol, tf);
         ensure_cells(vol, st);
         const SparseGrid g = sparse_grid(l, w, h, (uint32_t)opts.remarch_stride);
         const int shade = prm->shading == HIPDVR_SHADE_PHONG ? (prm->exact_shading ? 2 : 1) : 0;
-        launch_sparse(l, vol, tf, prm, d_entry, d_exit, w, h, g, shade, d_sparse, st);
+        launch_sparse(l, vol, tf, skip, prm, d_entry, d_exit, w, h, g, shade, d_sparse, st);
         hip_check(hipGetLastError(), "sparse re-march launch");
         hip_check(hipStreamSynchronize(st), "hipStreamSynchronize");
         *sw = (uint32_t)g.w;

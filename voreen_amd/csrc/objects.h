@@ -41,8 +41,10 @@ void fill_march_args(MarchArgs& a, const hipdvr_volume* vol, const hipdvr_tf* tf
                      unsigned long long* counters);
 OccArgs occupancy_args(const hipdvr_volume* vol, const hipdvr_tf* tf, const uint2* minmax, uint64_t count);
 void ensure_occupancy(hipdvr_ctx* ctx, hipdvr_volume* vol, const hipdvr_tf* tf);
-void ensure_skip(hipdvr_ctx* ctx, hipdvr_volume* vol, const hipdvr_tf* tf, SkipRule rule = kSkipAlpha,
-                 float iso = 0.0f);
+// The skip grid of vol for the rule and the mapping, ready for a frame on the
+// context's stream.
+const uint8_t* ensure_skip(hipdvr_ctx* ctx, hipdvr_volume* vol, const hipdvr_tf* tf, SkipRule rule = kSkipAlpha,
+                           float iso = 0.0f);
 uint64_t next_serial();   // of objects and tables, never the same twice
 // Opacity-corrected 2D table for this step on the device (host powf, as
 // cpuraycaster.cpp:289 evaluates it per sample).

@@ -28,7 +28,7 @@
 //             voxel value over the brick extended by one voxel on the upper
 //             side of every axis (clamped to the volume): every trilinear or
 //             nearest footprint whose lower corner lies in the brick is inside.
-//   d_skip    the skip grid of the cell kernels for the last TF mapping: per
+//   skips     skip grids of the cell kernels (SkipGrid), each for one TF mapping: per
 //             brick of 8^3 voxels 0 when it may hold alpha > 0, else the
 //             Chebyshev distance in bricks to the nearest brick that may (at
 //             most kSkipReach).  A ray crosses all bricks within distance - 1
@@ -41,6 +41,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <vector>
+
 #include "../../include/hipdvr.h"
 
 namespace hipdvr {
@@ -52,6 +54,23 @@ constexpr uint32_t kBandWords = 4100;
 // alpha lies outside the isosurface band; those whose pre-integrated entry
 // (with any predecessor from a neighbouring brick) has alpha 0.
 enum SkipRule { kSkipAlpha = 0, kSkipIso = 1, kSkipPairs = 2 };
+constexpr int kSkipRules = 3;
+
+// A skip grid.  Every rule has one that is rebuilt for each new mapping, so
+// that frames of different modes do not take each other's; a grid that a
+// captured frame reads is never rebuilt (its graph may be replayed at any
+// time), and a mapping that is not there yet while the stream is captured gets
+// a grid of its own, which the graph builds and no other frame uses.
+struct SkipGrid {
+    SkipRule rule = kSkipAlpha;
+    uint8_t* d = nullptr;            // the grid, and as many bytes of scratch behind it
+    uint32_t* d_band = nullptr;      // [kBandWords] table of the rule
+    uint64_t key[5] = {0, 0, 0, 0, 0};
+    bool captured = false;           // a captured frame reads it
+    bool in_graph = false;           // its build is part of a graph
+    // streams that are ordered after its build, the builder's first
+    std::vector<hipStream_t> streams;
+};
 
 struct VolumeDesc {
     uint32_t dims[3];
@@ -78,11 +97,11 @@ struct hipdvr_volume {
     uint64_t brick_count = 0;
     uint64_t tiled_elems = 0;
     uint2* d_minmax8 = nullptr;      // ranges of the 8^3 bricks
-    uint8_t* d_skip = nullptr;       // skip grid for the last TF mapping, and as many bytes of scratch
     uint32_t nskip[3] = {0, 0, 0};   // 8^3 bricks per axis
     uint64_t skip_count = 0;
-    uint64_t skip_key[5] = {0, 0, 0, 0, 0};
-    uint32_t* d_band = nullptr;      // [kBandWords] table of the skip grid's rule (SkipRule)
+    // the rules' own grids (in the allocation of d_minmax), then those that
+    // captured frames made necessary (each an allocation)
+    std::vector<hipdvr::SkipGrid> skips;
     void* d_cells = nullptr;         // cell records (null until first use)
     uint64_t cell_bytes = 0;
     bool cells_wide = false;         // more than 2^32 - 256 bytes: 64-bit addressing
@@ -130,6 +149,8 @@ struct OccArgs {
     const uint32_t* pair_reach;
 };
 void launch_occupancy(const OccArgs& a, hipStream_t st);
+// A further skip grid of the volume, also while a stream is captured.
+hipdvr::SkipGrid& add_skip_grid(hipdvr_volume* vol, SkipRule rule);
 // Skip grid (see above) of nb bricks from the ranges in a (a.occ and a.bits
 // unused); scratch holds as many bytes as the grid.
 void launch_skip_grid(const OccArgs& a, const uint32_t nb[3], uint8_t* skip, uint8_t* scratch, hipStream_t st);

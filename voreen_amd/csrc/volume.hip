@@ -437,6 +437,20 @@ void launch_pair_reach(const float4* table, uint32_t n, uint32_t* reach, hipStre
     hipLaunchKernelGGL(pair_reach_kernel, dim3(1), dim3(1024), 0, st, reach, n);
 }
 
+SkipGrid& add_skip_grid(hipdvr_volume* v, SkipRule rule) {
+    SkipGrid g;
+    g.rule = rule;
+    // an allocation is no part of a graph, and disturbs none
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    hip_check(hipThreadExchangeStreamCaptureMode(&mode), "hipThreadExchangeStreamCaptureMode");
+    const hipError_t e = hipMalloc((void**)&g.d_band, kBandWords * 4 + 2 * v->skip_count);
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    hip_check(e, "hipMalloc(skip grid)");
+    g.d = (uint8_t*)(g.d_band + kBandWords);
+    v->skips.push_back(g);
+    return v->skips.back();
+}
+
 hipdvr_volume* volume_create(hipdvr_ctx* ctx, hipStream_t st, const hipdvr_volume_desc* d,
                              const void* voxels, bool on_device) {
     for (int i = 0; i < 3; ++i)
@@ -471,21 +485,28 @@ hipdvr_volume* volume_create(hipdvr_ctx* ctx, hipStream_t st, const hipdvr_volum
         hip_check(hipMalloc(&v->d_linear, bytes), "hipMalloc(volume)");
         hip_check(hipMalloc(&v->d_tiled, v->tiled_elems * vsz), "hipMalloc(tiled volume)");
         // the brick tables in one allocation: ranges of the volume's bricks and
-        // of the 8^3 bricks, occupancy bits and bytes, skip grid and scratch
+        // of the 8^3 bricks, occupancy bits, the tables and grids (with scratch)
+        // of the skip rules, occupancy bytes
         v->occ_words = (uint32_t)((v->brick_count + 31) / 32);
         const size_t mm = v->brick_count * sizeof(uint2), mm8 = v->skip_count * sizeof(uint2);
         const size_t words = ((size_t)v->occ_words * 4 + 7) & ~(size_t)7;
         char* p = nullptr;
-        hip_check(hipMalloc((void**)&p, mm + mm8 + words + v->brick_count + 2 * v->skip_count +
-                                              kBandWords * 4 + 4),
+        hip_check(hipMalloc((void**)&p, mm + mm8 + words + kSkipRules * (kBandWords * 4 + 2 * v->skip_count) +
+                                              v->brick_count),
                   "hipMalloc(bricks)");
         v->d_minmax = (uint2*)p;
         v->d_minmax8 = (uint2*)(p + mm);
         v->d_occ_bits = (uint32_t*)(p + mm + mm8);
-        v->d_occ = (uint8_t*)(p + mm + mm8 + words);
-        v->d_skip = v->d_occ + v->brick_count;
-        const size_t band = mm + mm8 + words + v->brick_count + 2 * v->skip_count;
-        v->d_band = (uint32_t*)(p + ((band + 3) & ~(size_t)3));
+        uint32_t* band = (uint32_t*)(p + mm + mm8 + words);
+        uint8_t* bytes_at = (uint8_t*)(band + kSkipRules * kBandWords);
+        v->skips.resize(kSkipRules);
+        for (int r = 0; r < kSkipRules; ++r) {
+            v->skips[r].rule = (SkipRule)r;
+            v->skips[r].d_band = band + r * kBandWords;
+            v->skips[r].d = bytes_at;
+            bytes_at += 2 * v->skip_count;
+        }
+        v->d_occ = bytes_at;
         hip_check(hipMemcpyAsync(v->d_linear, voxels, bytes,
                                  on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, st),
                   "volume upload");
@@ -610,6 +631,7 @@ void volume_destroy(hipdvr_volume* v) {
     if (v->d_linear) (void)hipFree(v->d_linear);
     if (v->d_tiled) (void)hipFree(v->d_tiled);
     if (v->d_minmax) (void)hipFree(v->d_minmax);   // and the tables behind it
+    for (size_t i = kSkipRules; i < v->skips.size(); ++i) (void)hipFree(v->skips[i].d_band);
     if (v->d_grad) (void)hipFree(v->d_grad);
     delete v;
 }
