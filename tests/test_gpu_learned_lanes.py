@@ -1,0 +1,87 @@
+"""The learned march with 2 and 4 lanes per ray: its samples do not depend on
+the number of lanes, whatever the loop cap, so a frame of 2 lanes, one of 4 and
+the batched launch give the same image bit for bit."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def network(H, ctx):
+    """Skips nearly transparent bricks, steps further where the opacity of 32
+    samples (input 7) and the standard deviation (input 3) are small."""
+    w1, w2, w3 = np.zeros((16, 64), np.float32), np.zeros((64, 64), np.float32), np.zeros((64, 2), np.float32)
+    for u, (f, s) in enumerate(((7, 64.0), (7, 2.0), (3, 10.0))):
+        w1[f, u], w2[u, u] = s, 1.0
+    w3[0, 0], w3[1, 1], w3[2, 1] = -1.0, -1.0, -1.0
+    z = np.zeros(64, np.float32)
+    m = H.Mlp(ctx)
+    m.set_params(np.concatenate([w1.ravel(), z, w2.ravel(), z, w3.ravel(), np.array([0.2, 2.0], np.float32)]))
+    return m
+
+
+class Scene:
+    def __init__(self, ctx, dims, dtype):
+        from voreen_amd import hipdvr as H, workloads as W
+        self.ctx, self.H, self.W, self.dims = ctx, H, W, dims
+        vol = W.make_volume("c1", dims=dims)
+        self.vol = ctx.volume((vol >> 8).astype(np.uint8) if dtype == np.uint8 else vol)
+        keys, _ = W.make_tf("c1")
+        self.tf = ctx.transfunc(H.tf_from_keys(keys, 4096))
+        self.net = network(H, ctx)
+        self.learned = H.Learned(ctx, self.vol)
+        self.opts = H.learned_opts(psnr_floor=1e-3)   # the judge accepts everything
+
+    def view(self, image, cap, shading):
+        w, h = image
+        de, dx, do = (self.ctx.alloc(w * h * 16) for _ in range(3))
+        llf, urb = self.W.world_box(self.dims)
+        cam = self.W.orbit_camera(5, 36, radius=2.1)
+        self.ctx.entry_exit_device(cam, llf, urb, w, h, de, dx)
+        p = self.H.default_params(self.W.step_for(self.dims, 2.0), shading=shading, camera_pos=tuple(cam.eye))
+        p.loop_cap = cap
+        return de, dx, do, p
+
+    def frame(self, bufs, image, batch):
+        de, dx, do, p = bufs
+        p.batch = batch
+        do.upload(np.full((image[1], image[0], 4), -1.0, np.float32))
+        st = self.learned.render_device(self.tf, de, dx, image[0], image[1], p, do, opts=self.opts, stats=True)
+        assert not st["fell_back"]
+        return do.download((image[1], image[0], 4), np.float32)
+
+    def close(self):
+        for o in (self.learned, self.net, self.vol, self.tf):
+            o.close()
+
+
+@pytest.mark.parametrize("dims,dtype,image", [((96, 80, 72), np.uint16, (90, 70)), ((130, 65, 33), np.uint8, (64, 129))],
+                         ids=["u16", "u8"])
+@pytest.mark.parametrize("shading", [0, 1])
+def test_samples_do_not_depend_on_the_lanes(ctx, dims, dtype, image, shading):
+    s = Scene(ctx, dims, dtype)
+    H = s.H
+    try:
+        for cap in (0, 1, 2, 3, 5, 6, 37, 150):
+            print(f"[case] learned lanes {dims} {image} shading {shading} cap {cap}", flush=True)
+            bufs = s.view(image, cap, shading)
+            de, dx, do, p = bufs
+            s.learned.prepare(s.tf, p, s.net, opts=s.opts)
+            two, four = s.frame(bufs, image, 2), s.frame(bufs, image, 4)
+            b = H.Batch(ctx, [(s.vol, s.tf, de, dx, do, image[0], image[1], p)])
+            try:
+                b.set_learned([s.learned], s.opts)
+                for tile in (0, 1, 2):
+                    b.set_config(tile, 4, 2)
+                    do.upload(np.full((image[1], image[0], 4), -1.0, np.float32))
+                    b.launch_learned(stats=True)
+                    one = do.download((image[1], image[0], 4), np.float32)
+                    assert np.array_equal(two, one), f"cap {cap} tile {tile}: 2 lanes"
+                    assert np.array_equal(four, one), f"cap {cap} tile {tile}: 4 lanes"
+                assert cap or np.mean(one[..., 3] > 0) > 0.1
+            finally:
+                b.close()
+            for x in (de, dx, do):
+                x.free()
+    finally:
+        s.close()

@@ -92,9 +92,10 @@ __device__ __forceinline__ float4 learned_ray(const LearnedArgs& la, const CellF
                                               float4 e, float4 l, unsigned long long& n_samples,
                                               unsigned long long& n_shaded) {
     typedef typename CellFetch<T, WIDE>::rec_t rec_t;
-    // the brick is looked up from the position after every KS samples (and
-    // past its exit); position and exit parameter may disagree by a rounding
-    // at a face, so the samples depend on KS, but not on P
+    // the brick is looked up from the position, and the cap asked, after every
+    // KS samples (and past the brick's exit); position and exit parameter may
+    // disagree by a rounding at a face, so the samples depend on KS, but not on
+    // P
     constexpr int KS = PHONG ? 2 : 4;
     const MarchArgs& a = la.m;
     const float first[3] = {e.x, e.y, e.z}, last[3] = {l.x, l.y, l.z};
@@ -115,7 +116,7 @@ __device__ __forceinline__ float4 learned_ray(const LearnedArgs& la, const CellF
             bc[i] = (uint32_t)tex_to_voxel(first[i] + at * dir[i], a.fdims[i], a.fdm1[i]) >> kLBrickLog2;
         return (bc[2] * la.nb16[1] + bc[1]) * la.nb16[0] + bc[0];
     };
-    while (A < kErtOpacity && !(t > tend) && guard < a.loop_cap) {
+    while (A < kErtOpacity && !(t > tend) && (guard < a.loop_cap || (P < KS && phase != 0 && t < t_exit))) {
         if (phase == 0 || !(t < t_exit)) {
             phase = 0;
             uint32_t bc[3];
@@ -147,7 +148,7 @@ __device__ __forceinline__ float4 learned_ray(const LearnedArgs& la, const CellF
             bool valid = (k == 0) || (taken == k && !(tt > tend) && tt < t_exit);
             if (k > 0 && k % KS == 0 && valid) {
                 uint32_t bc[3];
-                valid = brick_at(tt, bc) == cur;
+                valid = guard + k < a.loop_cap && brick_at(tt, bc) == cur;
             }
             if (valid) {
                 int m = mmax;
