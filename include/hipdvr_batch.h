@@ -85,7 +85,7 @@ int hipdvr_batch_set_learned(hipdvr_batch* b, hipdvr_learned* const* learned, ui
 /* One batched launch with learned stepping: one launch marches
  * the judges' plain re-march of every learned view's sparse pixels (each ray
  * whole, so the sparse images equal the plain frames at those pixels
- * exactly) and the learned and plain jobs; then the judges of all learned
+ * exactly) and the plain jobs, another the learned jobs; then the judges of all learned
  * views run in one launch, and per learned view the plain frame, which runs
  * only when its view fell below the PSNR floor (the steps of
  * hipdvr_render_learned_device, for all views of the batch at once).  Asynchronous unless stats != NULL:

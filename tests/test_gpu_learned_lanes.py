@@ -1,6 +1,8 @@
-"""The learned march with 2 and 4 lanes per ray: its samples do not depend on
-the number of lanes, whatever the loop cap, so a frame of 2 lanes, one of 4 and
-the batched launch give the same image bit for bit."""
+"""The learned march with 1, 2 and 4 lanes per ray: its samples do not depend
+on the number of lanes, whatever the loop cap, so a frame of 2 lanes, one of 4
+and the batched launch (one lane, several samples in flight) give the same
+image bit for bit, and a frame large enough for one lane the image that 2 lanes
+give."""
 import numpy as np
 import pytest
 
@@ -83,5 +85,19 @@ def test_samples_do_not_depend_on_the_lanes(ctx, dims, dtype, image, shading):
                 b.close()
             for x in (de, dx, do):
                 x.free()
+    finally:
+        s.close()
+
+
+@pytest.mark.parametrize("shading,image", [(0, (1001, 819)), (1, (1331, 997))])
+def test_large_frame_equals_two_lanes(ctx, shading, image):
+    s = Scene(ctx, (64, 72, 80), np.uint16)
+    try:
+        print(f"[case] learned one lane {image} shading {shading}", flush=True)
+        bufs = s.view(image, 0, shading)
+        s.learned.prepare(s.tf, bufs[3], s.net, opts=s.opts)
+        assert np.array_equal(s.frame(bufs, image, 0), s.frame(bufs, image, 2))
+        for x in bufs[:3]:
+            x.free()
     finally:
         s.close()

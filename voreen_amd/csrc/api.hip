@@ -135,19 +135,14 @@ void ensure_occupancy(hipdvr_ctx* ctx, hipdvr_volume* vol, const hipdvr_tf* tf) 
     std::memcpy(vol->occ_key, key.k, sizeof key.k);
 }
 
-namespace {
-
-// Whether a graph is being captured from the context's stream.
-bool capturing(const hipdvr_ctx* ctx) {
+bool ctx_capturing(const hipdvr_ctx* ctx) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(ctx->stream, &cs) == hipSuccess) return cs != hipStreamCaptureStatusNone;
     (void)hipGetLastError();   // not left for the next call
     return false;
 }
 
-// Orders the context's stream (or, while that is captured, the caller) after
-// what the context submitted to `other` before it left it.
-void wait_left(hipdvr_ctx* ctx, hipStream_t other, bool on_host) {
+void ctx_wait_left(hipdvr_ctx* ctx, hipStream_t other, bool on_host) {
     for (const hipdvr_ctx::Left& l : ctx->left) {
         if (l.stream != other) continue;
         if (!on_host) {
@@ -162,6 +157,8 @@ void wait_left(hipdvr_ctx* ctx, hipStream_t other, bool on_host) {
         return;
     }
 }
+
+namespace {
 
 // The context leaves its stream: an event behind what it submitted there.
 // Never fails: without an event, the device is waited for.
@@ -200,11 +197,11 @@ const uint8_t* ensure_skip(hipdvr_ctx* ctx, hipdvr_volume* vol, const hipdvr_tf*
     if (rule == kSkipPairs) k[0] = tf->preint_serial;
     k[4] = ((uint64_t)rule << 32) | (rule == kSkipIso ? fbits(iso) : 0);
     const hipStream_t st = ctx->stream;
-    const bool in_capture = capturing(ctx);
+    const bool in_capture = ctx_capturing(ctx);
     for (SkipGrid& g : vol->skips) {
         if (g.in_graph || std::memcmp(k, g.key, sizeof k) != 0) continue;
         if (std::find(g.streams.begin(), g.streams.end(), st) == g.streams.end()) {
-            wait_left(ctx, g.streams.front(), in_capture);
+            ctx_wait_left(ctx, g.streams.front(), in_capture);
             g.streams.push_back(st);
         }
         g.captured = g.captured || in_capture;
@@ -216,7 +213,7 @@ const uint8_t* ensure_skip(hipdvr_ctx* ctx, hipdvr_volume* vol, const hipdvr_tf*
     if (!g) g = &add_skip_grid(vol, rule);
     // after the frames that still read it
     for (const hipStream_t s : g->streams)
-        if (s != st) wait_left(ctx, s, false);
+        if (s != st) ctx_wait_left(ctx, s, false);
     std::memset(g->key, 0, sizeof g->key);
     g->streams.assign(1, st);
     g->captured = g->in_graph = in_capture;
@@ -418,7 +415,7 @@ void render_device_impl(hipdvr_ctx* ctx, const hipdvr_volume* vol, const hipdvr_
                       p->filter == HIPDVR_FILTER_LINEAR && p->classification != HIPDVR_CLASS_TF2D &&
                       (modes || p->classification == HIPDVR_CLASS_PREINT) && cells_allowed(vol);
     if (cell_modes) {
-        cell_modes = !capturing(ctx) && try_cells(mvol, ctx->stream);
+        cell_modes = !ctx_capturing(ctx) && try_cells(mvol, ctx->stream);
     }
     const bool cell = kernel == HIPDVR_KERNEL_CELL;
     const bool slab = kernel == HIPDVR_KERNEL_SLAB;

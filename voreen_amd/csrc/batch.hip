@@ -20,11 +20,11 @@
 
 #include "../../include/hipdvr_batch.h"
 #include "../../include/hipdvr_learned.h"
+#include "batch_tiles.h"
 #include "ctx.h"
 #include "errors.h"
 #include "kernels.h"
 #include "learned.h"
-#include "learned_ray.h"
 #include "march_cell.h"
 #include "objects.h"
 #include "volume.h"
@@ -37,10 +37,6 @@ constexpr int kTileShapes = 3;
 constexpr size_t kCuLds = 160 * 1024, kWorkgroupLds = 64 * 1024;
 constexpr size_t kMarchStaticLds = sizeof(uint32_t) * kMaxTfWidth + sizeof(float) * 256;
 constexpr int kBrickSizes = 3;   // brick_log2 3, 4, 5
-
-// Pixels per wavefront: 8x8, 16x4, 32x2; a workgroup is 2x2 wavefronts.
-__host__ __device__ constexpr int wave_w(int tile) { return 8 << tile; }
-__host__ __device__ constexpr int wave_h(int tile) { return 64 / wave_w(tile); }
 
 // The order of the tiles.  The hardware hands consecutive workgroups to the
 // 8 XCDs in turn (workgroup b to XCD b % 8), and each XCD has its own L2.
@@ -71,55 +67,28 @@ inline uint64_t batch_grid(uint32_t total, int parts) {
     return (chunks + kXcds - 1) / kXcds * kXcds * kChunk * (uint64_t)parts;
 }
 
-// Tile (tx, ty) at position lt of a job of tiles_x x tiles_y tiles in block
-// order (a bijection of [0, tiles_x * tiles_y)).
-__device__ __forceinline__ void block_tile(uint32_t lt, uint32_t tiles_x, uint32_t tiles_y, uint32_t& tx,
-                                           uint32_t& ty) {
-    const uint32_t nby = (tiles_y + kBlockH - 1) / kBlockH, nbx = (tiles_x + kBlockW - 1) / kBlockW;
-    uint32_t by = lt / (kBlockH * tiles_x);
-    if (by > nby - 1) by = nby - 1;
-    const uint32_t r = lt - by * kBlockH * tiles_x;
-    const uint32_t bh = min((uint32_t)kBlockH, tiles_y - by * kBlockH);
-    uint32_t bx = r / (kBlockW * bh);
-    if (bx > nbx - 1) bx = nbx - 1;
-    const uint32_t r2 = r - bx * kBlockW * bh;
-    const uint32_t bw = min((uint32_t)kBlockW, tiles_x - bx * kBlockW);
-    ty = by * kBlockH + r2 / bw;
-    tx = bx * kBlockW + r2 % bw;
-}
-
 // One workgroup per P-th of a tile, P lanes per ray (march_cell.h).  The
 // tile's 2x2 regions of 64 pixels fall into parts of 64 / P rays; wavefront w
 // marches part `part` of region w, or, where the parts of a region are
 // narrower than it, its neighbours in the same part of the tile.
-// Wavefronts per SIMD of the learned launch: 36 views of 512^3 at 1024^2, 4 /
-// 5 / 6: 17.6 / 15.4 / 20.0 ms (six spill).
-template <bool WIDE, int SHADE, bool COUNT, int P, bool LEARNED>
-__global__ __launch_bounds__(256, SHADE == 2 ? 4 : (SHADE == 1 ? (LEARNED || COUNT ? 5 : 6) : (COUNT ? 6 : 7))) void batch_kernel(
-    const LearnedArgs* __restrict__ jobs, const uint32_t* __restrict__ tile_start, uint32_t njobs,
+template <bool WIDE, int SHADE, bool COUNT, int P>
+__global__ __launch_bounds__(256, SHADE == 2 ? 4 : (SHADE == 1 ? (COUNT ? 5 : 6) : (COUNT ? 6 : 7))) void batch_kernel(
+    const MarchArgs* __restrict__ jobs, const uint32_t* __restrict__ tile_start, uint32_t njobs,
     uint32_t total_tiles, unsigned long long* __restrict__ counters, uint32_t tile_shape) {
     const uint32_t block = linear_block(), slot = block / kXcds, part = slot % P, i = slot / P;
     const uint32_t tile = xcd_run(block % kXcds, i / kChunk) * kChunk + i % kChunk;
     if (tile >= total_tiles) return;
     __shared__ uint32_t s_tf[kMaxTfWidth];
     __shared__ float s_alpha[256];
-    // job of this tile: last j with tile_start[j] <= tile
-    uint32_t lo = 0, hi = njobs;
-    while (hi - lo > 1) {
-        const uint32_t mid = (lo + hi) >> 1;
-        if (tile_start[mid] <= tile) lo = mid;
-        else hi = mid;
-    }
-    const uint32_t job = __builtin_amdgcn_readfirstlane(lo);
-    const LearnedArgs& la = jobs[job];
-    const MarchArgs& a = la.m;
+    const uint32_t job = job_of_tile(tile_start, njobs, tile);
+    const MarchArgs& a = jobs[job];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, ray = lane / P, sub = lane % P;
     // a region and its parts, all powers of two
     const int WW = 8 << tile_shape, WH = 8 >> tile_shape;
     const int RH = ray_h<P>() < WH ? ray_h<P>() : WH, RW = 64 / P / RH, cols = WW / RW;
     uint32_t tx, ty;
-    block_tile(tile - tile_start[job], (uint32_t)(a.grid_w + 2 * WW - 1) / (2 * WW),
-               (uint32_t)(a.grid_h + 2 * WH - 1) / (2 * WH), tx, ty);
+    block_tile<kBlockW, kBlockH>(tile - tile_start[job], (uint32_t)(a.grid_w + 2 * WW - 1) / (2 * WW),
+                                 (uint32_t)(a.grid_h + 2 * WH - 1) / (2 * WH), tx, ty);
     // a job marches the pixels of its grid: the whole image, or (a judge's
     // re-march: pix_block > 1) the sparse pixels judge_pixel places, written
     // to out[gy * grid_w + gx]; their samples are not counted (the learned
@@ -141,28 +110,13 @@ __global__ __launch_bounds__(256, SHADE == 2 ? 4 : (SHADE == 1 ? (LEARNED || COU
     const bool hit = !is_background(e, l);
     RayCounters n;
     if (__syncthreads_or(hit)) {   // a workgroup of background pixels needs no tables
-        // a job with a stepping table marches with learned stepping
-        const bool learned = LEARNED && la.table != nullptr;
         for (int k = tid; k < a.tf_width; k += 256) s_tf[k] = a.tf[k];
-        s_alpha[tid] = learned ? la.alpha_m[tid] : a.alpha_corr[tid];
+        s_alpha[tid] = a.alpha_corr[tid];
         __syncthreads();
         if (hit) {
             // WIDE: 64-bit record addressing for every job (a volume's
             // records exceed 4 GiB); else 32-bit buffer offsets
-            if (LEARNED && learned) {
-                unsigned long long ns = 0, nsh = 0;
-                if (a.dtype == 0) {
-                    const CellFetch<uint8_t, WIDE> f = cell_fetch_of<uint8_t, WIDE>(a);
-                    res = learned_ray<uint8_t, WIDE, SHADE != 0, P>(la, f, s_tf, s_alpha, px, py, sub, e, l, ns, nsh);
-                } else {
-                    const CellFetch<uint16_t, WIDE> f = cell_fetch_of<uint16_t, WIDE>(a);
-                    res = learned_ray<uint16_t, WIDE, SHADE != 0, P>(la, f, s_tf, s_alpha, px, py, sub, e, l, ns,
-                                                                     nsh);
-                }
-                ++n.rays;
-                n.fetched += sub == 0 ? (uint32_t)ns : 0;   // the ray's, counted by one lane
-                n.shaded += sub == 0 ? (uint32_t)nsh : 0;
-            } else if (a.dtype == 0) {
+            if (a.dtype == 0) {
                 const CellFetch<uint8_t, WIDE> f = cell_fetch_of<uint8_t, WIDE>(a);
                 res = cell_ray<uint8_t, WIDE, SHADE, COUNT, P>(a, f, s_tf, s_alpha, px, py, sub, e, l, n);
             } else {
@@ -176,23 +130,20 @@ __global__ __launch_bounds__(256, SHADE == 2 ? 4 : (SHADE == 1 ? (LEARNED || COU
     if (COUNT) add_counters<P>(counters, n, sub == 0);
 }
 
-typedef void (*BatchKernel)(const LearnedArgs*, const uint32_t*, uint32_t, uint32_t, unsigned long long*,
-                            uint32_t);
+typedef void (*BatchKernel)(const MarchArgs*, const uint32_t*, uint32_t, uint32_t, unsigned long long*, uint32_t);
 
 template <bool WIDE, int SHADE, bool COUNT>
-BatchKernel pick_kernel(int lanes, bool learned) {
-    if constexpr (SHADE < 2)   // no learned job shades exactly
-        if (learned) return lanes == 2 ? batch_kernel<WIDE, SHADE, COUNT, 2, true> : batch_kernel<WIDE, SHADE, COUNT, 4, true>;
-    if (lanes == 2) return batch_kernel<WIDE, SHADE, COUNT, 2, false>;
-    if (lanes == 4) return batch_kernel<WIDE, SHADE, COUNT, 4, false>;
-    return batch_kernel<WIDE, SHADE, COUNT, 16, false>;
+BatchKernel pick_kernel(int lanes) {
+    if (lanes == 2) return batch_kernel<WIDE, SHADE, COUNT, 2>;
+    if (lanes == 4) return batch_kernel<WIDE, SHADE, COUNT, 4>;
+    return batch_kernel<WIDE, SHADE, COUNT, 16>;
 }
 
 template <bool WIDE>
-BatchKernel kernel_for_w(int shade, bool count, int lanes, bool learned) {
-    if (shade == 2) return count ? pick_kernel<WIDE, 2, true>(lanes, learned) : pick_kernel<WIDE, 2, false>(lanes, learned);
-    if (shade == 1) return count ? pick_kernel<WIDE, 1, true>(lanes, learned) : pick_kernel<WIDE, 1, false>(lanes, learned);
-    return count ? pick_kernel<WIDE, 0, true>(lanes, learned) : pick_kernel<WIDE, 0, false>(lanes, learned);
+BatchKernel kernel_for_w(int shade, bool count, int lanes) {
+    if (shade == 2) return count ? pick_kernel<WIDE, 2, true>(lanes) : pick_kernel<WIDE, 2, false>(lanes);
+    if (shade == 1) return count ? pick_kernel<WIDE, 1, true>(lanes) : pick_kernel<WIDE, 1, false>(lanes);
+    return count ? pick_kernel<WIDE, 0, true>(lanes) : pick_kernel<WIDE, 0, false>(lanes);
 }
 
 // Lanes per ray of a launch of `pixels` pixels whose finest step is `step`,
@@ -200,14 +151,14 @@ BatchKernel kernel_for_w(int shade, bool count, int lanes, bool learned) {
 // of many jobs fills the chip.  Start of the lines, 2 / 4 lanes in us: two
 // views of 390 K pixels 916 / 488, eleven of 5.7 M 1822 / 1772, 64 volumes of
 // 16.8 M unshaded 682 / 876, 12 views of 12.6 M with Phong 5995 / 7116.
-int batch_lanes(int batch, uint64_t pixels, float step, bool learned) {
-    if (!learned && (double)pixels * step <= 100.0) return 16;
+int batch_lanes(int batch, uint64_t pixels, float step) {
+    if ((double)pixels * step <= 100.0) return 16;
     if (pixels <= 1500000) return 4;
     return pixels > 6000000 ? 2 : batch;
 }
 
-BatchKernel kernel_for(bool wide, int shade, bool count, int lanes, bool learned) {
-    return wide ? kernel_for_w<true>(shade, count, lanes, learned) : kernel_for_w<false>(shade, count, lanes, learned);
+BatchKernel kernel_for(bool wide, int shade, bool count, int lanes) {
+    return wide ? kernel_for_w<true>(shade, count, lanes) : kernel_for_w<false>(shade, count, lanes);
 }
 
 }  // namespace
@@ -216,6 +167,21 @@ BatchKernel kernel_for(bool wide, int shade, bool count, int lanes, bool learned
 
 using namespace hipdvr;
 
+namespace {
+
+// Jobs of one plain launch: their arguments per brick size, their tiles per
+// tile shape.
+struct BatchList {
+    MarchArgs* d_args[kBrickSizes] = {};
+    uint32_t* d_tile_start[kTileShapes] = {};
+    uint32_t total_tiles[kTileShapes] = {};
+    uint32_t n = 0;
+    uint64_t pixels = 0;
+    float step = 0.f;   // the finest
+};
+
+}  // namespace
+
 struct hipdvr_batch {
     hipdvr_ctx* ctx = nullptr;
     std::vector<hipdvr_batch_job> jobs;    // in launch order (largest first)
@@ -223,13 +189,9 @@ struct hipdvr_batch {
     int shade = 0;                         // 0 none, 1 Phong, 2 exact Phong
     bool wide = false;                     // some volume's cell records exceed 4 GiB
     // per brick size: device brick tables per job and the jobs' arguments
-    // (march arguments, plus the stepping table of learned jobs)
     std::vector<void*> allocations;
-    std::vector<LearnedArgs> h_args[kBrickSizes];
-    LearnedArgs* d_args[kBrickSizes] = {nullptr, nullptr, nullptr};
-    // the same with the stepping tables of the learned jobs
-    // (hipdvr_batch_launch_learned; hipdvr_batch_launch stays plain)
-    LearnedArgs* d_largs[kBrickSizes] = {nullptr, nullptr, nullptr};
+    std::vector<MarchArgs> h_args[kBrickSizes];
+    BatchList plain;
     // learned jobs (hipdvr_batch_set_learned), per launch position: the judge's
     // grid, sparse image, sum and flag
     std::vector<hipdvr_learned*> learned;
@@ -239,16 +201,18 @@ struct hipdvr_batch {
     std::vector<float4*> d_sparse;
     std::vector<float*> d_sse;
     std::vector<int*> d_flag;
-    // the learned launch's job list: first each learned view's judge
-    // re-march (its sparse grid, marched plainly into its sparse image),
-    // then every job; its tile ranges per tile shape
-    uint32_t n_ljobs = 0;
+    // the learned launch's jobs (hipdvr_batch_launch_learned): those marched
+    // plainly (first each learned view's judge re-march, its sparse grid into
+    // its sparse image, then the plain jobs) and the learned ones
+    BatchList with_learned;
+    LearnedArgs* d_largs = nullptr;
+    uint32_t n_learned = 0;
     uint32_t* d_ltile_start[kTileShapes] = {};
     uint32_t ltotal_tiles[kTileShapes] = {};
+    uint32_t* d_queue = nullptr;
+    hipStream_t queue_stream = nullptr;   // of the last learned launch
     hipdvr::JudgeJob* d_judge = nullptr;
     uint32_t n_judge = 0;
-    uint32_t* d_tile_start[kTileShapes] = {};
-    uint32_t total_tiles[kTileShapes] = {};
     hipdvr_batch_config cfg{0, 4, 4, 0};
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
@@ -285,28 +249,74 @@ void validate_config(const hipdvr_batch_config& c) {
     if (c.resident < 0 || c.resident > 8) fail(HIPDVR_ERR_INVALID, "resident must be 0 (default) or 1..8");
 }
 
-void launch_batch(hipdvr_batch* b, bool count, bool learned = false) {
-    hipStream_t st = ctx_stream(b->ctx);
+void launch_list(hipdvr_batch* b, const BatchList& list, bool count, hipStream_t st) {
+    if (list.n == 0) return;
     const int t = b->cfg.tile, bs = b->cfg.brick_log2 - 3;
-    uint64_t pixels = 0;
-    float step = b->jobs[0].params.step;
-    for (const hipdvr_batch_job& j : b->jobs) {
-        pixels += (uint64_t)j.w * j.h;
-        step = std::min(step, j.params.step);
-    }
-    const int lanes = batch_lanes(b->cfg.batch, pixels, step, learned);
-    BatchKernel k = kernel_for(b->wide, b->shade, count, lanes, learned);
+    const int lanes = batch_lanes(b->cfg.batch, list.pixels, list.step);
+    BatchKernel k = kernel_for(b->wide, b->shade, count, lanes);
     // a residency limit: dynamic LDS up to a share of the CU's 160 KiB
     size_t pad = 0;
     if (b->cfg.resident > 0 && kCuLds / b->cfg.resident > kMarchStaticLds)
         pad = kCuLds / b->cfg.resident - kMarchStaticLds;
     if (pad > kWorkgroupLds - kMarchStaticLds) pad = kWorkgroupLds - kMarchStaticLds;
-    const uint32_t total = learned ? b->ltotal_tiles[t] : b->total_tiles[t];
-    hipLaunchKernelGGL(k, linear_grid(batch_grid(total, lanes)), dim3(256), pad, st,
-                       (const LearnedArgs*)(learned ? b->d_largs[bs] : b->d_args[bs]),
-                       (const uint32_t*)(learned ? b->d_ltile_start[t] : b->d_tile_start[t]),
-                       learned ? b->n_ljobs : (uint32_t)b->jobs.size(), total, b->ctx->d_counters, (uint32_t)t);
+    hipLaunchKernelGGL(k, linear_grid(batch_grid(list.total_tiles[t], lanes)), dim3(256), pad, st,
+                       (const MarchArgs*)list.d_args[bs], (const uint32_t*)list.d_tile_start[t], list.n,
+                       list.total_tiles[t], b->ctx->d_counters, (uint32_t)t);
     hip_check(hipGetLastError(), "batch launch");
+}
+
+void launch_batch(hipdvr_batch* b, bool count) { launch_list(b, b->plain, count, ctx_stream(b->ctx)); }
+
+// Tiles of the jobs' grids: start[k] of job k, start[n] in all.
+template <typename Job>
+std::vector<uint32_t> tile_starts(const std::vector<Job>& jobs, int t, const MarchArgs& (*args)(const Job&)) {
+    std::vector<uint32_t> start(jobs.size() + 1, 0);
+    const uint32_t tw = 2 * wave_w(t), th = 2 * wave_h(t);
+    for (size_t k = 0; k < jobs.size(); ++k) {
+        const MarchArgs& m = args(jobs[k]);
+        const uint64_t tiles = (uint64_t)((m.grid_w + tw - 1) / tw) * ((m.grid_h + th - 1) / th);
+        if (start[k] + tiles > kMaxTiles) fail(HIPDVR_ERR_UNSUPPORTED, "batch too large");
+        start[k + 1] = start[k] + (uint32_t)tiles;
+    }
+    return start;
+}
+const MarchArgs& plain_args(const MarchArgs& a) { return a; }
+const MarchArgs& learned_args(const LearnedArgs& a) { return a.m; }
+
+template <typename T>
+void upload(T* dst, const std::vector<T>& src, hipStream_t st) {
+    if (!src.empty())
+        hip_check(hipMemcpyAsync(dst, src.data(), src.size() * sizeof(T), hipMemcpyHostToDevice, st), "upload");
+}
+
+// A list's host side: what upload_list takes over.
+struct HostList {
+    std::vector<MarchArgs> args[kBrickSizes];
+    std::vector<uint32_t> start[kTileShapes];
+    void tiles() {
+        for (int t = 0; t < kTileShapes; ++t) start[t] = tile_starts(args[0], t, plain_args);
+    }
+};
+
+// Uploads a list into buffers of at least `capacity` jobs (asynchronous: the
+// caller waits before `h` goes).
+void upload_list(hipdvr_batch* b, BatchList& list, const HostList& h, size_t capacity, hipStream_t st) {
+    for (int bs = 0; bs < kBrickSizes; ++bs) {
+        if (!list.d_args[bs]) list.d_args[bs] = dev_alloc<MarchArgs>(b, capacity * sizeof(MarchArgs));
+        upload(list.d_args[bs], h.args[bs], st);
+    }
+    for (int t = 0; t < kTileShapes; ++t) {
+        if (!list.d_tile_start[t]) list.d_tile_start[t] = dev_alloc<uint32_t>(b, (capacity + 1) * 4);
+        upload(list.d_tile_start[t], h.start[t], st);
+        list.total_tiles[t] = h.start[t].back();
+    }
+    list.n = (uint32_t)h.args[0].size();
+    list.pixels = 0;
+    list.step = INFINITY;
+    for (const MarchArgs& m : h.args[0]) {
+        list.pixels += (uint64_t)m.grid_w * m.grid_h;
+        list.step = std::min(list.step, m.step);
+    }
 }
 
 }  // namespace
@@ -357,8 +367,8 @@ int hipdvr_batch_create(hipdvr_ctx* ctx, const hipdvr_batch_job* jobs, uint32_t 
                 b->wide = b->wide || j.volume->cells_wide;
             }
             for (int bs = 0; bs < kBrickSizes; ++bs) {
-                std::vector<LearnedArgs>& args = b->h_args[bs];
-                args.assign(n, LearnedArgs{});
+                std::vector<MarchArgs>& args = b->h_args[bs];
+                args.assign(n, MarchArgs{});
                 const uint32_t bl = (uint32_t)bs + 3;
                 for (uint32_t i = 0; i < n; ++i) {
                     const hipdvr_batch_job& j = b->jobs[i];
@@ -374,33 +384,19 @@ int hipdvr_batch_create(hipdvr_ctx* ctx, const hipdvr_batch_job* jobs, uint32_t 
                     uint8_t* skip = (uint8_t*)(mm + count);
                     launch_brick_minmax(v, bl, nb, mm, st);
                     launch_skip_grid(occupancy_args(v, j.tf, mm, count), nb, skip, skip + count, st);
-                    MarchArgs& a = args[i].m;
+                    MarchArgs& a = args[i];
                     fill_march_args(a, v, j.tf, &j.params, j.d_entry, j.d_exit, j.d_out, j.w, j.h, nullptr);
                     a.cells = v->d_cells;
                     a.skip = skip;
                     a.skip_log2 = bl;
                     for (int k = 0; k < 3; ++k) a.nskip[k] = nb[k];
                 }
-                b->d_args[bs] = dev_alloc<LearnedArgs>(b, n * sizeof(LearnedArgs));
-                hip_check(hipMemcpyAsync(b->d_args[bs], args.data(), n * sizeof(LearnedArgs), hipMemcpyHostToDevice,
-                                         st),
-                          "upload");
-                hip_check(hipStreamSynchronize(st), "hipStreamSynchronize");
             }
-            for (int t = 0; t < kTileShapes; ++t) {
-                std::vector<uint32_t> start(n + 1, 0);
-                const uint32_t tw = 2 * wave_w(t), th = 2 * wave_h(t);
-                for (uint32_t i = 0; i < n; ++i) {
-                    const uint64_t tiles = (uint64_t)((b->jobs[i].w + tw - 1) / tw) * ((b->jobs[i].h + th - 1) / th);
-                    if (start[i] + tiles > kMaxTiles) fail(HIPDVR_ERR_UNSUPPORTED, "batch too large");
-                    start[i + 1] = start[i] + (uint32_t)tiles;
-                }
-                b->total_tiles[t] = start[n];
-                b->d_tile_start[t] = dev_alloc<uint32_t>(b, (n + 1) * 4);
-                hip_check(hipMemcpyAsync(b->d_tile_start[t], start.data(), (n + 1) * 4, hipMemcpyHostToDevice, st),
-                          "upload");
-                hip_check(hipStreamSynchronize(st), "hipStreamSynchronize");
-            }
+            HostList list;
+            for (int bs = 0; bs < kBrickSizes; ++bs) list.args[bs] = b->h_args[bs];
+            list.tiles();
+            upload_list(b, b->plain, list, n, st);
+            hip_check(hipStreamSynchronize(st), "hipStreamSynchronize");
             b->learned.assign(n, nullptr);
             b->plain_learned.assign(n, 0);
             hip_check(hipGetLastError(), "batch setup");
@@ -560,9 +556,7 @@ int hipdvr_batch_set_learned(hipdvr_batch* b, hipdvr_learned* const* learned, ui
         std::vector<float4*> sparse(nj, nullptr);
         std::vector<float*> sse(nj, nullptr);
         std::vector<int*> flag(nj, nullptr);
-        bool any = false;
-        std::vector<LearnedArgs> largs[kBrickSizes];
-        for (int bs = 0; bs < kBrickSizes; ++bs) largs[bs] = b->h_args[bs];
+        std::vector<LearnedArgs> largs;
         for (size_t i = 0; i < nj; ++i) {
             hipdvr_learned* l = learned[b->order[i]];
             const hipdvr_batch_job& j = b->jobs[i];
@@ -583,10 +577,11 @@ int hipdvr_batch_set_learned(hipdvr_batch* b, hipdvr_learned* const* learned, ui
                 plain_lv[i] = 1;
                 continue;
             }
-            for (int bs = 0; bs < kBrickSizes; ++bs) learned_stepping_args(l, &j.params, largs[bs][i]);
+            largs.push_back(LearnedArgs{});
+            largs.back().m = b->h_args[0][i];
+            learned_stepping_args(l, &j.params, largs.back());
             lv[i] = l;
             grids[i] = learned_judge_grid(j.w, j.h, lopts);
-            any = true;
         }
         for (size_t i = 0; i < nj; ++i) {
             if (!lv[i]) continue;
@@ -603,8 +598,9 @@ int hipdvr_batch_set_learned(hipdvr_batch* b, hipdvr_learned* const* learned, ui
             flag[i] = dev_alloc<int>(b, 64);
         }
         // the learned launch's jobs: each learned view's judge re-march
-        // (plain, into its sparse image), then every job; and the judges
-        std::vector<LearnedArgs> ljobs[kBrickSizes];
+        // (plain, into its sparse image), the plain jobs, the learned ones; and
+        // the judges
+        HostList list;
         std::vector<JudgeJob> judges;
         const float mse_max = powf(10.f, -lopts.psnr_floor / 10.f);
         for (size_t i = 0; i < nj; ++i) {
@@ -612,18 +608,14 @@ int hipdvr_batch_set_learned(hipdvr_batch* b, hipdvr_learned* const* learned, ui
             const JudgeGrid& g = grids[i];
             const hipdvr_batch_job& j = b->jobs[i];
             for (int bs = 0; bs < kBrickSizes; ++bs) {
-                LearnedArgs sj;
-                std::memset(&sj, 0, sizeof(sj));
-                sj.m = b->h_args[bs][i].m;
-                sj.m.out = sparse[i];
-                sj.m.counters = nullptr;
-                sj.m.cond_flag = nullptr;
-                sj.m.grid_w = g.w;
-                sj.m.grid_h = g.h;
-                sj.m.stride = (int32_t)g.stride;
-                sj.m.pix_block = (int32_t)g.block;
-                sj.m.pix_offset = (int32_t)g.offs;
-                ljobs[bs].push_back(sj);
+                MarchArgs sj = b->h_args[bs][i];
+                sj.out = sparse[i];
+                sj.grid_w = g.w;
+                sj.grid_h = g.h;
+                sj.stride = (int32_t)g.stride;
+                sj.pix_block = (int32_t)g.block;
+                sj.pix_offset = (int32_t)g.offs;
+                list.args[bs].push_back(sj);
             }
             JudgeJob jj;
             jj.learned = (const float4*)j.d_out;
@@ -641,39 +633,25 @@ int hipdvr_batch_set_learned(hipdvr_batch* b, hipdvr_learned* const* learned, ui
             jj.mse_max = mse_max;
             judges.push_back(jj);
         }
-        for (int bs = 0; bs < kBrickSizes; ++bs) ljobs[bs].insert(ljobs[bs].end(), largs[bs].begin(), largs[bs].end());
-        const uint32_t nl = (uint32_t)ljobs[0].size();
+        for (int bs = 0; bs < kBrickSizes; ++bs)
+            for (size_t i = 0; i < nj; ++i)
+                if (!lv[i]) list.args[bs].push_back(b->h_args[bs][i]);
+        list.tiles();
         std::vector<uint32_t> lstart[kTileShapes];
-        for (int t = 0; t < kTileShapes; ++t) {
-            const uint32_t tw = 2 * wave_w(t), th = 2 * wave_h(t);
-            lstart[t].assign(nl + 1, 0);
-            for (uint32_t k = 0; k < nl; ++k) {
-                const MarchArgs& m = ljobs[0][k].m;
-                const uint64_t tiles = (uint64_t)((m.grid_w + tw - 1) / tw) * ((m.grid_h + th - 1) / th);
-                if (lstart[t][k] + tiles > kMaxTiles) fail(HIPDVR_ERR_UNSUPPORTED, "batch too large");
-                lstart[t][k + 1] = lstart[t][k] + (uint32_t)tiles;
-            }
-        }
-        // capacity: every job of the batch twice
-        for (int bs = 0; bs < kBrickSizes; ++bs)
-            if (!b->d_largs[bs]) b->d_largs[bs] = dev_alloc<LearnedArgs>(b, 2 * nj * sizeof(LearnedArgs));
+        for (int t = 0; t < kTileShapes; ++t) lstart[t] = tile_starts(largs, t, learned_args);
+        if (!b->d_largs) b->d_largs = dev_alloc<LearnedArgs>(b, nj * sizeof(LearnedArgs));
         for (int t = 0; t < kTileShapes; ++t)
-            if (!b->d_ltile_start[t]) b->d_ltile_start[t] = dev_alloc<uint32_t>(b, (2 * nj + 1) * 4);
+            if (!b->d_ltile_start[t]) b->d_ltile_start[t] = dev_alloc<uint32_t>(b, (nj + 1) * 4);
+        if (!b->d_queue) b->d_queue = dev_alloc<uint32_t>(b, kLearnedQueueBytes);
         if (!b->d_judge) b->d_judge = dev_alloc<JudgeJob>(b, nj * sizeof(JudgeJob));
-        for (int bs = 0; bs < kBrickSizes; ++bs)
-            hip_check(hipMemcpyAsync(b->d_largs[bs], ljobs[bs].data(), nl * sizeof(LearnedArgs), hipMemcpyHostToDevice,
-                                     st),
-                      "upload");
-        for (int t = 0; t < kTileShapes; ++t)
-            hip_check(hipMemcpyAsync(b->d_ltile_start[t], lstart[t].data(), (nl + 1) * 4, hipMemcpyHostToDevice, st),
-                      "upload");
-        if (!judges.empty())
-            hip_check(hipMemcpyAsync(b->d_judge, judges.data(), judges.size() * sizeof(JudgeJob), hipMemcpyHostToDevice,
-                                     st),
-                      "upload");
+        // every learned view gives a judge's job, the others themselves
+        upload_list(b, b->with_learned, list, nj, st);
+        upload(b->d_largs, largs, st);
+        for (int t = 0; t < kTileShapes; ++t) upload(b->d_ltile_start[t], lstart[t], st);
+        upload(b->d_judge, judges, st);
         hip_check(hipStreamSynchronize(st), "hipStreamSynchronize");
-        b->n_ljobs = nl;
-        for (int t = 0; t < kTileShapes; ++t) b->ltotal_tiles[t] = lstart[t][nl];
+        b->n_learned = (uint32_t)largs.size();
+        for (int t = 0; t < kTileShapes; ++t) b->ltotal_tiles[t] = lstart[t].back();
         b->n_judge = (uint32_t)judges.size();
         b->lopts = lopts;
         b->learned.swap(lv);
@@ -703,10 +681,20 @@ int hipdvr_batch_launch_learned(hipdvr_batch* b, hipdvr_learned_stats* stats) {
         const bool count = stats != nullptr;
         if (count) launch_zero_u64(b->ctx->d_counters, kNumCounters, st);
         const bool timed = ctx_timing_start(b->ctx);
-        if (!b->d_largs[0]) fail(HIPDVR_ERR_INVALID, "hipdvr_batch_set_learned has not been called");
+        if (!b->d_largs) fail(HIPDVR_ERR_INVALID, "hipdvr_batch_set_learned has not been called");
         // 1. the judges' plain re-marches of the learned views' sparse pixels
-        //    and every job, learned or plain, in one launch
-        launch_batch(b, count, true);
+        //    and the plain jobs in one launch, then the learned jobs in
+        //    another (side by side on two streams they took a twentieth
+        //    longer: the persistent grid no longer fills the chip evenly)
+        launch_list(b, b->with_learned, count, st);
+        if (any) {
+            // the queue's counters serve one launch at a time
+            if (b->queue_stream && b->queue_stream != st) ctx_wait_left(b->ctx, b->queue_stream, ctx_capturing(b->ctx));
+            b->queue_stream = st;
+            const int t = b->cfg.tile;
+            launch_learned_batch(b->d_largs, b->d_ltile_start[t], b->n_learned, b->ltotal_tiles[t], t, shade != 0,
+                                 b->wide, b->cfg.resident, b->d_queue, count ? b->ctx->d_counters : nullptr, st);
+        }
         if (any) {
             // 2. the judges of all learned views in one launch, then per
             //    learned view the plain frame, launched always, which runs
@@ -715,10 +703,10 @@ int hipdvr_batch_launch_learned(hipdvr_batch* b, hipdvr_learned_stats* stats) {
             for (size_t i = 0; i < nj; ++i) {
                 if (!b->learned[i]) continue;
                 const hipdvr_batch_job& j = b->jobs[i];
-                MarchArgs fb = b->h_args[bs][i].m;
+                MarchArgs fb = b->h_args[bs][i];
                 fb.counters = nullptr;
                 fb.cond_flag = b->d_flag[i];
-                launch_march_cell(fb, fb.dtype, shade, false, j.volume->cells_wide, 0, st);
+                launch_fallback(fb, fb.dtype, shade, j.volume->cells_wide, st);
             }
         }
         hip_check(hipGetLastError(), "batched learned launch");

@@ -385,6 +385,20 @@ void fill_learned_args(LearnedArgs& la, hipdvr_learned* l, const hipdvr_tf* tf, 
     la.alpha_m = l->d_alpha_m;
 }
 
+// Lanes per ray of a learned frame.  Fewer lanes sooner than the plain frame:
+// what all lanes of a ray do alike (the passes that skip bricks, the chain of
+// positions) is a larger part of the learned march.
+// 512^3 with a trained network, us per frame with 1 / 2 / 4 lanes, Phong:
+// 512^2 567 / 481 / 358, 600^2 533 / 415 / 397, 660^2 592 / 450 / 454, 724^2
+// 593 / 431 / 494, 1024^2 676 / 642 / 801, 1200^2 739 / 755 / 963, 1300^2 801
+// / 831 / 1098, 2048^2 1431 / 1663 / 2371; unshaded: 600^2 295 / 291 / 259,
+// 724^2 304 / 303 / 321, 1024^2 414 / 437 / 511, 2048^2 917 / 1119 / 1531.
+int learned_lanes(const hipdvr_params* p, uint64_t pixels) {
+    if (p->batch) return frame_lanes(p->batch, pixels, p->step);
+    if (pixels > (p->shading == HIPDVR_SHADE_NONE ? 800000u : 1300000u)) return 1;
+    return pixels > 430000 ? 2 : frame_lanes(0, pixels, p->step);
+}
+
 }  // namespace
 
 namespace hipdvr {
@@ -622,12 +636,7 @@ int hipdvr_render_learned_device(hipdvr_learned* l, const hipdvr_tf* tf, const f
         fill_learned_args(la, l, tf, prm, d_entry, d_exit, d_out, w, h);
         la.m.cells = vol->d_cells;
         la.m.skip = skip;
-        // Two lanes per ray sooner than the plain frame: the passes that skip
-        // bricks are taken by all lanes of a ray alike.  512^3, 1024^2 with a
-        // trained network, frames/s with 1 / 2 / 4 lanes: 1040 / 1543 / 1261.
-        const uint64_t pixels = (uint64_t)w * h;
-        const int lanes = prm->batch == 0 && pixels > 600000 ? 2 : frame_lanes(prm->batch, pixels, prm->step);
-        launch_learned(la, phong, count, vol->cells_wide, lanes, st);
+        launch_learned(la, phong, count, vol->cells_wide, learned_lanes(prm, (uint64_t)w * h), st);
         hip_check(hipStreamWaitEvent(st, l->join, 0), "hipStreamWaitEvent");
         // 3. judge: flag = PSNR below the floor
         const float mse_max = powf(10.f, -opts.psnr_floor / 10.f);
@@ -639,7 +648,7 @@ int hipdvr_render_learned_device(hipdvr_learned* l, const hipdvr_tf* tf, const f
         fill_march_args(fb, vol, tf, prm, d_entry, d_exit, d_out, w, h, nullptr);
         fb.skip = skip;
         fb.cond_flag = l->d_flag;
-        launch_march_cell(fb, vol->desc.dtype, shade, false, vol->cells_wide, 0, st);
+        launch_fallback(fb, vol->desc.dtype, shade, vol->cells_wide, st);
         hip_check(hipGetLastError(), "learned render launch");
         if (timed) ctx_timing_stop(l->ctx);
         if (count) {

@@ -8,6 +8,7 @@
 #include "kernels.h"
 #include "learned.h"
 #include "learned_ray.h"
+#include "residency.h"
 #include "march_cell.h"
 #include "march_common.h"
 
@@ -411,7 +412,7 @@ void launch_targets(const float* err, const unsigned int* visits, const float* f
 
 // Tiles and lanes as march_cell_kernel.
 template <typename T, bool WIDE, bool PHONG, bool COUNT, int P>
-__global__ __launch_bounds__(256, PHONG ? 5 : 6) void learned_kernel(const LearnedArgs la) {
+__global__ __launch_bounds__(256, P == 1 ? (PHONG ? 4 : 5) : (PHONG ? 5 : 6)) void learned_kernel(const LearnedArgs la) {
     const MarchArgs& a = la.m;
     const uint32_t tiles_x = (a.w + 15) / 16;
     const uint32_t tiles_y = (a.h + 15) / 16;
@@ -438,8 +439,12 @@ __global__ __launch_bounds__(256, PHONG ? 5 : 6) void learned_kernel(const Learn
         s_alpha[threadIdx.x] = la.alpha_m[threadIdx.x];
         __syncthreads();
         const CellFetch<T, WIDE> f = cell_fetch_of<T, WIDE>(a);
-        if (hit)
-            res = learned_ray<T, WIDE, PHONG, P>(la, f, s_tf, s_alpha, px, py, sub, e, l, n_samples, n_shaded);
+        if (hit) {
+            if constexpr (P == 1)
+                res = learned_ray_single<T, WIDE, PHONG>(la, f, s_tf, s_alpha, px, py, e, l, n_samples, n_shaded);
+            else
+                res = learned_ray<T, WIDE, PHONG, P>(la, f, s_tf, s_alpha, px, py, sub, e, l, n_samples, n_shaded);
+        }
     }
     if (inside && sub == 0) a.out[pix] = res;
     if (COUNT) {
@@ -448,6 +453,9 @@ __global__ __launch_bounds__(256, PHONG ? 5 : 6) void learned_kernel(const Learn
     }
 }
 
+// Static LDS of learned_kernel: the tables, and what __syncthreads_or takes.
+constexpr size_t kLearnedLds = sizeof(uint32_t) * kMaxTfWidth + sizeof(float) * 256 + 256;
+
 template <typename T, bool WIDE, int P>
 static void launch_learned_t(const LearnedArgs& la, bool phong, bool count, hipStream_t st) {
     const dim3 grid = linear_grid((uint64_t)xcd_tile_grid((la.m.w + 15) / 16, (la.m.h + 15) / 16) * P);
@@ -455,8 +463,13 @@ static void launch_learned_t(const LearnedArgs& la, bool phong, bool count, hipS
         if (count) hipLaunchKernelGGL((learned_kernel<T, WIDE, true, true, P>), grid, dim3(256), 0, st, la);
         else hipLaunchKernelGGL((learned_kernel<T, WIDE, true, false, P>), grid, dim3(256), 0, st, la);
     } else {
-        if (count) hipLaunchKernelGGL((learned_kernel<T, WIDE, false, true, P>), grid, dim3(256), 0, st, la);
-        else hipLaunchKernelGGL((learned_kernel<T, WIDE, false, false, P>), grid, dim3(256), 0, st, la);
+        // one lane per ray: five workgroups per CU.  With four / five / six /
+        // the seven that its registers allow, us per unshaded frame of 512^3:
+        // 1024^2 404 / 414 / 453 / 460, 1200^2 457 / 431 / 430 / 452, 2048^2
+        // 994 / 917 / 896 / 887
+        const size_t pad = P == 1 ? residency_pad(kLearnedLds, 5) : 0;
+        if (count) hipLaunchKernelGGL((learned_kernel<T, WIDE, false, true, P>), grid, dim3(256), pad, st, la);
+        else hipLaunchKernelGGL((learned_kernel<T, WIDE, false, false, P>), grid, dim3(256), pad, st, la);
     }
 }
 
@@ -472,7 +485,8 @@ static void launch_learned_p(const LearnedArgs& la, bool phong, bool count, bool
 }
 
 void launch_learned(const LearnedArgs& la, bool phong, bool count, bool wide, int lanes, hipStream_t st) {
-    if (lanes <= 2) launch_learned_p<2>(la, phong, count, wide, st);
+    if (lanes == 1) launch_learned_p<1>(la, phong, count, wide, st);
+    else if (lanes == 2) launch_learned_p<2>(la, phong, count, wide, st);
     else launch_learned_p<4>(la, phong, count, wide, st);
 }
 

@@ -83,6 +83,11 @@ __device__ __forceinline__ float alpha_for_multiple(float a1, int m) {
     return 1.0f - qm;
 }
 
+// Samples after which a ray's brick is looked up again: two when shaded, else
+// four.
+template <bool PHONG>
+constexpr int kLearnedFlight = PHONG ? 2 : 4;
+
 // One ray of the learned march from entry point e to exit point l (neither
 // the background), by P lanes (march_cell.h) of which this is lane `sub`:
 // returns the composited RGBA in each of them.
@@ -95,8 +100,8 @@ __device__ __forceinline__ float4 learned_ray(const LearnedArgs& la, const CellF
     // the brick is looked up from the position, and the cap asked, after every
     // KS samples (and past the brick's exit); position and exit parameter may
     // disagree by a rounding at a face, so the samples depend on KS, but not on
-    // P
-    constexpr int KS = PHONG ? 2 : 4;
+    // P; they are those of learned_ray_single
+    constexpr int KS = kLearnedFlight<PHONG>;
     const MarchArgs& a = la.m;
     const float first[3] = {e.x, e.y, e.z}, last[3] = {l.x, l.y, l.z};
     float dir[3];
@@ -225,6 +230,127 @@ __device__ __forceinline__ float4 learned_ray(const LearnedArgs& la, const CellF
         probe = A == A0;
         phase = P < KS && taken == P ? (phase + P) % KS : 0;
         t = tt;
+    }
+    return make_float4(r, g, bb, A);
+}
+
+// The same ray by one lane with K samples in flight.  Several lanes follow a
+// pass's chain of positions each; one lane computes it once.  So this is the
+// faster form where a launch has rays enough to fill the chip (batches, large
+// frames), and the other where the longest rays bound the frame (lines and
+// figures at learned_lanes and in batch_learned.hip).  All samples are
+// reconstructed: asking the exact skip grid costs a single lane as much as the
+// quarter of the samples that it would leave out.
+template <typename T, bool WIDE, bool PHONG>
+__device__ __forceinline__ float4 learned_ray_single(const LearnedArgs& la, const CellFetch<T, WIDE>& f,
+                                                     const uint32_t* s_tf, const float* s_alpha, int px, int py,
+                                                     float4 e, float4 l, unsigned long long& n_samples,
+                                                     unsigned long long& n_shaded) {
+    constexpr int K = kLearnedFlight<PHONG>;
+    typedef typename CellFetch<T, WIDE>::rec_t rec_t;
+    const MarchArgs& a = la.m;
+    const float first[3] = {e.x, e.y, e.z}, last[3] = {l.x, l.y, l.z};
+    float dir[3];
+    const float tend = ray_setup(first, last, a.step, dir);
+    const uint32_t oct = (dir[0] < 0.f ? 1u : 0u) | (dir[1] < 0.f ? 2u : 0u) | (dir[2] < 0.f ? 4u : 0u);
+    const BoxExit bx = box_exit_setup(a, dir);
+    float t = 0.f, r = 0.f, g = 0.f, bb = 0.f, A = 0.f;
+    int guard = 0;
+    bool finished = false;
+    uint32_t cur = 0xffffffffu;   // brick of the cached table entry
+    float t_exit = 0.f;
+    int mmax = 1;
+    bool skip = false;
+    while (!finished && !(t > tend) && guard < a.loop_cap) {
+        float s[3], vp[3];
+        for (int i = 0; i < 3; ++i) {
+            s[i] = first[i] + t * dir[i];
+            vp[i] = tex_to_voxel(s[i], a.fdims[i], a.fdm1[i]);
+        }
+        uint32_t bc[3];
+        for (int i = 0; i < 3; ++i) bc[i] = (uint32_t)vp[i] >> kLBrickLog2;
+        const uint32_t brick = (bc[2] * la.nb16[1] + bc[1]) * la.nb16[0] + bc[0];
+        if (brick != cur) {
+            cur = brick;
+            const uint8_t ent = la.table[brick * 8 + oct];
+            t_exit = kLearnedFastExit ? box_exit_fast(bx, first, dir, bc, kLBrick, la.nb16)
+                                      : box_exit(a, first, dir, bc, kLBrick, la.nb16);
+            skip = (ent & 0x80) != 0;
+            mmax = 1 << (ent & 3);
+        }
+        if (skip) {
+            // skip to the first step-grid point past the brick (a point that
+            // rounding leaves inside it is stepped on by the next pass)
+            const float k = floorf((t_exit - t) / a.step);
+            t = t + (fmaxf(k, 0.f) + 1.f) * a.step;
+            ++guard;
+            continue;
+        }
+        // up to K samples of this brick, their loads in flight together
+        float tk[K], pk[K][3];
+        int mk[K];
+        rec_t rk[K];
+        typename CellFetch<T, WIDE>::off_t ik[K];
+        bool valid[K];
+        float tt = t;
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            valid[k] = (k == 0) || (valid[k - 1] && !(tt > tend) && tt < t_exit);
+            tk[k] = tt;
+            int m = mmax;
+            if (m > 1 && tt + (float)m * a.step > t_exit) {
+                const float c = ceilf((t_exit - tt) / a.step);
+                m = c < 1.f ? 1 : (c < (float)m ? (int)c : m);
+            }
+            mk[k] = m;
+            if (valid[k]) {
+                const float sk[3] = {first[0] + tt * dir[0], first[1] + tt * dir[1], first[2] + tt * dir[2]};
+                ik[k] = cell_of<T, WIDE>(f, a, sk, pk[k]);
+                rk[k] = f.load(ik[k]);
+            }
+            tt = tt + (float)m * a.step;
+        }
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            if (!valid[k] || finished) break;
+            ++n_samples;
+            ++guard;
+            float v[8];
+            CellRecord<T>::unpack(rk[k], v);
+            const float inten = trilerp(v, pk[k]);
+            const uint32_t c8 = s_tf[tf_index(inten, a)];
+            const float ca = alpha_for_multiple(s_alpha[c8 >> 24], mk[k]);
+            if (ca > 0.f) {
+                float col[3] = {byte_norm(c8 & 0xffu), byte_norm((c8 >> 8) & 0xffu),
+                                byte_norm((c8 >> 16) & 0xffu)};
+                if (PHONG) {
+                    const float t0 = tk[k];
+                    const float ss[3] = {first[0] + t0 * dir[0], first[1] + t0 * dir[1],
+                                         first[2] + t0 * dir[2]};
+                    const float u[3] = {(a.fdims[0] * ss[0]) + (-0.5f), (a.fdims[1] * ss[1]) + (-0.5f),
+                                        (a.fdims[2] * ss[2]) + (-0.5f)};
+                    float gr[3];
+                    if (t0 == 0.0f) clip_border_gradient(a, px, py, ss, dir, gr);
+                    else if (!cell_gradient_interior<T, WIDE>(f, a, u, rk[k], ik[k], pk[k], gr))
+                        cell_gradient<T, WIDE, true>(f, a, ss, gr);
+                    float pos[3];
+                    for (int i = 0; i < 3; ++i)
+                        pos[i] = (((ss[i] * a.fdims[i]) - 0.5f) * a.spacing[i]) + a.offset[i];
+                    phong_fast(a, gr, pos, col);
+                    ++n_shaded;
+                }
+                const float w = (1.f - A) * ca;
+                r += w * col[0];
+                g += w * col[1];
+                bb += w * col[2];
+                A += w;
+            }
+            if (A >= kErtOpacity) {
+                A = 1.f;
+                finished = true;
+            }
+            t = tk[k] + (float)mk[k] * a.step;
+        }
     }
     return make_float4(r, g, bb, A);
 }

@@ -45,6 +45,11 @@ void ensure_occupancy(hipdvr_ctx* ctx, hipdvr_volume* vol, const hipdvr_tf* tf);
 // context's stream.
 const uint8_t* ensure_skip(hipdvr_ctx* ctx, hipdvr_volume* vol, const hipdvr_tf* tf, SkipRule rule = kSkipAlpha,
                            float iso = 0.0f);
+// Whether a graph is being captured from the context's stream.
+bool ctx_capturing(const hipdvr_ctx* ctx);
+// Orders the context's stream (on_host: the caller, for a stream that is being
+// captured) after what the context submitted to `other` before it left it.
+void ctx_wait_left(hipdvr_ctx* ctx, hipStream_t other, bool on_host);
 uint64_t next_serial();   // of objects and tables, never the same twice
 // Opacity-corrected 2D table for this step on the device (host powf, as
 // cpuraycaster.cpp:289 evaluates it per sample).
