@@ -27,6 +27,7 @@
 #include "learned.h"
 #include "march_cell.h"
 #include "objects.h"
+#include "residency.h"
 #include "volume.h"
 
 namespace hipdvr {
@@ -34,8 +35,6 @@ namespace hipdvr {
 namespace {
 
 constexpr int kTileShapes = 3;
-constexpr size_t kCuLds = 160 * 1024, kWorkgroupLds = 64 * 1024;
-constexpr size_t kMarchStaticLds = sizeof(uint32_t) * kMaxTfWidth + sizeof(float) * 256;
 constexpr int kBrickSizes = 3;   // brick_log2 3, 4, 5
 
 // The order of the tiles.  The hardware hands consecutive workgroups to the
@@ -254,11 +253,12 @@ void launch_list(hipdvr_batch* b, const BatchList& list, bool count, hipStream_t
     const int t = b->cfg.tile, bs = b->cfg.brick_log2 - 3;
     const int lanes = batch_lanes(b->cfg.batch, list.pixels, list.step);
     BatchKernel k = kernel_for(b->wide, b->shade, count, lanes);
-    // a residency limit: dynamic LDS up to a share of the CU's 160 KiB
     size_t pad = 0;
-    if (b->cfg.resident > 0 && kCuLds / b->cfg.resident > kMarchStaticLds)
-        pad = kCuLds / b->cfg.resident - kMarchStaticLds;
-    if (pad > kWorkgroupLds - kMarchStaticLds) pad = kWorkgroupLds - kMarchStaticLds;
+    if (b->cfg.resident > 0) {
+        hipFuncAttributes fa;
+        hip_check(hipFuncGetAttributes(&fa, (const void*)k), "hipFuncGetAttributes");
+        pad = residency_pad(fa.sharedSizeBytes, b->cfg.resident);
+    }
     hipLaunchKernelGGL(k, linear_grid(batch_grid(list.total_tiles[t], lanes)), dim3(256), pad, st,
                        (const MarchArgs*)list.d_args[bs], (const uint32_t*)list.d_tile_start[t], list.n,
                        list.total_tiles[t], b->ctx->d_counters, (uint32_t)t);
