@@ -44,8 +44,9 @@ typedef struct hipdvr_batch_config {
     int32_t tile;           /* HIPDVR_TILE_* */
     int32_t brick_log2;     /* empty-space bricks of 8^3, 16^3, 32^3: 3, 4, 5 */
     int32_t batch;          /* lanes of a wavefront that march a ray together, each one sample
-                               of a pass: 2 or 4 (launches below 1.5 M pixels take at least
-                               four, those above 6 M two) */
+                               of a pass: 2 or 4 for launches of middle size.  A launch of
+                               few rays takes at least four, one of many two, whatever is set
+                               (the lines: 1.5 M and 6 M pixels of the finest step's rays) */
     int32_t resident;       /* workgroups per CU at a time, 1..8 (at most what fits); 0: as many
                                as fit */
 } hipdvr_batch_config;

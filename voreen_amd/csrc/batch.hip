@@ -7,9 +7,9 @@
 // tile, which finds its job in the list's prefix sums and loads that job's TF
 // into LDS.  The hardware's dispatcher is the work queue: workgroups start in
 // list order as others end.  (A persistent grid that took tiles from counters
-// kept every job's arguments live across its loop and spilled 120 to 250
-// scalar registers into the march: 12 views of 512^3 with two lanes per ray
-// 7.1 ms against 6.0.)
+// kept every job's arguments live across its loop, at two to four times the
+// scalar registers that these kernels spill, and was slower: 12 views of 512^3
+// with two lanes per ray 7.1 ms against 6.0.)
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -69,7 +69,9 @@ inline uint64_t batch_grid(uint32_t total, int parts) {
 // One workgroup per P-th of a tile, P lanes per ray (march_cell.h).  The
 // tile's 2x2 regions of 64 pixels fall into parts of 64 / P rays; wavefront w
 // marches part `part` of region w, or, where the parts of a region are
-// narrower than it, its neighbours in the same part of the tile.
+// narrower than it, its neighbours in the same part of the tile.  Wavefronts
+// per SIMD, unshaded, 64 uneven volumes with two lanes, 6 / 7 / 8: 672 / 616 /
+// 608 us.
 template <bool WIDE, int SHADE, bool COUNT, int P>
 __global__ __launch_bounds__(256, SHADE == 2 ? 4 : (SHADE == 1 ? (COUNT ? 5 : 6) : (COUNT ? 6 : 7))) void batch_kernel(
     const MarchArgs* __restrict__ jobs, const uint32_t* __restrict__ tile_start, uint32_t njobs,
@@ -145,15 +147,22 @@ BatchKernel kernel_for_w(int shade, bool count, int lanes) {
     return count ? pick_kernel<WIDE, 0, true>(lanes) : pick_kernel<WIDE, 0, false>(lanes);
 }
 
-// Lanes per ray of a launch of `pixels` pixels whose finest step is `step`,
-// for the configuration's batch: as frame_lanes, with the lines where a launch
-// of many jobs fills the chip.  Start of the lines, 2 / 4 lanes in us: two
-// views of 390 K pixels 916 / 488, eleven of 5.7 M 1822 / 1772, 64 volumes of
-// 16.8 M unshaded 682 / 876, 12 views of 12.6 M with Phong 5995 / 7116.
-int batch_lanes(int batch, uint64_t pixels, float step) {
+// Lanes per ray of a launch of `pixels` pixels whose finest step is `step`, for
+// the configuration's batch.  `rays` are its pixels by the length of their
+// rays, in those of the longest (BatchList): what a launch with few of them
+// waits for is the chain of the longest rays, which more lanes shorten; a
+// launch of many issues all the time, and more lanes issue more.  2 / 4 lanes,
+// us: uneven volumes (64..384 an axis, unshaded) 8 of them (1.2 M rays) 349 /
+// 239, 16 (2.4 M) 436 / 312, 32 (4.9 M) 480 / 463, 48 (7.3 M) 555 / 670, 64
+// (9.8 M) 616 / 884; views of 512^3 at 1024^2 with Phong, 1 of them 1235 /
+// 1193, 2 2025 / 2011, 4 3626 / 3790, 6 5209 / 5550, 12 9914 / 10841; unshaded
+// 1 688 / 736, 4 1873 / 2244, 12 5032 / 6329.  So below the first line two
+// lanes are never much better, above the second never worse; in between the
+// configuration decides.
+int batch_lanes(int batch, uint64_t pixels, double rays, float step) {
     if ((double)pixels * step <= 100.0) return 16;
-    if (pixels <= 1500000) return 4;
-    return pixels > 6000000 ? 2 : batch;
+    if (rays <= 1.5e6) return 4;
+    return rays > 6.0e6 ? 2 : batch;
 }
 
 BatchKernel kernel_for(bool wide, int shade, bool count, int lanes) {
@@ -177,6 +186,7 @@ struct BatchList {
     uint32_t n = 0;
     uint64_t pixels = 0;
     float step = 0.f;   // the finest
+    double rays = 0.0;  // pixels, each counting as its step's share of the finest
 };
 
 }  // namespace
@@ -248,10 +258,12 @@ void validate_config(const hipdvr_batch_config& c) {
     if (c.resident < 0 || c.resident > 8) fail(HIPDVR_ERR_INVALID, "resident must be 0 (default) or 1..8");
 }
 
+int list_lanes(const BatchList& l, int batch) { return batch_lanes(batch, l.pixels, l.rays, l.step); }
+
 void launch_list(hipdvr_batch* b, const BatchList& list, bool count, hipStream_t st) {
     if (list.n == 0) return;
     const int t = b->cfg.tile, bs = b->cfg.brick_log2 - 3;
-    const int lanes = batch_lanes(b->cfg.batch, list.pixels, list.step);
+    const int lanes = list_lanes(list, b->cfg.batch);
     BatchKernel k = kernel_for(b->wide, b->shade, count, lanes);
     size_t pad = 0;
     if (b->cfg.resident > 0) {
@@ -317,6 +329,8 @@ void upload_list(hipdvr_batch* b, BatchList& list, const HostList& h, size_t cap
         list.pixels += (uint64_t)m.grid_w * m.grid_h;
         list.step = std::min(list.step, m.step);
     }
+    list.rays = 0.0;
+    for (const MarchArgs& m : h.args[0]) list.rays += (double)m.grid_w * m.grid_h * (list.step / m.step);
 }
 
 }  // namespace
@@ -396,6 +410,7 @@ int hipdvr_batch_create(hipdvr_ctx* ctx, const hipdvr_batch_job* jobs, uint32_t 
             for (int bs = 0; bs < kBrickSizes; ++bs) list.args[bs] = b->h_args[bs];
             list.tiles();
             upload_list(b, b->plain, list, n, st);
+            if (list_lanes(b->plain, b->cfg.batch) == 2) b->cfg.batch = 2;
             hip_check(hipStreamSynchronize(st), "hipStreamSynchronize");
             b->learned.assign(n, nullptr);
             b->plain_learned.assign(n, 0);
@@ -512,6 +527,9 @@ int hipdvr_batch_autotune(hipdvr_batch* b, uint32_t reps, hipdvr_batch_config* b
             for (int t = 0; t < 3; ++t)
                 for (int bl = 3; bl <= 5; ++bl)
                     for (int k : {2, 4}) {
+                        // (where the size decides, both are the same launch)
+                        const int lanes = list_lanes(b->plain, k);
+                        if (list_lanes(b->plain, 6 - k) == lanes && k != (lanes == 2 ? 2 : 4)) continue;
                         const float ms = time_config(hipdvr_batch_config{t, bl, k, 0});
                         if (ms < win_ms) {
                             win_ms = ms;
