@@ -243,8 +243,8 @@ __device__ __forceinline__ bool cell_gradient_interior(const CellFetch<T, WIDE>&
     return true;
 }
 
-// Counters of a lane (COUNT builds); a lane marches few enough samples for 32
-// bits, the sums over the launch have 64.  rays, skipped and the passes are the
+// Counters of a lane (COUNT builds); a lane marches at most 2^31 samples (the
+// loop cap), sums have 64 bits.  rays, skipped and the passes are the
 // ray's, alike in its P lanes; fetched and shaded are the lane's own samples.
 struct RayCounters {
     uint32_t rays = 0, skipped = 0, fetched = 0, shaded = 0, passes = 0, shade_passes = 0;
@@ -259,14 +259,15 @@ struct RayCounters {
 // 326 so (270 without counters).
 template <int P>
 __device__ __forceinline__ void add_counters(unsigned long long* c, const RayCounters& n, bool own) {
-    __shared__ uint32_t s_count[4][kNumCounters];
-    uint32_t v[kNumCounters] = {own ? n.rays : 0, (own ? n.skipped : 0) + n.fetched, n.fetched, n.shaded,
-                                n.passes * P + n.skipped, n.shade_passes * P};
+    typedef unsigned long long count_t;
+    __shared__ count_t s_count[4][kNumCounters];
+    count_t v[kNumCounters] = {own ? n.rays : 0, (count_t)(own ? n.skipped : 0) + n.fetched, n.fetched, n.shaded,
+                               (count_t)n.passes * P + n.skipped, (count_t)n.shade_passes * P};
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1)
 #pragma unroll
         for (int k = 0; k < kNumCounters; ++k) {
-            const uint32_t o = __shfl_xor(v[k], off, 64);
+            const count_t o = __shfl_xor(v[k], off, 64);
             v[k] = k < 4 ? v[k] + o : (o > v[k] ? o : v[k]);
         }
     if ((threadIdx.x & 63) == 0) {
@@ -275,7 +276,7 @@ __device__ __forceinline__ void add_counters(unsigned long long* c, const RayCou
     }
     __syncthreads();
     if (threadIdx.x < kNumCounters) {
-        unsigned long long sum = 0;
+        count_t sum = 0;
 #pragma unroll
         for (int w = 0; w < 4; ++w) sum += s_count[w][threadIdx.x];
         if (sum) atomicAdd(c + threadIdx.x, sum);
