@@ -347,6 +347,7 @@ void fill_march_args(MarchArgs& a, const hipdvr_volume* vol, const hipdvr_tf* tf
     a.tf2d_h = (int32_t)tf->h2d;
     for (int i = 0; i < 4; ++i) a.tf2d_dom[i] = tf->dom2d[i];
     fill_alpha_table(p->step, a.alpha_corr);
+    a.nan_empty = !tf->host_rgba.empty() && !(a.alpha_corr[tf->host_rgba[3]] > 0.0f) ? 1 : 0;
 }
 
 void ensure_tf2d(hipdvr_tf* tf, float step, hipStream_t st) {

@@ -178,7 +178,9 @@ __device__ __forceinline__ float4 learned_ray(const LearnedArgs& la, const CellF
             uint32_t b8[3];
             for (int i = 0; i < 3; ++i)
                 b8[i] = (uint32_t)tex_to_voxel(s[i], a.fdims[i], a.fdm1[i]) >> a.skip_log2;
-            mine = a.skip[cell_mul24(cell_mul24(b8[2], a.nskip[1]) + b8[1], a.nskip[0]) + b8[0]] == 0;
+            // (a degenerate ray's positions say nothing about its samples)
+            const float sum = (s[0] + s[1]) + s[2];
+            mine = sum != sum || a.skip[cell_mul24(cell_mul24(b8[2], a.nskip[1]) + b8[1], a.nskip[0]) + b8[0]] == 0;
         }
         if (mine) {
             float p[3];

@@ -445,7 +445,7 @@ __device__ __forceinline__ void cell_march(const MarchArgs& a, const CellFetch<T
             const uint32_t brick = cell_mul24(cell_mul24(b[2], a.nskip[1]) + b[1], a.nskip[0]) + b[0];
             if (brick != cur_brick) {
                 cur_brick = brick;
-                empty = a.skip[brick];
+                empty = nan_ray ? a.nan_empty : a.skip[brick];
                 if (empty) t_lim = empty_box_limit_rcp(a.nskip, first, rdir, rfd, b, bl, empty);
             }
             if (empty) {

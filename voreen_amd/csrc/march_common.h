@@ -41,6 +41,7 @@ struct MarchArgs {
     const uint8_t* skip;
     const uint2* skip_minmax;   // raw value range of every brick of the skip grid
     uint32_t skip_log2, nskip[3];
+    uint32_t nan_empty;         // 1: the TF entry of a sample that is not a number (the first) is invisible
     uint32_t dims[3];
     uint32_t nbricks[3];
     uint32_t brick_log2;
