@@ -126,7 +126,10 @@ void launch_brick_minmax(const hipdvr_volume* vol, uint32_t bl, const uint32_t n
 // Raw minimum and maximum voxel of the whole volume (synchronous).
 void volume_raw_minmax(const hipdvr_volume* vol, hipStream_t st, uint32_t out[2]);
 // Build the cell records if they are not there yet (synchronous).
-// try_cells: false, and no error, where there is no memory for them.
+// try_cells: for frames that do without them as well; false, and no error,
+// where they would take more than half of the free device memory (a frame must
+// not leave a program without room for what it allocates next), or an
+// allocation fails.
 bool try_cells(hipdvr_volume* vol, hipStream_t st);
 void ensure_cells(hipdvr_volume* vol, hipStream_t st);
 

@@ -588,10 +588,12 @@ uint64_t cell_record_bytes(const hipdvr_volume* v) {
 
 bool cells_allowed(const hipdvr_volume* v) { return cell_record_bytes(v) <= kMaxCellBytes; }
 
-bool try_cells(hipdvr_volume* v, hipStream_t st) {
-    if (v->d_cells) return true;
+namespace {
+
+// Builds the records; false, and nothing done, where the memory for them is
+// not there.
+bool build_cells(hipdvr_volume* v, hipStream_t st) {
     const uint64_t bytes = cell_record_bytes(v);
-    if (bytes > kMaxCellBytes) return false;
     const uint64_t total = bytes / (v->desc.dtype == HIPDVR_U8 ? 8 : 16);
     void* p = nullptr;
     const hipError_t e0 = hipMalloc(&p, bytes);
@@ -619,10 +621,19 @@ bool try_cells(hipdvr_volume* v, hipStream_t st) {
     return true;
 }
 
+}  // namespace
+
+bool try_cells(hipdvr_volume* v, hipStream_t st) {
+    if (v->d_cells) return true;
+    size_t free_bytes = 0, all = 0;
+    hip_check(hipMemGetInfo(&free_bytes, &all), "hipMemGetInfo");
+    return cells_allowed(v) && cell_record_bytes(v) <= free_bytes / 2 && build_cells(v, st);
+}
+
 void ensure_cells(hipdvr_volume* v, hipStream_t st) {
     if (v->d_cells) return;
     if (!cells_allowed(v)) fail(HIPDVR_ERR_UNSUPPORTED, "cell records of this volume exceed the size limit");
-    if (!try_cells(v, st)) hip_check(hipErrorOutOfMemory, "hipMalloc(cell records)");
+    if (!build_cells(v, st)) hip_check(hipErrorOutOfMemory, "hipMalloc(cell records)");
 }
 
 void volume_destroy(hipdvr_volume* v) {
