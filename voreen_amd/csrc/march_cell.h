@@ -283,7 +283,7 @@ __device__ __forceinline__ void add_counters(unsigned long long* c, const RayCou
     }
 }
 
-// Lanes per ray.  P neighbouring lanes of a wavefront (1, 2, 4, 8 or 16)
+// Lanes per ray.  P neighbouring lanes of a wavefront (2, 4 or 16)
 // march one ray together: in every pass lane `sub` of the ray fetches,
 // classifies and shades sample `sub` of the next P, and all P lanes then
 // composite the P results in order, so each lane holds the ray's state and
@@ -292,10 +292,10 @@ __device__ __forceinline__ void add_counters(unsigned long long* c, const RayCou
 // round trips and several hundred instructions per pass; P lanes cut it P
 // times, and neighbouring lanes read neighbouring samples, mostly of one
 // record group, in one load.  sub_value reads lane j's value (a move within
-// the VALU, no LDS).  What that gives is in kernels.h (frame_lanes); with six
-// wavefronts per SIMD, which one sample per lane leaves the registers for,
-// 512^3 / 1024^2 with Phong went from 1.04 ms (two samples in flight in one
-// lane, four wavefronts) to 0.68.
+// the VALU, no LDS).  What that gives is in kernels.h (frame_lanes).  One
+// sample per lane fits six wavefronts per SIMD but for 1 to 7 of the shaded
+// kernels' registers (10 in batches): 512^3 / 1024^2 with Phong went from 1.04
+// ms (two samples in flight in one lane, four wavefronts) to 0.68.
 template <int CTRL>
 __device__ __forceinline__ float dpp_move(float v) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
@@ -323,12 +323,10 @@ __device__ __forceinline__ float row_value(float v, int j) {
 }
 template <int P>
 __device__ __forceinline__ float sub_value(float v, int j) {
-    static_assert(P == 1 || P == 2 || P == 4 || P == 8 || P == 16, "lanes per ray");
-    if (P == 1) return v;
+    static_assert(P == 2 || P == 4 || P == 16, "lanes per ray");
     if (P == 2) return j == 0 ? dpp_move<0xA0>(v) : dpp_move<0xF5>(v);   // quad permutations
     if (P == 4) return j == 0 ? dpp_move<0x00>(v) : j == 1 ? dpp_move<0x55>(v) : j == 2 ? dpp_move<0xAA>(v)
                                                                                        : dpp_move<0xFF>(v);
-    if (P == 8) return (threadIdx.x & 8) ? row_value(v, j + 8) : row_value(v, j);
     return row_value(v, j);
 }
 template <int P>
@@ -358,7 +356,7 @@ __device__ __forceinline__ void count_pass(RayCounters& n, float ca, float A0, f
 
 // The place of a wavefront's rays in the image: 64 / P rays, ray_w<P>() wide.
 template <int P>
-__host__ __device__ constexpr int ray_w() { return P <= 2 ? 8 : (P <= 8 ? 4 : 2); }
+__host__ __device__ constexpr int ray_w() { return P <= 2 ? 8 : (P == 4 ? 4 : 2); }
 template <int P>
 __host__ __device__ constexpr int ray_h() { return 64 / P / ray_w<P>(); }
 
@@ -405,7 +403,6 @@ __device__ __forceinline__ void cell_march(const MarchArgs& a, const CellFetch<T
     uint32_t cur_brick = 0xffffffffu;
     uint32_t empty = 0;   // the skip grid's entry of the current brick
     float t_lim = 0.0f;
-    bool probe = true;
     // reciprocals for the empty-brick bound (a bound with a 0.05-voxel
     // margin needs no correctly rounded quotient); an axis with |dir| below
     // 1e-30 cannot move 0.05 voxel within a ray and bounds nothing
@@ -419,7 +416,7 @@ __device__ __forceinline__ void cell_march(const MarchArgs& a, const CellFetch<T
         rfd[i] = __builtin_amdgcn_rcpf(a.fdims[i]);
         nan_ray = nan_ray || !(fabsf(dir[i]) < INFINITY) || first[i] != first[i];
     }
-    bool finished = false;
+    bool probe = true, finished = false;
     while (!finished && loop < cap) {
         // this lane's sample and the next pass's first
         float tm = t, t_next = t;

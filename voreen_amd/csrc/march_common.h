@@ -491,30 +491,10 @@ __device__ __forceinline__ float empty_brick_limit(const MarchArgs& a, const flo
     return tl;
 }
 
-// empty_brick_limit from the reciprocals rdir = 1/dir (0: the axis bounds
+// The same for the box of bricks within d - 1 bricks (all empty) of brick b, on
+// a grid of nb bricks, from the reciprocals rdir = 1/dir (0: the axis bounds
 // nothing) and rfd = 1/fdims, each within a few ulp: the limit moves by far
-// less than the 0.05-voxel margin.
-__device__ __forceinline__ float empty_brick_limit_rcp(const MarchArgs& a, const float first[3],
-                                                       const float rdir[3], const float rfd[3],
-                                                       const float vp[3], uint32_t bl) {
-    float tl = INFINITY;
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-        const uint32_t b = (uint32_t)vp[i] >> bl;
-        const float B = (float)(1u << bl);
-        if (rdir[i] > 0.0f && b + 1 < a.nbricks[i]) {
-            const float vb = (float)(b + 1) * B - 0.05f;
-            tl = fminf(tl, ((vb + 0.5f) * rfd[i] - first[i]) * rdir[i]);
-        } else if (rdir[i] < 0.0f && b > 0) {
-            const float vb = (float)b * B + 0.05f;
-            tl = fminf(tl, ((vb + 0.5f) * rfd[i] - first[i]) * rdir[i]);
-        }
-    }
-    return tl;
-}
-
-// empty_brick_limit_rcp for the box of bricks within d - 1 bricks (all empty)
-// of brick b, on a grid of nb bricks; selects instead of branches, since the
+// less than the 0.05-voxel margin.  Selects instead of branches, since the
 // lanes of a wavefront face different ways.
 __device__ __forceinline__ float empty_box_limit_rcp(const uint32_t nb[3], const float first[3], const float rdir[3],
                                                      const float rfd[3], const uint32_t b[3], uint32_t bl,
@@ -534,16 +514,14 @@ __device__ __forceinline__ float empty_box_limit_rcp(const uint32_t nb[3], const
     return tl;
 }
 
-// 64-lane maximum of a per-lane counter, times `times` (the wavefront's rays),
-// added once per wavefront.
-__device__ __forceinline__ void wave_add_max64(unsigned long long* dst, unsigned long long v,
-                                               unsigned long long times = 64ull) {
+// 64-lane maximum of a per-lane counter, times 64, added once per wavefront.
+__device__ __forceinline__ void wave_add_max64(unsigned long long* dst, unsigned long long v) {
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) {
         const unsigned long long o = __shfl_xor(v, off, 64);
         v = o > v ? o : v;
     }
-    if ((threadIdx.x & 63) == 0 && v) atomicAdd(dst, times * v);
+    if ((threadIdx.x & 63) == 0 && v) atomicAdd(dst, 64ull * v);
 }
 
 // 64-lane sum of a per-lane counter; lane 0 adds it to the global counter.
