@@ -7,7 +7,6 @@
 // TF indexing and opacity correction, same ERT.  The TF (RGBA8, <= 4096
 // entries) and the 256-entry opacity-correction table sit in LDS.
 #include "march_common.h"
-#include "march_modes.h"
 #include "kernels.h"
 
 namespace hipdvr {
@@ -329,6 +328,18 @@ __global__ __launch_bounds__(256) void march_ref_kernel(const MarchArgs a) {
     }
 }
 
+// compositeMIDAhelper, mod_compositing.frag:112-129 (maxIntensity read only).
+__device__ __forceinline__ void mida_helper(float res[4], float voxel, const float col[4], float max_int,
+                                            float gamma) {
+    float delta = 0.0f;
+    if (voxel > max_int) delta = voxel - max_int;
+    const float beta = 1.0f - delta * (1.0f + gamma);
+    const float k = (1.0f - beta * res[3]) * col[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) res[i] = beta * res[i] + k * col[i];
+    res[3] = beta * res[3] + (1.0f - beta * res[3]) * col[3];
+}
+
 // Compositing modes other than DVR with TF classification: the GLSL
 // compositing functions (mod_compositing.frag:85-213) applied where the TF
 // alpha is > 0, after shading (rc_singlevolume.frag:222-236), on the
@@ -386,16 +397,50 @@ __global__ __launch_bounds__(256) void march_modes_kernel(const MarchArgs a) {
                     shade_model(a, gr, pos, col);
                     ++n_shaded;
                 }
-                if (mode == kCompFHP) {
-                    for (int i = 0; i < 3; ++i) col[i] = s[i];
+                if (mode == kCompMIP) {
+                    if (rw > max_int) {
+                        for (int i = 0; i < 4; ++i) out[i] = col[i];
+                        max_int = rw;
+                    }
+                } else if (mode == kCompMOP) {
+                    if (col[3] > out[3])
+                        for (int i = 0; i < 4; ++i) out[i] = col[i];
+                } else if (mode == kCompMIDA) {
+                    col[3] = s_alpha[c8 >> 24];
+                    if (a.gamma <= 0.0f) {
+                        mida_helper(out, rw, col, max_int, a.gamma);
+                    } else {
+                        float mip[4], mida[4];
+                        for (int i = 0; i < 4; ++i) mip[i] = mida[i] = out[i];
+                        if (rw > max_int) {
+                            for (int i = 0; i < 4; ++i) mip[i] = col[i];
+                            max_int = rw;
+                        }
+                        mida_helper(mida, rw, col, max_int, 0.0f);
+                        for (int i = 0; i < 4; ++i) out[i] = a.gamma * mip[i] + (1.0f - a.gamma) * mida[i];
+                    }
+                } else if (mode == kCompISO) {
+                    if (col[3] >= a.iso_value - 0.02f && col[3] <= a.iso_value + 0.02f) {
+                        out[0] = col[0];
+                        out[1] = col[1];
+                        out[2] = col[2];
+                        out[3] = 1.0f;
+                    }
+                } else if (mode == kCompFHP) {
+                    if (out[0] == 0.f && out[1] == 0.f && out[2] == 0.f) {
+                        out[0] = s[0];
+                        out[1] = s[1];
+                        out[2] = s[2];
+                        out[3] = 1.0f;
+                    }
                 } else if (mode == kCompFHN) {
-                    const float l2 = gr[0] * gr[0] + gr[1] * gr[1] + gr[2] * gr[2];
-                    const float rl = l2 > 0.f ? 1.0f / sqrtf(l2) : 0.f;
-                    for (int i = 0; i < 3; ++i) col[i] = ((gr[i] * rl) / 2.0f) + 0.5f;
+                    if (out[0] == 0.f && out[1] == 0.f && out[2] == 0.f) {
+                        const float l2 = gr[0] * gr[0] + gr[1] * gr[1] + gr[2] * gr[2];
+                        const float rl = l2 > 0.f ? 1.0f / sqrtf(l2) : 0.f;
+                        for (int i = 0; i < 3; ++i) out[i] = ((gr[i] * rl) / 2.0f) + 0.5f;
+                        out[3] = 1.0f;
+                    }
                 }
-                const float alpha = mode == kCompMIDA ? s_alpha[c8 >> 24] : col[3];
-                if (mode != kCompISO || (alpha >= a.iso_value - 0.02f && alpha <= a.iso_value + 0.02f))
-                    mode_composite(a, mode, rw, col, alpha, out, max_int);
             }
             if (ert && out[3] >= kErtOpacity) {
                 out[3] = 1.0f;
