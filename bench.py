@@ -7,7 +7,7 @@ Workload (default `--config c1`): 512^3 uint16 nested-shell volume, 6-key TF
 frames).  Volume, TF and all entry/exit images are resident in HBM before the
 timed region.  The step's views are rendered twice: as 36 per-frame march
 launches on the library's stream (what HIPRaycaster::process issues; the
-`per_frame` figures) and as one persistent batched launch of all 36 views
+`per_frame` figures) and as one batched launch of all 36 views
 (hipdvr_batch, autotuned, replayed from a captured graph), whose images equal
 the per-frame ones bit for bit.  `value` is the batched rate when a step has
 more than one view (C0's single view: the per-frame launch).
@@ -57,7 +57,7 @@ def parse():
     ap.add_argument("--steps", type=int, default=3)
     ap.add_argument("--warmup", type=int, default=1)
     ap.add_argument("--config", default="c1", choices=["c0", "c1", "c2", "c4"],
-                    help="c2: 64 uneven volumes at 512^2 in one batched persistent launch; "
+                    help="c2: 64 uneven volumes at 512^2 in one batched launch; "
                          "c4: 8 GiB turbulence volume, 8 views of 3840x2160 in one batched launch")
     ap.add_argument("--jobs", type=int, default=64, help="c2: number of volumes")
     ap.add_argument("--no-autotune", action="store_true", help="c2: keep the default configuration")
@@ -415,7 +415,7 @@ def host_path_leg(ctx, v, t, bufs, params, wimg, himg, kernel_ms, reps=20):
 
 def main_batch(args):
     """64 uneven volumes (log-uniform 64..384 per axis, u8/u16, blob volumes,
-    own TF and orbit camera), 512^2 each, one persistent launch replayed from
+    own TF and orbit camera), 512^2 each, one launch replayed from
     a captured hipGraph; one step = one batch = all jobs' frames."""
     from voreen_amd import hipdvr as H, workloads as W
     t_setup = time.perf_counter()
@@ -465,7 +465,7 @@ def main_batch(args):
         "warmup": args.warmup, "ms_per_step": round(elapsed / args.steps * 1e3, 3), "higher_is_better": True,
         "scaling": "weak", "vs_baseline": None, "dtype": "f32", "data": "synthetic",
         "config": {"workload": f"c2: {len(jobs)} uneven volumes (64..384 per axis, u8/u16), 512x512 each, "
-                               "one persistent launch from a captured hipGraph per step",
+                               "one launch from a captured hipGraph per step",
                    "autotuned": {"tile": ["8x8", "16x4", "32x2"][tuned[0]], "brick": 1 << tuned[1],
                                  "batch": tuned[2], "resident_per_cu": tuned[3], "ms": tuned_ms}},
         "gsamples_per_s": round(st["samples"] * args.steps / elapsed / 1e9, 4),
@@ -509,7 +509,7 @@ def batched_mode(args, nviews):
 
 
 def batched_views_leg(ctx, v, t, bufs, params, wimg, himg, args, bytes_orbit):
-    """All views of the step in one persistent launch (hipdvr_batch_*,
+    """All views of the step in one launch (hipdvr_batch_*,
     autotuned configuration, captured graph), each view's image compared with
     its single-frame image (the per-view launches just timed left them in
     the output buffers).  A reported rate beside `value`, which stays the
@@ -559,7 +559,7 @@ def psnr_db(a, b):
 def main_c4(args):
     """Large-volume stress: 2048x2048x1024 uint16 turbulence (8 GiB, 40% of
     the voxels empty) made on the device, 8 views of 3840x2160 with Phong.
-    One step = the 8 views in one batched persistent launch (plain path).
+    One step = the 8 views in one batched launch (plain path).
     Beside it: the same views as single frames, learned stepping per view and
     all 8 learned views in one batched launch (hipdvr_batch_launch_learned;
     network trained on plain traces of a 512^3 volume of the same generator:
@@ -611,7 +611,7 @@ def main_c4(args):
     single_s = time.perf_counter() - t0
     progress(f"single frames: {nviews / single_s:.3f} views/s")
 
-    # the batched launch: all views, one persistent grid, captured graph
+    # the batched launch: all views, captured graph
     outs = [ctx.alloc(img_bytes) for _ in range(nviews)]
     b = H.Batch(ctx, [(v, t, de, dx, o, wimg, himg, p) for (de, dx, _), p, o in zip(bufs, params, outs)])
     b.set_config(H.TILE_8x8, args.brick_log2, 2)
@@ -871,7 +871,7 @@ def main():
         ctx.synchronize()
         a.free()
         b.free()
-    # the step's views in one persistent launch: the timed figure when a step
+    # the step's views in one launch: the timed figure when a step
     # has more than one view
     bv = None
     if batched_mode(args, nviews):
@@ -888,7 +888,7 @@ def main():
         traffic = {"bytes": pmc["traffic_bytes"], "source": pmc["source"]}
     elif not bv and args.kernel == "auto" and args.batch == 0 and args.brick_log2 == 4:
         traffic = measured_traffic(args.config, "phong" if cfg["shading"] else "none")
-    launch = (f"all {nviews} views of a step in one persistent batched launch (hipdvr_batch, autotuned, "
+    launch = (f"all {nviews} views of a step in one batched launch (hipdvr_batch, autotuned, "
               "graph-replayed); per-frame launches under per_frame" if bv else "one launch per view")
     out = {
         "metric": "frames/s + Gsamples/s at 1024^2, 512^3 u16; learned vs plain at >=45 dB PSNR",

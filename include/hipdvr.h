@@ -230,7 +230,9 @@ int hipdvr_abi_version(void);
  * (no counterpart in the reference): lets a caller that loads a prebuilt
  * library check that it matches the sources shipped with it. */
 const char* hipdvr_source_digest(void);
-/* use a caller-owned HIP stream (hipStream_t as void*; NULL = context stream) */
+/* use a caller-owned HIP stream (hipStream_t as void*; NULL = context stream).
+ * Frames of one volume on several streams are ordered only where one builds
+ * what the other reads (the volume's empty-space tables). */
 int hipdvr_set_stream(hipdvr_ctx* ctx, void* stream);
 int hipdvr_synchronize(hipdvr_ctx* ctx);
 

@@ -1,4 +1,4 @@
-"""Batched persistent launch (include/hipdvr_batch.h): every job's image equals
+"""Batched launch (include/hipdvr_batch.h): every job's image equals
 its single-frame render bit for bit, for every configuration, through a
 captured graph replayed between eager work, and after autotuning."""
 import numpy as np

@@ -1,9 +1,8 @@
-"""Learned stepping inside the batched persistent launch
+"""Learned stepping inside the batched launch
 (hipdvr_batch_set_learned / hipdvr_batch_launch_learned): a learned job's
 image equals its single-view learned render (hipdvr_render_learned_device) bit
 for bit; its judge marches the sparse pixels whole, so the judged PSNR is the
-learned image's PSNR against the plain frame at exactly those pixels (the
-single-view judge joins ray segments: the same up to float rounding); plain
+learned image's PSNR against the plain frame at exactly those pixels; plain
 jobs of the same launch equal their plain frames; a bad network trips that
 job's judge so it falls back to the plain frame exactly; invalid learned sets
 are refused."""
@@ -135,8 +134,7 @@ def test_batch_learned_equals_single_learned(ctx, scene, shading):
                     host = _judge_psnr(r, plain)
                     # float32 sums on the device, float64 here
                     assert abs(st[i]["sparse_psnr"] - host) < 1e-2, (i, st[i]["sparse_psnr"], host)
-                    # the single-view judge's segment joins round (~1e-7): above
-                    # 100 dB both say the sparse pixels match
+                    # above 100 dB both say the sparse pixels match
                     q_b, q_s = st[i]["sparse_psnr"], ref_st[i]["sparse_psnr"]
                     assert abs(q_b - q_s) < 1e-2 or min(q_b, q_s) > 100.0, (i, q_b, q_s)
                     assert st[i]["fell_back"] == ref_st[i]["fell_back"], f"job {i}"

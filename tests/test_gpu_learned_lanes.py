@@ -101,3 +101,25 @@ def test_large_frame_equals_two_lanes(ctx, shading, image):
             x.free()
     finally:
         s.close()
+
+
+@pytest.mark.parametrize("shading,exact", [(0, 0), (1, 0), (1, 1)])
+def test_judge_pixels_equal_the_plain_frame(ctx, shading, exact):
+    s = Scene(ctx, (96, 80, 72), np.uint16)
+    H, image = s.H, (200, 170)
+    try:
+        print(f"[case] judge pixels shading {shading} exact {exact}", flush=True)
+        de, dx, do, p = bufs = s.view(image, 0, shading)
+        p.exact_shading = exact
+        s.ctx.render_device(s.vol, s.tf, de, dx, image[0], image[1], p, do)
+        s.ctx.synchronize()
+        plain = do.download((image[1], image[0], 4), np.float32)
+        gw, gh = H.learned_sparse_dims(*image)
+        ds = ctx.alloc(gw * gh * 16)
+        assert s.learned.sparse_remarch(s.tf, de, dx, image[0], image[1], p, ds) == (gw, gh)
+        xs, ys = ([(g // 8) * 64 + 28 + g % 8 for g in range(n)] for n in (gw, gh))
+        assert np.array_equal(ds.download((gh, gw, 4), np.float32), plain[np.ix_(ys, xs)])
+        for x in (*bufs[:3], ds):
+            x.free()
+    finally:
+        s.close()

@@ -167,8 +167,8 @@ def test_bad_weights_fall_back_to_plain(ctx, scene):
 
 @pytest.mark.parametrize("shading", [0, 1])
 def test_sparse_remarch_equals_plain(ctx, scene, shading):
-    """The judge's segmented plain re-march equals the plain frame at the
-    sparse pixels up to the float rounding of the segment joins."""
+    """The judge's plain re-march gives the plain frame at the sparse pixels
+    (bit for bit: test_gpu_learned_lanes.py)."""
     from voreen_amd import hipdvr as H
     print(f"[case] sparse re-march shading {shading}", flush=True)
     plain, st, p = _plain(ctx, scene, shading)

@@ -74,8 +74,11 @@ __host__ __device__ constexpr uint32_t cell_axis_mask(int i) {
 }
 
 // Product of two numbers below 2^24 (full rate on the VALU, a quarter of it
-// for 32-bit factors).  Brick numbers stay below it: a volume's records are
-// capped at 96 GiB, 2^18 bricks of 512 KiB, and its 8^3 skip bricks at 2^24.
+// for 32-bit factors).  In a brick's number ((z * ny) + y) * nx + x the factors
+// z, ny, nx and the inner sum, below nz * ny, stay below it: a volume's records
+// are capped at 96 GiB, 3 * 2^17 bricks (uint8; uint16 half as many), a brick is
+// at least one along x and holds 4 x 4 of the 8^3 skip bricks across it, so nz *
+// ny is at most 6.3 M.  (The product itself may pass 2^24.)
 __host__ __device__ __forceinline__ uint32_t cell_mul24(uint32_t a, uint32_t b) {
 #ifdef __HIP_DEVICE_COMPILE__
     return __umul24(a, b);

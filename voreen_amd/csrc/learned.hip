@@ -244,9 +244,8 @@ namespace {
 // in every stride * kJudgeBlock pixels, centred in it (judge_pixel).  The
 // same 1/stride^2 of the pixels as a uniform grid, but neighbouring judge
 // rays share their cell records in the caches: on 512^3 / 1024^2 with Phong
-// the re-march takes 0.70 ms (segments 0.43, join 0.28) against 0.78 ms for
-// every stride-th pixel, and the learned frame runs 1161 against 1090
-// frames/s.
+// the re-march takes 209 us against 236 for every stride-th pixel, and the
+// learned frame 677 against 713.
 constexpr uint32_t kJudgeBlock = 8;
 
 struct SparseGrid {
