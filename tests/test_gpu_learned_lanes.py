@@ -34,11 +34,11 @@ class Scene:
         self.learned = H.Learned(ctx, self.vol)
         self.opts = H.learned_opts(psnr_floor=1e-3)   # the judge accepts everything
 
-    def view(self, image, cap, shading):
+    def view(self, image, cap, shading, radius=2.1):
         w, h = image
         de, dx, do = (self.ctx.alloc(w * h * 16) for _ in range(3))
         llf, urb = self.W.world_box(self.dims)
-        cam = self.W.orbit_camera(5, 36, radius=2.1)
+        cam = self.W.orbit_camera(5, 36, radius=radius)
         self.ctx.entry_exit_device(cam, llf, urb, w, h, de, dx)
         p = self.H.default_params(self.W.step_for(self.dims, 2.0), shading=shading, camera_pos=tuple(cam.eye))
         p.loop_cap = cap
@@ -123,3 +123,54 @@ def test_judge_pixels_equal_the_plain_frame(ctx, shading, exact):
             x.free()
     finally:
         s.close()
+
+
+@pytest.mark.parametrize("images", [[(700, 600), (40, 37), (130, 57)], [(40, 37)] * 260], ids=["uneven", "many"])
+@pytest.mark.parametrize("shading", [0, 1])
+def test_fallback_frames_equal_the_plain_frames(ctx, shading, images):
+    """The views of a batch fall back (uint8 and uint16 volumes, more tiles
+    than the resident grid, more views than a workgroup has lanes), then every
+    second one."""
+    scenes = [Scene(ctx, (64, 72, 80), np.uint16), Scene(ctx, (60, 48, 52), np.uint8)]
+    H = scenes[0].H
+    bad = H.Mlp(ctx, seed=3)
+    w = bad.params()
+    w[-2] = 50.0      # skip every brick
+    bad.set_params(w)
+    views, bufs = [], {}
+    for i, image in enumerate(images):
+        key = (i % 2, image)
+        if key not in bufs:
+            bufs[key] = scenes[i % 2].view(image, 0, shading, radius=1.0)   # (judge pixels see the volume)
+        de, dx, _, p = bufs[key]
+        views.append((scenes[i % 2], de, dx, ctx.alloc(image[0] * image[1] * 16), image, p))
+    try:
+        print(f"[case] learned fallback {len(images)} views shading {shading}", flush=True)
+        ref = []
+        for s, de, dx, do, image, p in views:
+            s.ctx.render_device(s.vol, s.tf, de, dx, image[0], image[1], p, do)
+            s.ctx.synchronize()
+            ref.append(do.download((image[1], image[0], 4), np.float32))
+        for s in scenes:
+            s.learned.prepare(s.tf, next(v[5] for v in views if v[0] is s), bad)
+        b = H.Batch(ctx, [(s.vol, s.tf, de, dx, do, image[0], image[1], p) for s, de, dx, do, image, p in views])
+        try:
+            for step in (1, 2):
+                b.set_learned([v[0].learned if i % step == 0 else None for i, v in enumerate(views)])
+                for v, r in zip(views, ref):
+                    v[3].upload(np.full(r.shape, -1.0, np.float32))
+                st = b.launch_learned(stats=True)
+                for i, (v, r) in enumerate(zip(views, ref)):
+                    assert st[i]["fell_back"] == (i % step == 0), f"view {i} of every {step}"
+                    assert np.array_equal(v[3].download(r.shape, np.float32), r), f"view {i} of every {step}"
+        finally:
+            b.close()
+    finally:
+        for v in views:
+            v[3].free()
+        for de, dx, do, _ in bufs.values():
+            for x in (de, dx, do):
+                x.free()
+        bad.close()
+        for s in scenes:
+            s.close()
