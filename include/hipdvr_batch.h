@@ -87,8 +87,8 @@ int hipdvr_batch_set_learned(hipdvr_batch* b, hipdvr_learned* const* learned, ui
  * the judges' plain re-march of every learned view's sparse pixels (each ray
  * whole, so the sparse images equal the plain frames at those pixels
  * exactly) and the plain jobs, another the learned jobs; then the judges of all learned
- * views run in one launch, and a last one renders the plain frames of the
- * views that fell below the PSNR floor (the steps of
+ * views run in one launch, and per learned view the plain frame, which runs
+ * only when its view fell below the PSNR floor (the steps of
  * hipdvr_render_learned_device, for all views of the batch at once).  Asynchronous unless stats != NULL:
  * n_jobs entries in the caller's order, sparse_psnr and fell_back per learned
  * job, samples and shaded the totals of the whole launch. */

@@ -48,10 +48,6 @@ constexpr int kBrickSizes = 3;   // brick_log2 3, 4, 5
 // 8x4 824 us, 6.56 ms.
 constexpr int kBlockW = 2, kBlockH = 2;
 constexpr uint32_t kChunk = kBlockW * kBlockH;
-// Workgroups of fallback_kernel: six per compute unit, and whole rounds over
-// the XCDs.
-constexpr uint32_t kFallbackGrid = 256 * 6;
-static_assert(kFallbackGrid % kXcds == 0, "a workgroup's tiles are its XCD's");
 constexpr uint64_t kMaxTiles = 0x3fffff00;   // of a launch: four parts each below 2^32
 
 // The run that XCD x takes in round m: the round's eight runs in an order that
@@ -133,57 +129,6 @@ __global__ __launch_bounds__(256, SHADE == 2 ? 4 : (SHADE == 1 ? (COUNT ? 5 : 6)
     if (inside && sub == 0) a.out[(size_t)gy * a.grid_w + gx] = res;
     if (sparse) n = RayCounters();
     if (COUNT) add_counters<P>(counters, n, sub == 0);
-}
-
-// The plain frames of the jobs whose cond_flag is set, two lanes per ray: what a
-// learned launch falls back to, mostly none.  A resident grid that looks the
-// flags over and leaves, in one launch for all jobs of a voxel type: with a
-// launch for each of 36 views the learned launch took 13.65 ms, so it takes
-// 13.45; with 1, 6 and 36 views that fall back 15.2, 19.4 and 41.3.
-template <typename T, bool WIDE, int SHADE>
-__global__ __launch_bounds__(256, 6) void fallback_kernel(const MarchArgs* __restrict__ jobs, uint32_t njobs) {
-    constexpr int P = 2, RW = ray_w<P>(), RH = ray_h<P>(), PX = 16 / (2 * RW);
-    __shared__ uint32_t s_tf[kMaxTfWidth];
-    __shared__ float s_alpha[256];
-    __shared__ uint32_t s_set[256];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, ray = lane / P, sub = lane % P;
-    for (uint32_t j0 = 0; j0 < njobs; j0 += 256) {
-        const bool set = j0 + tid < njobs && jobs[j0 + tid].dtype == (sizeof(T) == 1 ? 0 : 1) &&
-                         *jobs[j0 + tid].cond_flag != 0;
-        s_set[tid] = set ? 1 : 0;
-        if (!__syncthreads_or(set)) continue;
-        for (uint32_t j = j0; j < j0 + 256 && j < njobs; ++j) {
-            if (!__builtin_amdgcn_readfirstlane(s_set[j - j0])) continue;   // the whole workgroup
-            const MarchArgs& a = jobs[j];
-            __syncthreads();   // the job before no longer reads the tables
-            for (int k = tid; k < a.tf_width; k += 256) s_tf[k] = a.tf[k];
-            s_alpha[tid] = a.alpha_corr[tid];
-            __syncthreads();
-            // the tiles of a single frame, in its order (march_cell_kernel)
-            const uint32_t tiles_x = (a.w + 15) / 16, tiles_y = (a.h + 15) / 16;
-            const uint32_t parts = xcd_tile_grid(tiles_x, tiles_y) * P;
-            // from another start in every frame, or the same workgroups would
-            // have the middle tiles of all of them (36 frames 41.3 ms, 61 so)
-            for (uint32_t i = (blockIdx.x + j * 53 * kXcds) % gridDim.x; i < parts; i += gridDim.x) {
-                const uint32_t slot = i / kXcds, part = slot % P;
-                uint32_t tx, ty;
-                if (!xcd_tile((slot / P) * kXcds + i % kXcds, tiles_x, tiles_y, tx, ty)) continue;
-                const int px = (int)tx * 16 + ((int)(part % PX) * 2 + (wave & 1)) * RW + ray % RW;
-                const int py = (int)ty * 16 + ((int)(part / PX) * 2 + (wave >> 1)) * RH + ray / RW;
-                if (px >= a.w || py >= a.h) continue;
-                const size_t pix = (size_t)py * a.w + px;
-                const float4 e = a.entry[pix], l = a.exit[pix];
-                float4 res = make_float4(0.f, 0.f, 0.f, 0.f);
-                if (!is_background(e, l)) {
-                    RayCounters n;
-                    const CellFetch<T, WIDE> f = cell_fetch_of<T, WIDE>(a);
-                    res = cell_ray<T, WIDE, SHADE, false, P>(a, f, s_tf, s_alpha, px, py, sub, e, l, n);
-                }
-                if (sub == 0) a.out[pix] = res;
-            }
-        }
-        __syncthreads();   // the flags are rewritten
-    }
 }
 
 typedef void (*BatchKernel)(const MarchArgs*, const uint32_t*, uint32_t, uint32_t, unsigned long long*, uint32_t);
@@ -273,7 +218,6 @@ struct hipdvr_batch {
     uint32_t n_learned = 0;
     uint32_t* d_ltile_start[kTileShapes] = {};
     uint32_t ltotal_tiles[kTileShapes] = {};
-    MarchArgs* d_fallback[kBrickSizes] = {};   // the learned jobs' plain frames, run if flagged
     uint32_t* d_queue = nullptr;
     hipStream_t queue_stream = nullptr;   // of the last learned launch
     hipdvr::JudgeJob* d_judge = nullptr;
@@ -331,15 +275,6 @@ void launch_list(hipdvr_batch* b, const BatchList& list, bool count, hipStream_t
                        (const MarchArgs*)list.d_args[bs], (const uint32_t*)list.d_tile_start[t], list.n,
                        list.total_tiles[t], b->ctx->d_counters, (uint32_t)t);
     hip_check(hipGetLastError(), "batch launch");
-}
-
-// The frames of those of n jobs whose cond_flag is set (volumes of voxel T).
-template <typename T>
-void launch_fallbacks(const MarchArgs* jobs, uint32_t n, int shade, bool wide, hipStream_t st) {
-    const auto k = wide ? (shade ? fallback_kernel<T, true, 1> : fallback_kernel<T, true, 0>)
-                        : (shade ? fallback_kernel<T, false, 1> : fallback_kernel<T, false, 0>);
-    hipLaunchKernelGGL(k, dim3(kFallbackGrid), dim3(256), 0, st, jobs, n);
-    hip_check(hipGetLastError(), "fallback launch");
 }
 
 void launch_batch(hipdvr_batch* b, bool count) { launch_list(b, b->plain, count, ctx_stream(b->ctx)); }
@@ -725,22 +660,11 @@ int hipdvr_batch_set_learned(hipdvr_batch* b, hipdvr_learned* const* learned, ui
         if (!b->d_largs) b->d_largs = dev_alloc<LearnedArgs>(b, nj * sizeof(LearnedArgs));
         for (int t = 0; t < kTileShapes; ++t)
             if (!b->d_ltile_start[t]) b->d_ltile_start[t] = dev_alloc<uint32_t>(b, (nj + 1) * 4);
-        // the learned jobs' plain frames
-        std::vector<MarchArgs> fallback[kBrickSizes];
-        for (int bs = 0; bs < kBrickSizes; ++bs) {
-            for (size_t i = 0; i < nj; ++i) {
-                if (!lv[i]) continue;
-                fallback[bs].push_back(b->h_args[bs][i]);
-                fallback[bs].back().cond_flag = flag[i];
-            }
-            if (!b->d_fallback[bs]) b->d_fallback[bs] = dev_alloc<MarchArgs>(b, nj * sizeof(MarchArgs));
-        }
         if (!b->d_queue) b->d_queue = dev_alloc<uint32_t>(b, kLearnedQueueBytes);
         if (!b->d_judge) b->d_judge = dev_alloc<JudgeJob>(b, nj * sizeof(JudgeJob));
         // every learned view gives a judge's job, the others themselves
         upload_list(b, b->with_learned, list, nj, st);
         upload(b->d_largs, largs, st);
-        for (int bs = 0; bs < kBrickSizes; ++bs) upload(b->d_fallback[bs], fallback[bs], st);
         for (int t = 0; t < kTileShapes; ++t) upload(b->d_ltile_start[t], lstart[t], st);
         upload(b->d_judge, judges, st);
         hip_check(hipStreamSynchronize(st), "hipStreamSynchronize");
@@ -763,6 +687,7 @@ int hipdvr_batch_launch_learned(hipdvr_batch* b, hipdvr_learned_stats* stats) {
         ctx_set_device(b->ctx);
         hipStream_t st = ctx_stream(b->ctx);
         const size_t nj = b->jobs.size();
+        const int bs = b->cfg.brick_log2 - 3;
         const int shade = b->shade;
         bool any = false;
         for (size_t i = 0; i < nj; ++i) {
@@ -789,18 +714,18 @@ int hipdvr_batch_launch_learned(hipdvr_batch* b, hipdvr_learned_stats* stats) {
                                  b->wide, b->cfg.resident, b->d_queue, count ? b->ctx->d_counters : nullptr, st);
         }
         if (any) {
-            // 2. the judges of all learned views in one launch, then the plain
-            //    frames of the views they have flagged
+            // 2. the judges of all learned views in one launch, then per
+            //    learned view the plain frame, launched always, which runs
+            //    only when its view was flagged
             launch_judge_multi(b->d_judge, b->n_judge, st);
-            bool u8 = false, u16 = false;
             for (size_t i = 0; i < nj; ++i) {
                 if (!b->learned[i]) continue;
-                if (b->jobs[i].volume->desc.dtype == HIPDVR_U8) u8 = true;
-                else u16 = true;
+                const hipdvr_batch_job& j = b->jobs[i];
+                MarchArgs fb = b->h_args[bs][i];
+                fb.counters = nullptr;
+                fb.cond_flag = b->d_flag[i];
+                launch_march_cell(fb, fb.dtype, shade, false, j.volume->cells_wide, 0, st);
             }
-            const MarchArgs* fb = b->d_fallback[b->cfg.brick_log2 - 3];
-            if (u8) launch_fallbacks<uint8_t>(fb, b->n_learned, shade, b->wide, st);
-            if (u16) launch_fallbacks<uint16_t>(fb, b->n_learned, shade, b->wide, st);
         }
         hip_check(hipGetLastError(), "batched learned launch");
         if (timed) ctx_timing_stop(b->ctx);

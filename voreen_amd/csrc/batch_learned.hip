@@ -8,8 +8,8 @@
 // instructions for 36 views, 9.7 G with two lanes), and a grid that stays
 // resident and takes tiles from counters, so that a workgroup loads a job's
 // tables once and starts no new wavefronts.  36 views of 512^3 at 1024^2 with
-// Phong and a trained network, with judges and fallback: 13.45 ms; as workgroups
-// of their own with one lane 14.9 ms, with two 16.3, with four 22.5.
+// Phong and a trained network, with the judges: 13.6 ms; as workgroups of their
+// own with one lane 14.9 ms, with two 16.3, with four 22.5.
 #include <hip/hip_runtime.h>
 
 #include "batch_tiles.h"

@@ -30,9 +30,6 @@ void launch_march_fast(const MarchArgs& a, int dtype, int filter, bool phong, bo
 // grid's pixels are placed by judge_pixel (a.pix_block; 1 for a whole frame).
 void launch_march_cell(const MarchArgs& a, int dtype, int shade, bool count, bool wide, int batch,
                        hipStream_t st);
-// The plain frame that replaces a learned one below its floor: a launch with
-// a.cond_flag, which mostly finds it 0.
-void launch_fallback(const MarchArgs& a, int dtype, int shade, bool wide, hipStream_t st);
 // The other compositing modes (preint false) or the pre-integrated
 // classification on the cell records, linear filter and central differences:
 // the reference-layout kernels' results bit for bit.  Without a.skip nothing

@@ -647,7 +647,7 @@ int hipdvr_render_learned_device(hipdvr_learned* l, const hipdvr_tf* tf, const f
         fill_march_args(fb, vol, tf, prm, d_entry, d_exit, d_out, w, h, nullptr);
         fb.skip = skip;
         fb.cond_flag = l->d_flag;
-        launch_fallback(fb, vol->desc.dtype, shade, vol->cells_wide, st);
+        launch_march_cell(fb, vol->desc.dtype, shade, false, vol->cells_wide, 0, st);
         hip_check(hipGetLastError(), "learned render launch");
         if (timed) ctx_timing_stop(l->ctx);
         if (count) {

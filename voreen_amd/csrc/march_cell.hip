@@ -92,11 +92,4 @@ void launch_march_cell(const MarchArgs& a, int dtype, int shade, bool count, boo
     }
 }
 
-// Above 600 K pixels two lanes per ray, whose workgroups are half as many to
-// start and leave at once: 1024^2 7 us against 11 with four, whose frame would
-// take 674 us instead of 714 where it runs.
-void launch_fallback(const MarchArgs& a, int dtype, int shade, bool wide, hipStream_t st) {
-    launch_march_cell(a, dtype, shade, false, wide, (uint64_t)a.grid_w * a.grid_h > 600000 ? 2 : 0, st);
-}
-
 }  // namespace hipdvr
