@@ -1,8 +1,8 @@
 """The learned march with 1, 2 and 4 lanes per ray: its samples do not depend
-on the number of lanes, whatever the loop cap, so a frame of 2 lanes, one of 4
-and the batched launch (one lane, several samples in flight) give the same
-image bit for bit, and a frame large enough for one lane the image that 2 lanes
-give."""
+on the number of lanes, whatever the loop cap, so a frame of 2 lanes, one of 4 and the batched
+launch (by its size 4 lanes, 2, or one with several samples in flight) give the
+same image bit for bit, and a frame large enough for one lane the image that 2
+lanes give."""
 import numpy as np
 import pytest
 
@@ -99,6 +99,86 @@ def test_large_frame_equals_two_lanes(ctx, shading, image):
         assert np.array_equal(s.frame(bufs, image, 0), s.frame(bufs, image, 2))
         for x in bufs[:3]:
             x.free()
+    finally:
+        s.close()
+
+
+# pixels of the first image: two lanes per ray, one (unshaded, with Phong)
+@pytest.mark.parametrize("shading,image", [(0, (1301, 1201)), (1, (1301, 1201)), (0, (3103, 2917)), (1, (3607, 3391))],
+                         ids=["unshaded-2", "phong-2", "unshaded-1", "phong-1"])
+def test_large_batch_equals_two_lane_frames(ctx, shading, image):
+    """Learned views of both voxel types and odd sizes and a plain one, in a
+    launch of 1.5 to 6 M pixels and in one large enough for one lane."""
+    scenes = [Scene(ctx, (64, 72, 80), np.uint16), Scene(ctx, (60, 48, 52), np.uint8)]
+    jobs = [(scenes[i], im) for i, im in ((0, image), (1, (131, 57)), (0, (40, 37)), (1, (63, 129)))]
+    plain = 2
+    views = [(s, im, s.view(im, 0, shading)) for s, im in jobs]
+    try:
+        print(f"[case] learned batch {image} shading {shading}", flush=True)
+        for s in scenes:
+            s.learned.prepare(s.tf, next(v[2][3] for v in views if v[0] is s), s.net, opts=s.opts)
+        ref = []
+        for i, (s, im, bufs) in enumerate(views):
+            if i != plain:
+                ref.append(s.frame(bufs, im, 2))
+                continue
+            de, dx, do, p = bufs
+            s.ctx.render_device(s.vol, s.tf, de, dx, im[0], im[1], p, do)
+            s.ctx.synchronize()
+            ref.append(do.download((im[1], im[0], 4), np.float32))
+        b = scenes[0].H.Batch(ctx, [(s.vol, s.tf, de, dx, do, im[0], im[1], p) for s, im, (de, dx, do, p) in views])
+        try:
+            b.set_learned([None if i == plain else v[0].learned for i, v in enumerate(views)], scenes[0].opts)
+            for tile, resident in ((0, 0), (1, 2), (2, 8)):
+                b.set_config(tile, 3, 2, resident)
+                for v, r in zip(views, ref):
+                    v[2][2].upload(np.full(r.shape, -1.0, np.float32))
+                b.launch_learned(stats=True)
+                for i, (v, r) in enumerate(zip(views, ref)):
+                    assert np.array_equal(v[2][2].download(r.shape, np.float32), r), f"view {i} tile {tile}"
+        finally:
+            b.close()
+        for v in views:
+            for x in v[2][:3]:
+                x.free()
+    finally:
+        for s in scenes:
+            s.close()
+
+
+@pytest.mark.parametrize("shading", [0, 1])
+def test_records_past_4_gib(ctx, shading):
+    """Volumes addressed with 64 bits: batches of 4 and 2 lanes and a frame
+    large enough for one lane elsewhere, against frames of 2 and 4 lanes."""
+    from voreen_amd import hipdvr as H, workloads as W
+    s = Scene.__new__(Scene)
+    s.ctx, s.H, s.W, s.dims = ctx, H, W, (2048, 1024, 144)
+    vox, _ = ctx.synth_turbulence(0x51, s.dims, 0.4)
+    s.vol = ctx.volume_device(vox, s.dims, H.U16)
+    vox.free()
+    _, tf = W.make_tf("c4")
+    s.tf, s.net = ctx.transfunc(tf), network(H, ctx)
+    s.learned, s.opts = H.Learned(ctx, s.vol), H.learned_opts(psnr_floor=1e-3)
+    try:
+        for image in ((131, 77), (1381, 1301)):
+            print(f"[case] learned 64-bit {image} shading {shading}", flush=True)
+            bufs = s.view(image, 0, shading, radius=1.4)
+            de, dx, do, p = bufs
+            s.learned.prepare(s.tf, p, s.net, opts=s.opts)
+            two, four = s.frame(bufs, image, 2), s.frame(bufs, image, 4)
+            assert np.mean(two[..., 3] > 0) > 0.1
+            assert np.array_equal(two, four) and np.array_equal(two, s.frame(bufs, image, 0))
+            b = H.Batch(ctx, [(s.vol, s.tf, de, dx, do, image[0], image[1], p)])
+            try:
+                b.set_learned([s.learned], s.opts)
+                b.set_config(0, 3, 2)
+                do.upload(np.full(two.shape, -1.0, np.float32))
+                b.launch_learned(stats=True)
+                assert np.array_equal(two, do.download(two.shape, np.float32))
+            finally:
+                b.close()
+            for x in (de, dx, do):
+                x.free()
     finally:
         s.close()
 

@@ -37,34 +37,7 @@ namespace {
 constexpr int kTileShapes = 3;
 constexpr int kBrickSizes = 3;   // brick_log2 3, 4, 5
 
-// The order of the tiles.  The hardware hands consecutive workgroups to the
-// 8 XCDs in turn (workgroup b to XCD b % 8), and each XCD has its own L2.
-// Tiles come in blocks of kBlockW x kBlockH tiles of one job (blocks row by
-// row, tiles row by row inside a block; edge blocks smaller); consecutive runs
-// of kChunk tiles of the launch's tile range are dealt to the XCDs in turn, so
-// the tiles an XCD marches at a time are a few compact blocks whose rays share
-// that XCD's L2, and the eight march neighbouring ones.  Blocks of 2x2 tiles:
-// 64 uneven volumes 709 us, 12 views of 512^3 6.43 ms; 4x4 695 us, 6.51 ms;
-// 8x4 824 us, 6.56 ms.
-constexpr int kBlockW = 2, kBlockH = 2;
-constexpr uint32_t kChunk = kBlockW * kBlockH;
 constexpr uint64_t kMaxTiles = 0x3fffff00;   // of a launch: four parts each below 2^32
-
-// The run that XCD x takes in round m: the round's eight runs in an order that
-// changes from round to round without a pattern, so that no XCD meets the same
-// column of an image whatever its width (dealt in a fixed order, 12 views of
-// 1024^2 took 13.1 ms, the XCDs of the middle columns marching alone for half
-// of it).
-__host__ __device__ inline uint32_t xcd_run(uint32_t x, uint32_t m) {
-    return kXcds * m + (x ^ ((m * 0x9E3779B1u) >> 29));
-}
-
-// Workgroups for `total` tiles in P parts each: whole rounds of runs (those
-// past the last tile leave at once).
-inline uint64_t batch_grid(uint32_t total, int parts) {
-    const uint64_t chunks = ((uint64_t)total + kChunk - 1) / kChunk;
-    return (chunks + kXcds - 1) / kXcds * kXcds * kChunk * (uint64_t)parts;
-}
 
 // One workgroup per P-th of a tile, P lanes per ray (march_cell.h).  The
 // tile's 2x2 regions of 64 pixels fall into parts of 64 / P rays; wavefront w
@@ -77,7 +50,7 @@ __global__ __launch_bounds__(256, SHADE == 2 ? 4 : (SHADE == 1 ? (COUNT ? 5 : 6)
     const MarchArgs* __restrict__ jobs, const uint32_t* __restrict__ tile_start, uint32_t njobs,
     uint32_t total_tiles, unsigned long long* __restrict__ counters, uint32_t tile_shape) {
     const uint32_t block = linear_block(), slot = block / kXcds, part = slot % P, i = slot / P;
-    const uint32_t tile = xcd_run(block % kXcds, i / kChunk) * kChunk + i % kChunk;
+    const uint32_t tile = xcd_run(block % kXcds, i / kTileRun) * kTileRun + i % kTileRun;
     if (tile >= total_tiles) return;
     __shared__ uint32_t s_tf[kMaxTfWidth];
     __shared__ float s_alpha[256];
@@ -88,7 +61,7 @@ __global__ __launch_bounds__(256, SHADE == 2 ? 4 : (SHADE == 1 ? (COUNT ? 5 : 6)
     const int WW = 8 << tile_shape, WH = 8 >> tile_shape;
     const int RH = ray_h<P>() < WH ? ray_h<P>() : WH, RW = 64 / P / RH, cols = WW / RW;
     uint32_t tx, ty;
-    block_tile<kBlockW, kBlockH>(tile - tile_start[job], (uint32_t)(a.grid_w + 2 * WW - 1) / (2 * WW),
+    block_tile<kTileBlockW, kTileBlockH>(tile - tile_start[job], (uint32_t)(a.grid_w + 2 * WW - 1) / (2 * WW),
                                  (uint32_t)(a.grid_h + 2 * WH - 1) / (2 * WH), tx, ty);
     // a job marches the pixels of its grid: the whole image, or (a judge's
     // re-march: pix_block > 1) the sparse pixels judge_pixel places, written
@@ -216,6 +189,8 @@ struct hipdvr_batch {
     BatchList with_learned;
     LearnedArgs* d_largs = nullptr;
     uint32_t n_learned = 0;
+    uint64_t learned_pixels = 0;
+    double learned_faces = 0.0;   // voxels of a face of each learned job's volume, if it were a cube
     uint32_t* d_ltile_start[kTileShapes] = {};
     uint32_t ltotal_tiles[kTileShapes] = {};
     uint32_t* d_queue = nullptr;
@@ -259,6 +234,29 @@ void validate_config(const hipdvr_batch_config& c) {
 }
 
 int list_lanes(const BatchList& l, int batch) { return batch_lanes(batch, l.pixels, l.rays, l.step); }
+
+// Lanes per ray of the learned jobs: one, in a persistent launch of their own
+// (launch_learned_batch), or 2 or 4 in one launch with the plain jobs
+// (launch_learned_mixed).  One lane repeats no skipping among the lanes of a
+// ray, so it is the better the more rays there are to fill the chip with; but a
+// wavefront then holds 64 rays, which part ways where an image has few pixels
+// for its volume's voxels, and the judges' few rays march alone before.  One /
+// two lanes, ms (blobs in 512^3): 1024^2 with Phong 4 views 2.10 / 1.93, 12 5.11
+// / 5.32, 24 9.56 / 10.68, unshaded 4 1.27 / 1.23, 12 3.03 / 3.29, 24 5.62 /
+// 6.48; 1080p 4 views 2.38 / 2.10, 8 3.98 / 4.02, unshaded 1.40 / 1.35, 2.32 /
+// 2.53; 768^2 (2.25 pixels to a voxel) 36 views 10.6 / 10.3, 5.71 / 5.91; 512^2
+// (one pixel) 96 views 18.6 / 14.8, 8.67 / 7.86.  Turbulence in 512^3 and blobs
+// in 256^3 have their lines within a factor of 1.5 of these.  Records past 4 GiB,
+// whose loads take longer, never take one lane: 8 views of 2048 x 2048 x 1024 at
+// 3840 x 2160 105 / 66.6 ms.
+int learned_batch_lanes(const hipdvr_batch* b) {
+    if (!b->wide && b->learned_pixels > (b->shade ? 12000000u : 9000000u) &&
+        (double)b->learned_pixels >= 2.5 * b->learned_faces)
+        return 1;
+    const uint64_t pixels = b->learned_pixels + b->with_learned.pixels;
+    if (pixels <= 1500000) return 4;
+    return pixels > 6000000 ? 2 : b->cfg.batch;
+}
 
 void launch_list(hipdvr_batch* b, const BatchList& list, bool count, hipStream_t st) {
     if (list.n == 0) return;
@@ -656,7 +654,11 @@ int hipdvr_batch_set_learned(hipdvr_batch* b, hipdvr_learned* const* learned, ui
                 if (!lv[i]) list.args[bs].push_back(b->h_args[bs][i]);
         list.tiles();
         std::vector<uint32_t> lstart[kTileShapes];
-        for (int t = 0; t < kTileShapes; ++t) lstart[t] = tile_starts(largs, t, learned_args);
+        for (int t = 0; t < kTileShapes; ++t) {
+            lstart[t] = tile_starts(largs, t, learned_args);
+            if ((uint64_t)lstart[t].back() + list.start[t].back() > kMaxTiles)
+                fail(HIPDVR_ERR_UNSUPPORTED, "batch too large");
+        }
         if (!b->d_largs) b->d_largs = dev_alloc<LearnedArgs>(b, nj * sizeof(LearnedArgs));
         for (int t = 0; t < kTileShapes; ++t)
             if (!b->d_ltile_start[t]) b->d_ltile_start[t] = dev_alloc<uint32_t>(b, (nj + 1) * 4);
@@ -669,6 +671,15 @@ int hipdvr_batch_set_learned(hipdvr_batch* b, hipdvr_learned* const* learned, ui
         upload(b->d_judge, judges, st);
         hip_check(hipStreamSynchronize(st), "hipStreamSynchronize");
         b->n_learned = (uint32_t)largs.size();
+        b->learned_pixels = 0;
+        b->learned_faces = 0.0;
+        for (size_t i = 0; i < nj; ++i) {
+            if (!lv[i]) continue;
+            const hipdvr_batch_job& j = b->jobs[i];
+            b->learned_pixels += (uint64_t)j.w * j.h;
+            const uint32_t* d = j.volume->desc.dims;
+            b->learned_faces += std::pow((double)d[0] * d[1] * d[2], 2.0 / 3.0);
+        }
         for (int t = 0; t < kTileShapes; ++t) b->ltotal_tiles[t] = lstart[t].back();
         b->n_judge = (uint32_t)judges.size();
         b->lopts = lopts;
@@ -700,19 +711,23 @@ int hipdvr_batch_launch_learned(hipdvr_batch* b, hipdvr_learned_stats* stats) {
         if (count) launch_zero_u64(b->ctx->d_counters, kNumCounters, st);
         const bool timed = ctx_timing_start(b->ctx);
         if (!b->d_largs) fail(HIPDVR_ERR_INVALID, "hipdvr_batch_set_learned has not been called");
-        // 1. the judges' plain re-marches of the learned views' sparse pixels
-        //    and the plain jobs in one launch, then the learned jobs in
-        //    another (side by side on two streams they took a twentieth
-        //    longer: the persistent grid no longer fills the chip evenly)
-        launch_list(b, b->with_learned, count, st);
-        if (any) {
+        // 1. the judges' plain re-marches of the learned views' sparse pixels,
+        //    the plain jobs and the learned ones
+        const BatchList& plain = b->with_learned;
+        const int t = b->cfg.tile;
+        const int lanes = any ? learned_batch_lanes(b) : 0;
+        if (lanes < 2) launch_list(b, plain, count, st);
+        if (lanes == 1) {
             // the queue's counters serve one launch at a time
             if (b->queue_stream && b->queue_stream != st) ctx_wait_left(b->ctx, b->queue_stream, ctx_capturing(b->ctx));
             b->queue_stream = st;
-            const int t = b->cfg.tile;
             launch_learned_batch(b->d_largs, b->d_ltile_start[t], b->n_learned, b->ltotal_tiles[t], t, shade != 0,
-                                 b->wide, b->cfg.resident, b->d_queue, count ? b->ctx->d_counters : nullptr, st);
+                                 b->cfg.resident, b->d_queue, count ? b->ctx->d_counters : nullptr, st);
         }
+        if (lanes > 1)
+            launch_learned_mixed(plain.d_args[bs], plain.d_tile_start[t], plain.n, plain.n ? plain.total_tiles[t] : 0,
+                                 b->d_largs, b->d_ltile_start[t], b->n_learned, b->ltotal_tiles[t], t, lanes,
+                                 shade != 0, b->wide, b->cfg.resident, count ? b->ctx->d_counters : nullptr, st);
         if (any) {
             // 2. the judges of all learned views in one launch, then per
             //    learned view the plain frame, launched always, which runs

@@ -1,15 +1,22 @@
 // batch_learned.hip -- the learned jobs of a batched launch
-// (hipdvr_batch_launch_learned): every learned view's tiles in one persistent
-// launch.
+// (hipdvr_batch_launch_learned), in one of two forms (batch.hip,
+// learned_batch_lanes, chooses by the launch's size).
 //
-// The launch has rays enough to fill the chip and is bound by the instructions
-// it issues: one lane per ray with two (Phong) or four samples in flight,
-// which computes a pass's chain of positions once (learned_ray.h; 7.4 G vector
-// instructions for 36 views, 9.7 G with two lanes), and a grid that stays
-// resident and takes tiles from counters, so that a workgroup loads a job's
-// tables once and starts no new wavefronts.  36 views of 512^3 at 1024^2 with
-// Phong and a trained network, with the judges: 13.6 ms; as workgroups of their
-// own with one lane 14.9 ms, with two 16.3, with four 22.5.
+// Large launches have rays enough to fill the chip and are bound by the
+// instructions they issue.  A persistent launch marches every learned view's
+// tiles with one lane per ray and two (Phong) or four samples in flight, which
+// computes a pass's chain of positions once (learned_ray.h; 7.4 G vector
+// instructions for 36 views, 9.7 G with two lanes); its grid stays resident and
+// takes tiles from counters, so that a workgroup loads a job's tables once and
+// starts no new wavefronts.  36 views of 512^3 at 1024^2 with Phong and a trained
+// network, with the judges: 13.6 ms; as workgroups of their own with one lane
+// 14.9 ms, with two 16.3, with four 22.5.
+//
+// The others are bound by the chain of a ray's samples, or by loads of records
+// past 4 GiB: a plain grid marches the judges' rays, the plain jobs and the
+// learned ones side by side with two or four lanes per ray.  One view of 512^3 at
+// 1024^2 0.76 ms (in the persistent launch 0.90), 36 of 512^2 5.90 (7.44), 8 of
+// 2048 x 2048 x 1024 at 3840 x 2160 66.9 (105).
 #include <hip/hip_runtime.h>
 
 #include "batch_tiles.h"
@@ -17,6 +24,7 @@
 #include "learned.h"
 #include "learned_ray.h"
 #include "march_cell.h"
+#include "residency.h"
 
 namespace hipdvr {
 
@@ -64,7 +72,7 @@ __device__ __forceinline__ uint32_t take_tile(uint32_t* counter, uint32_t x, uin
 }
 
 // A workgroup is a tile's 2x2 regions of 64 pixels, one per wavefront.
-template <bool WIDE, bool PHONG, bool COUNT>
+template <bool PHONG, bool COUNT>
 __global__ __launch_bounds__(256) void learned_batch_kernel(const LearnedArgs* __restrict__ jobs,
                                                             const uint32_t* __restrict__ tile_start, uint32_t njobs,
                                                             uint32_t total_tiles, uint32_t tile_shape,
@@ -102,14 +110,14 @@ __global__ __launch_bounds__(256) void learned_batch_kernel(const LearnedArgs* _
             const float4 e = a.entry[pix], l = a.exit[pix];
             float4 res = make_float4(0.f, 0.f, 0.f, 0.f);
             if (!is_background(e, l)) {
-                // WIDE: 64-bit record addressing for every job (a volume's
-                // records exceed 4 GiB); else 32-bit buffer offsets
                 if (a.dtype == 0) {
-                    const CellFetch<uint8_t, WIDE> f = cell_fetch_of<uint8_t, WIDE>(a);
-                    res = learned_ray_single<uint8_t, WIDE, PHONG>(la, f, s_tf, s_alpha, px, py, e, l, n_samples, n_shaded);
+                    const CellFetch<uint8_t, false> f = cell_fetch_of<uint8_t, false>(a);
+                    res = learned_ray_single<uint8_t, false, PHONG>(la, f, s_tf, s_alpha, px, py, e, l, n_samples,
+                                                                    n_shaded);
                 } else {
-                    const CellFetch<uint16_t, WIDE> f = cell_fetch_of<uint16_t, WIDE>(a);
-                    res = learned_ray_single<uint16_t, WIDE, PHONG>(la, f, s_tf, s_alpha, px, py, e, l, n_samples, n_shaded);
+                    const CellFetch<uint16_t, false> f = cell_fetch_of<uint16_t, false>(a);
+                    res = learned_ray_single<uint16_t, false, PHONG>(la, f, s_tf, s_alpha, px, py, e, l, n_samples,
+                                                                     n_shaded);
                 }
                 ++n_rays;
             }
@@ -124,21 +132,121 @@ __global__ __launch_bounds__(256) void learned_batch_kernel(const LearnedArgs* _
     }
 }
 
-typedef void (*LearnedBatchKernel)(const LearnedArgs*, const uint32_t*, uint32_t, uint32_t, uint32_t, uint32_t*,
-                                   unsigned long long*);
+// The plain jobs and the learned ones in one launch, the plain first (the judges'
+// re-marches start while the chip fills), by workgroups of their own: one per
+// P-th of a tile, P lanes per ray, as batch_kernel.
+template <bool WIDE, bool PHONG, bool COUNT, int P>
+__global__ __launch_bounds__(256, PHONG ? 5 : (COUNT ? 6 : 7)) void mixed_kernel(
+    const MarchArgs* __restrict__ plain, const uint32_t* __restrict__ plain_start, uint32_t nplain, uint32_t plain_tiles,
+    const LearnedArgs* __restrict__ jobs, const uint32_t* __restrict__ tile_start, uint32_t njobs, uint32_t total_tiles,
+    uint32_t tile_shape, unsigned long long* __restrict__ counters) {
+    const uint32_t block = linear_block(), slot = block / kXcds, part = slot % P, i = slot / P;
+    uint32_t tile = xcd_run(block % kXcds, i / kTileRun) * kTileRun + i % kTileRun;
+    if (tile >= plain_tiles + total_tiles) return;
+    __shared__ uint32_t s_tf[kMaxTfWidth];
+    __shared__ float s_alpha[256];
+    const bool learned = tile >= plain_tiles;
+    if (learned) tile -= plain_tiles;
+    const uint32_t* start = learned ? tile_start : plain_start;
+    const uint32_t job = job_of_tile(start, learned ? njobs : nplain, tile);
+    const LearnedArgs& la = jobs[learned ? job : 0];
+    const MarchArgs& a = learned ? la.m : plain[job];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, ray = lane / P, sub = lane % P;
+    const int WW = 8 << tile_shape, WH = 8 >> tile_shape;
+    const int RH = ray_h<P>() < WH ? ray_h<P>() : WH, RW = 64 / P / RH, cols = WW / RW;
+    uint32_t tx, ty;
+    block_tile<kTileBlockW, kTileBlockH>(tile - start[job], (uint32_t)(a.grid_w + 2 * WW - 1) / (2 * WW),
+                                         (uint32_t)(a.grid_h + 2 * WH - 1) / (2 * WH), tx, ty);
+    const bool sparse = a.pix_block > 1;   // a judge's re-march (batch_kernel)
+    const int q = (int)part * 4 + wave, region = q / P, rp = q % P;
+    const int gx = ((int)tx * 2 + (region & 1)) * WW + (rp % cols) * RW + ray % RW;
+    const int gy = ((int)ty * 2 + (region >> 1)) * WH + (rp / cols) * RH + ray / RW;
+    const bool inside = gx < a.grid_w && gy < a.grid_h;
+    const int px = sparse ? judge_pixel(gx, a.stride, a.pix_block, a.pix_offset) : gx;
+    const int py = sparse ? judge_pixel(gy, a.stride, a.pix_block, a.pix_offset) : gy;
+    float4 e = make_float4(0.f, 0.f, 0.f, 0.f), l = e, res = e;
+    if (inside) {
+        const size_t pix = (size_t)py * a.w + px;
+        e = a.entry[pix];
+        l = a.exit[pix];
+    }
+    const bool hit = !is_background(e, l);
+    RayCounters n;
+    if (__syncthreads_or(hit)) {
+        for (int k = tid; k < a.tf_width; k += 256) s_tf[k] = a.tf[k];
+        s_alpha[tid] = learned ? la.alpha_m[tid] : a.alpha_corr[tid];
+        __syncthreads();
+        if (hit) {
+            if (learned) {
+                unsigned long long ns = 0, nsh = 0;
+                if (a.dtype == 0) {
+                    const CellFetch<uint8_t, WIDE> f = cell_fetch_of<uint8_t, WIDE>(a);
+                    res = learned_ray<uint8_t, WIDE, PHONG, P>(la, f, s_tf, s_alpha, px, py, sub, e, l, ns, nsh);
+                } else {
+                    const CellFetch<uint16_t, WIDE> f = cell_fetch_of<uint16_t, WIDE>(a);
+                    res = learned_ray<uint16_t, WIDE, PHONG, P>(la, f, s_tf, s_alpha, px, py, sub, e, l, ns, nsh);
+                }
+                ++n.rays;
+                n.fetched += sub == 0 ? (uint32_t)ns : 0;   // the ray's, counted by one lane
+                n.shaded += sub == 0 ? (uint32_t)nsh : 0;
+            } else if (a.dtype == 0) {
+                const CellFetch<uint8_t, WIDE> f = cell_fetch_of<uint8_t, WIDE>(a);
+                res = cell_ray<uint8_t, WIDE, PHONG ? 1 : 0, COUNT, P>(a, f, s_tf, s_alpha, px, py, sub, e, l, n);
+            } else {
+                const CellFetch<uint16_t, WIDE> f = cell_fetch_of<uint16_t, WIDE>(a);
+                res = cell_ray<uint16_t, WIDE, PHONG ? 1 : 0, COUNT, P>(a, f, s_tf, s_alpha, px, py, sub, e, l, n);
+            }
+        }
+    }
+    if (inside && sub == 0) a.out[(size_t)gy * a.grid_w + gx] = res;
+    if (sparse) n = RayCounters();
+    if (COUNT) add_counters<P>(counters, n, sub == 0);
+}
 
-template <bool WIDE>
-LearnedBatchKernel pick(bool phong, bool count) {
-    if (phong) return count ? learned_batch_kernel<WIDE, true, true> : learned_batch_kernel<WIDE, true, false>;
-    return count ? learned_batch_kernel<WIDE, false, true> : learned_batch_kernel<WIDE, false, false>;
+typedef void (*ResidentKernel)(const LearnedArgs*, const uint32_t*, uint32_t, uint32_t, uint32_t, uint32_t*,
+                               unsigned long long*);
+typedef void (*MixedKernel)(const MarchArgs*, const uint32_t*, uint32_t, uint32_t, const LearnedArgs*, const uint32_t*,
+                            uint32_t, uint32_t, uint32_t, unsigned long long*);
+
+ResidentKernel resident_kernel(bool phong, bool count) {
+    if (phong) return count ? learned_batch_kernel<true, true> : learned_batch_kernel<true, false>;
+    return count ? learned_batch_kernel<false, true> : learned_batch_kernel<false, false>;
+}
+template <bool WIDE, int P>
+MixedKernel mixed_of(bool phong, bool count) {
+    if (phong) return count ? mixed_kernel<WIDE, true, true, P> : mixed_kernel<WIDE, true, false, P>;
+    return count ? mixed_kernel<WIDE, false, true, P> : mixed_kernel<WIDE, false, false, P>;
+}
+template <int P>
+MixedKernel mixed_of(bool wide, bool phong, bool count) {
+    return wide ? mixed_of<true, P>(phong, count) : mixed_of<false, P>(phong, count);
 }
 
 }  // namespace
 
+void launch_learned_mixed(const MarchArgs* plain, const uint32_t* plain_start, uint32_t nplain, uint32_t plain_tiles,
+                          const LearnedArgs* jobs, const uint32_t* tile_start, uint32_t njobs, uint32_t total_tiles,
+                          int tile_shape, int lanes, bool phong, bool wide, int resident, unsigned long long* counters,
+                          hipStream_t st) {
+    const bool count = counters != nullptr;
+    const MixedKernel k = lanes == 2 ? mixed_of<2>(wide, phong, count) : mixed_of<4>(wide, phong, count);
+    size_t pad = 0;
+    if (resident > 0) {
+        hipFuncAttributes fa;
+        hip_check(hipFuncGetAttributes(&fa, (const void*)k), "hipFuncGetAttributes");
+        pad = residency_pad(fa.sharedSizeBytes, resident);
+    }
+    hipLaunchKernelGGL(k, linear_grid(batch_grid(plain_tiles + total_tiles, lanes)), dim3(256), pad, st, plain,
+                       plain_start, nplain, plain_tiles, jobs, tile_start, njobs, total_tiles, (uint32_t)tile_shape,
+                       counters);
+    hip_check(hipGetLastError(), "learned batch launch");
+}
+
 void launch_learned_batch(const LearnedArgs* jobs, const uint32_t* tile_start, uint32_t njobs, uint32_t total_tiles,
-                          int tile_shape, bool phong, bool wide, int resident, uint32_t* queue,
-                          unsigned long long* counters, hipStream_t st) {
-    const LearnedBatchKernel k = wide ? pick<true>(phong, counters != nullptr) : pick<false>(phong, counters != nullptr);
+                          int tile_shape, bool phong, int resident, uint32_t* queue, unsigned long long* counters,
+                          hipStream_t st) {
+    const bool count = counters != nullptr;
+    const ResidentKernel k = resident_kernel(phong, count);
     int per_cu = 0, device = 0, cus = 0;
     hip_check(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)k, 256, 0), "occupancy query");
     hip_check(hipGetDevice(&device), "hipGetDevice");

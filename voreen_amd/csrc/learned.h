@@ -50,7 +50,7 @@ void launch_trace(const LearnedArgs& la, float* err, unsigned int* visits, hipSt
 void launch_targets(const float* err, const unsigned int* visits, const float* feat, uint32_t rows,
                     float tau_skip, float tau_step, float* out_x, float* out_t, unsigned int* count,
                     uint32_t capacity, hipStream_t st);
-// lanes per ray: 1, 2 or 4 (more run as four)
+// lanes per ray: 1 (wide: 2), 2 or 4 (more run as four)
 void launch_learned(const LearnedArgs& la, bool phong, bool count, bool wide, int lanes, hipStream_t st);
 
 // For batched launches (batch.hip): the judge's sparse grid of a w x h image
@@ -84,14 +84,20 @@ struct JudgeJob {
     float denom, mse_max;
 };
 void launch_judge_multi(const JudgeJob* jobs, uint32_t n, hipStream_t st);
-// The learned jobs of a batch in one persistent launch (batch_learned.hip):
-// njobs jobs of total_tiles tiles of the shape, tile_start[njobs + 1] their
-// first tiles; resident: workgroups per CU at most (0: as many as fit); queue:
-// kLearnedQueueBytes of device memory; counters: as MarchArgs::counters, or
-// null.
+// The learned jobs of a batch in one persistent launch, one lane per ray
+// (batch_learned.hip; records within 4 GiB): njobs jobs of total_tiles tiles of
+// the shape, tile_start[njobs + 1] their first tiles; resident: workgroups per CU
+// at most (0: as many as fit); queue: kLearnedQueueBytes of device memory;
+// counters: as MarchArgs::counters, or null.
 constexpr size_t kLearnedQueueBytes = 1024;
 void launch_learned_batch(const LearnedArgs* jobs, const uint32_t* tile_start, uint32_t njobs, uint32_t total_tiles,
-                          int tile_shape, bool phong, bool wide, int resident, uint32_t* queue,
-                          unsigned long long* counters, hipStream_t st);
+                          int tile_shape, bool phong, int resident, uint32_t* queue, unsigned long long* counters,
+                          hipStream_t st);
+// The plain jobs of a learned launch and the learned ones in one plain grid, 2 or
+// 4 lanes per ray, each list as above (the plain one's may be empty).
+void launch_learned_mixed(const MarchArgs* plain, const uint32_t* plain_start, uint32_t nplain, uint32_t plain_tiles,
+                          const LearnedArgs* jobs, const uint32_t* tile_start, uint32_t njobs, uint32_t total_tiles,
+                          int tile_shape, int lanes, bool phong, bool wide, int resident, unsigned long long* counters,
+                          hipStream_t st);
 
 }  // namespace hipdvr

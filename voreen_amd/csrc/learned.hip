@@ -392,10 +392,13 @@ void fill_learned_args(LearnedArgs& la, hipdvr_learned* l, const hipdvr_tf* tf, 
 // 593 / 431 / 494, 1024^2 676 / 642 / 801, 1200^2 739 / 755 / 963, 1300^2 801
 // / 831 / 1098, 2048^2 1431 / 1663 / 2371; unshaded: 600^2 295 / 291 / 259,
 // 724^2 304 / 303 / 321, 1024^2 414 / 437 / 511, 2048^2 917 / 1119 / 1531.
-int learned_lanes(const hipdvr_params* p, uint64_t pixels) {
+// Records past 4 GiB, whose loads take longer, always by 2 (2048 x 2048 x 1024,
+// ms): with Phong 1024^2 4.52 / 4.51 / 3.71, 3840 x 2160 12.8 / 9.00 / 8.49,
+// unshaded 1.87 / 1.72 / 1.68 and 4.18 / 3.93 / 4.29.
+int learned_lanes(const hipdvr_params* p, uint64_t pixels, bool wide) {
     if (p->batch) return frame_lanes(p->batch, pixels, p->step);
-    if (pixels > (p->shading == HIPDVR_SHADE_NONE ? 800000u : 1300000u)) return 1;
-    return pixels > 430000 ? 2 : frame_lanes(0, pixels, p->step);
+    if (!wide && pixels > (p->shading == HIPDVR_SHADE_NONE ? 800000u : 1300000u)) return 1;
+    return pixels > (wide ? 600000u : 430000u) ? 2 : frame_lanes(0, pixels, p->step);
 }
 
 }  // namespace
@@ -635,7 +638,8 @@ int hipdvr_render_learned_device(hipdvr_learned* l, const hipdvr_tf* tf, const f
         fill_learned_args(la, l, tf, prm, d_entry, d_exit, d_out, w, h);
         la.m.cells = vol->d_cells;
         la.m.skip = skip;
-        launch_learned(la, phong, count, vol->cells_wide, learned_lanes(prm, (uint64_t)w * h), st);
+        launch_learned(la, phong, count, vol->cells_wide, learned_lanes(prm, (uint64_t)w * h, vol->cells_wide),
+                       st);
         hip_check(hipStreamWaitEvent(st, l->join, 0), "hipStreamWaitEvent");
         // 3. judge: flag = PSNR below the floor
         const float mse_max = powf(10.f, -opts.psnr_floor / 10.f);

@@ -475,12 +475,14 @@ static void launch_learned_t(const LearnedArgs& la, bool phong, bool count, hipS
 
 template <int P>
 static void launch_learned_p(const LearnedArgs& la, bool phong, bool count, bool wide, hipStream_t st) {
-    if (la.u16) {
-        if (wide) launch_learned_t<uint16_t, true, P>(la, phong, count, st);
-        else launch_learned_t<uint16_t, false, P>(la, phong, count, st);
+    if (wide) {
+        constexpr int PW = P == 1 ? 2 : P;   // one lane is for records within 4 GiB
+        if (la.u16) launch_learned_t<uint16_t, true, PW>(la, phong, count, st);
+        else launch_learned_t<uint8_t, true, PW>(la, phong, count, st);
+    } else if (la.u16) {
+        launch_learned_t<uint16_t, false, P>(la, phong, count, st);
     } else {
-        if (wide) launch_learned_t<uint8_t, true, P>(la, phong, count, st);
-        else launch_learned_t<uint8_t, false, P>(la, phong, count, st);
+        launch_learned_t<uint8_t, false, P>(la, phong, count, st);
     }
 }
 
