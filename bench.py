@@ -665,7 +665,9 @@ def main_c4(args):
             out["roofline"]["valu_insts_per_launch"] = int(pmc["valu_insts"])
             out["roofline"]["valu_issue_frac"] = round(
                 pmc["valu_insts"] / (sum(launch_ms) / len(launch_ms) / 1e3 * VALU_ISSUE_PEAK), 4)
-    assert st["samples"] == samples and st["fetched"] == fetched and st["shaded"] == shaded
+    # (single frames skip by bricks of 8^3, the batch by those of its configuration)
+    assert st["samples"] == samples and st["shaded"] == shaded
+    assert args.brick_log2 != 3 or st["fetched"] == fetched
     for o in outs:
         o.free()
     if args.copy_calibration:
