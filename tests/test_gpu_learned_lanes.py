@@ -208,9 +208,8 @@ def test_judge_pixels_equal_the_plain_frame(ctx, shading, exact):
 @pytest.mark.parametrize("images", [[(700, 600), (40, 37), (130, 57)], [(40, 37)] * 260], ids=["uneven", "many"])
 @pytest.mark.parametrize("shading", [0, 1])
 def test_fallback_frames_equal_the_plain_frames(ctx, shading, images):
-    """The views of a batch fall back (uint8 and uint16 volumes, more tiles
-    than the resident grid, more views than a workgroup has lanes), then every
-    second one."""
+    """The views of a batch fall back (uint8 and uint16 volumes, uneven images,
+    many views), then every second one."""
     scenes = [Scene(ctx, (64, 72, 80), np.uint16), Scene(ctx, (60, 48, 52), np.uint8)]
     H = scenes[0].H
     bad = H.Mlp(ctx, seed=3)

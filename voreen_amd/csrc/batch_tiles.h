@@ -42,15 +42,15 @@ __device__ __forceinline__ void block_tile(uint32_t lt, uint32_t tiles_x, uint32
     tx = bx * BW + r2 % bw;
 }
 
-// The order of the tiles of a launch whose workgroups each take a part of one.  The hardware hands consecutive workgroups to the
-// 8 XCDs in turn (workgroup b to XCD b % 8), and each XCD has its own L2.
-// Tiles come in blocks of kTileBlockW x kTileBlockH tiles of one job (blocks row by
-// row, tiles row by row inside a block; edge blocks smaller); consecutive runs
-// of kTileRun tiles of the launch's tile range are dealt to the XCDs in turn, so
-// the tiles an XCD marches at a time are a few compact blocks whose rays share
-// that XCD's L2, and the eight march neighbouring ones.  Blocks of 2x2 tiles:
-// 64 uneven volumes 709 us, 12 views of 512^3 6.43 ms; 4x4 695 us, 6.51 ms;
-// 8x4 824 us, 6.56 ms.
+// The order of the tiles of a plain grid, whose workgroups each take a part of
+// one.  The hardware hands consecutive workgroups to the 8 XCDs in turn (workgroup
+// b to XCD b % 8), and each XCD has its own L2.  Tiles come in blocks of
+// kTileBlockW x kTileBlockH tiles of one job (blocks row by row, tiles row by row
+// inside a block; edge blocks smaller); consecutive runs of kTileRun tiles of the
+// launch's tile range are dealt to the XCDs in turn, so the tiles an XCD marches
+// at a time are a few compact blocks whose rays share that XCD's L2, and the eight
+// march neighbouring ones.  Blocks of 2x2 tiles: 64 uneven volumes 709 us, 12
+// views of 512^3 6.43 ms; 4x4 695 us, 6.51 ms; 8x4 824 us, 6.56 ms.
 constexpr int kTileBlockW = 2, kTileBlockH = 2;
 constexpr uint32_t kTileRun = kTileBlockW * kTileBlockH;
 
